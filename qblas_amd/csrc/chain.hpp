@@ -1,0 +1,265 @@
+// chain.hpp -- accumulating correctly rounded FMA chains, acc = RN(a*b + acc), the step of every
+// REFERENCE-order kernel (the serial loops of include/quadblas/algorithms/level1.hpp:20-25,
+// level2.hpp:35-44,69-80, level3.hpp:200-210).  Same values as fma_packed on packed operands, bit
+// for bit, with the accumulator and the operands held in forms the step needs no shifting for.
+//
+//   cop   an operand, unpacked once: four 29-bit limbs of the 113-bit significand (so the columns
+//         of a product, sums of at most four 58-bit products, fit 64 bits), exponent, sign as a
+//         mask and the number of trailing zero bits.  Zero, subnormal, Inf and NaN operands carry
+//         the exponent CH_ESPECIAL, which no step's range check passes.
+//   cacc  the accumulator: a 160-bit two's complement frame W (five 32-bit words, the lowest always
+//         zero between steps) with value W 2^(E-152).  The leading bit lies anywhere in bits
+//         146..158, so a step that moves it by a few bits needs no renormalisation.
+//
+// One step: the product's columns (16 v_mad_u64_u32, each column's carry the next one's addend), its
+// bits 72.. as a frame with leading bit 152/153 at exponent ea + eb; the frame with the lower
+// exponent is shifted right onto the other one's grid (whole words by bit masks, then a funnel),
+// added in two's complement, and rounded in place at the 113th bit below the leading one.  Bits of the product
+// below the grid act through a sticky bit only, which its trailing zeros (the sum of the operands')
+// decide without looking at them: floor(x) plus a sticky bit rounds x correctly, as the grid lies
+// at least 34 bits below the rounding position.  About 120 VALU instructions; 401 with sign and
+// magnitude in 64-bit words and a case per exponent order.
+// Left to the packed operation (chain_slow): special operands or accumulators, exponents near the
+// ends of the range, an accumulator more than 32 bits below the product's grid, and sums that
+// cancel by 26 bits or more.
+#pragma once
+#include "q128.hpp"
+
+namespace qb {
+
+constexpr int32_t CH_ESPECIAL = 1 << 22;  // exponent of an operand or accumulator the step does not take
+constexpr int32_t CH_EZERO = -(1 << 24);  // exponent of a zero accumulator
+constexpr int32_t CH_EMAX = 16300;        // |exponent| of a step: every result is then a normal number
+
+struct cop {
+  uint32_t l[4];  // significand = sum l[i] 2^(29 i)
+  int32_t e;      // value = (-1)^neg significand 2^(e - 112)
+  uint32_t neg;   // 0 or ~0
+  int32_t tz;     // trailing zero bits of the significand
+  uint32_t pad;
+};
+struct cacc {
+  uint32_t w[4];  // words 1..4 of the frame (word 0 is zero); the packed value if E == CH_ESPECIAL
+  int32_t E;
+};
+
+QB_HD uint32_t ch_alignbit(uint32_t hi, uint32_t lo, uint32_t s) {  // (hi:lo) >> (s & 31), low word
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_alignbit(hi, lo, s);
+#else
+  return (uint32_t)((((uint64_t)hi << 32) | lo) >> (s & 31));
+#endif
+}
+// leading bits equal to the sign bit (0xffffffff when all are)
+QB_HD uint32_t ch_signbits(uint32_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t r;
+  asm("v_ffbh_i32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+#else
+  const uint32_t v = x ^ (uint32_t)((int32_t)x >> 31);
+  return v ? (uint32_t)__builtin_clz(v) : 0xffffffffu;
+#endif
+}
+// bit B of x as a mask.  Inline assembly on the device: seen as a sign, the compiler turns selects by
+// the mask into a compare and two or three instructions each instead of one v_bfi_b32
+template <int B>
+QB_HD uint32_t ch_mask(uint32_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t r;
+  asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(r) : "v"(x), "n"(B));
+  return r;
+#else
+  return 0u - ((x >> B) & 1u);
+#endif
+}
+QB_HD uint32_t ch_sel(uint32_t mask, uint32_t a, uint32_t b) { return (mask & a) | (~mask & b); }
+QB_HD uint32_t ch_addc(uint32_t a, uint32_t b, uint32_t ci, uint32_t &co) {
+#if defined(__clang__)
+  uint32_t c;
+  const uint32_t r = __builtin_addc(a, b, ci, &c);
+  co = c;
+  return r;
+#else
+  const uint64_t r = (uint64_t)a + b + ci;
+  co = (uint32_t)(r >> 32);
+  return (uint32_t)r;
+#endif
+}
+QB_HD int ch_ctz64(uint64_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __ffsll((unsigned long long)x) - 1;
+#else
+  return __builtin_ctzll(x);
+#endif
+}
+
+QB_HD cop cop_unpack(q128 a) {
+  cop r;
+  const uint32_t be = q_bexp(a);
+  const uint64_t mh = (a.hi & FRAC_HI_MASK) | HIDDEN;
+  r.l[0] = (uint32_t)a.lo & 0x1fffffffu;
+  r.l[1] = (uint32_t)(a.lo >> 29) & 0x1fffffffu;
+  r.l[2] = ch_alignbit((uint32_t)mh, (uint32_t)(a.lo >> 32), 26) & 0x1fffffffu;
+  r.l[3] = (uint32_t)(mh >> 23);
+  r.e = (be == 0 || be == 0x7fffu) ? CH_ESPECIAL : (int32_t)be - QBIAS;
+  r.neg = (uint32_t)((int32_t)(uint32_t)(a.hi >> 32) >> 31);
+  r.tz = a.lo ? ch_ctz64(a.lo) : 64 + ch_ctz64(mh);
+  r.pad = 0;
+  return r;
+}
+
+QB_HD void cacc_init(cacc &c) {
+  c.w[0] = c.w[1] = c.w[2] = c.w[3] = 0;
+  c.E = CH_EZERO;
+}
+QB_HD void cacc_set(cacc &c, q128 v) {
+  if (q_bexp(v) == 0x7fffu) {
+    c.w[0] = (uint32_t)v.lo;
+    c.w[1] = (uint32_t)(v.lo >> 32);
+    c.w[2] = (uint32_t)v.hi;
+    c.w[3] = (uint32_t)(v.hi >> 32);
+    c.E = CH_ESPECIAL;
+    return;
+  }
+  const uq u = unpack_finite(v);
+  if ((u.mh | u.ml) == 0) {
+    cacc_init(c);
+    c.w[0] = u.s;  // the sign of a zero: below every grid it is shifted to
+    return;
+  }
+  // leading bit (112 of m) to bit 153: words 1..4 hold m << 9
+  const uint64_t lo = u.ml << 9, hi = (u.mh << 9) | (u.ml >> 55);
+  const uint64_t x = u.s ? ~0ull : 0ull;
+  const uint64_t l2 = (lo ^ x) + (x & 1), h2 = (hi ^ x) + ((x & 1) & (lo == 0));
+  c.w[0] = (uint32_t)l2;
+  c.w[1] = (uint32_t)(l2 >> 32);
+  c.w[2] = (uint32_t)h2;
+  c.w[3] = (uint32_t)(h2 >> 32);
+  c.E = u.e - 1;
+}
+QB_HD q128 cacc_get(const cacc &c) {
+  uint64_t lo = ((uint64_t)c.w[1] << 32) | c.w[0], hi = ((uint64_t)c.w[3] << 32) | c.w[2];
+  if (c.E == CH_ESPECIAL) return q_make(lo, hi);
+  if (c.E == CH_EZERO) return q_zero(c.w[0]);
+  const uint64_t x = (uint64_t)((int64_t)hi >> 63);
+  lo = (lo ^ x) + (x & 1);
+  hi = (hi ^ x) + ((x & 1) & (lo == 0));
+  const int lz = clz64(hi) - 1;  // the leading bit lies in 114..126 of (hi:lo): one to bit 126
+  uq u;
+  const uint64_t h = shl_fill(hi, lo, lz), l = lo << lz;
+  u.mh = h >> 14;
+  u.ml = shr_fill(h, l, 14);
+  u.e = c.E + 6 - lz;  // bit 126 of (hi:lo) is bit 158 of the frame
+  u.s = (uint32_t)(x & 1);
+  return pack(u);
+}
+
+// acc = RN(a*b + acc).  Returns false, leaving acc as it was, when the packed operation has to do it.
+QB_HD bool cacc_step(cacc &acc, const cop &a, const cop &b) {
+  // product: column k at bit 29 k, carries folded into the next column's addend
+  uint64_t c0 = (uint64_t)a.l[0] * b.l[0];
+  uint64_t c1 = (uint64_t)a.l[0] * b.l[1] + (c0 >> 29);
+  c1 = (uint64_t)a.l[1] * b.l[0] + c1;
+  uint64_t c2 = (uint64_t)a.l[0] * b.l[2] + (c1 >> 29);
+  c2 = (uint64_t)a.l[1] * b.l[1] + c2;
+  c2 = (uint64_t)a.l[2] * b.l[0] + c2;
+  uint64_t c3 = (uint64_t)a.l[0] * b.l[3] + (c2 >> 29);
+  c3 = (uint64_t)a.l[1] * b.l[2] + c3;
+  c3 = (uint64_t)a.l[2] * b.l[1] + c3;
+  c3 = (uint64_t)a.l[3] * b.l[0] + c3;
+  uint64_t c4 = (uint64_t)a.l[1] * b.l[3] + (c3 >> 29);
+  c4 = (uint64_t)a.l[2] * b.l[2] + c4;
+  c4 = (uint64_t)a.l[3] * b.l[1] + c4;
+  uint64_t c5 = (uint64_t)a.l[2] * b.l[3] + (c4 >> 29);
+  c5 = (uint64_t)a.l[3] * b.l[2] + c5;
+  const uint64_t c6 = (uint64_t)a.l[3] * b.l[3] + (c5 >> 29);
+  // bits 72.. of the product (29-bit digits of the columns) as the frame, its sign applied as a
+  // complement; the missing +1 goes in as the sum's carry when nothing is lost below the grid
+  const uint32_t neg = a.neg ^ b.neg;
+  uint32_t P[5];
+  P[0] = ((((uint32_t)c2 >> 14) & 0x7fffu) | ((uint32_t)c3 << 15)) ^ neg;
+  P[1] = ((((uint32_t)c3 >> 17) & 0xfffu) | ((uint32_t)c4 << 12)) ^ neg;
+  P[2] = ((((uint32_t)c4 >> 20) & 0x1ffu) | ((uint32_t)c5 << 9)) ^ neg;
+  P[3] = ((((uint32_t)c5 >> 23) & 0x3fu) | ((uint32_t)c6 << 6)) ^ neg;
+  P[4] = ch_alignbit((uint32_t)(c6 >> 32), (uint32_t)c6, 26) ^ neg;
+  const int32_t Ep = a.e + b.e;
+  const int32_t d = acc.E - Ep;
+  const uint32_t pbig = ch_mask<31>((uint32_t)d);
+  const int32_t ad = d < 0 ? -d : d;
+  const uint32_t sh = (uint32_t)(ad < 159 ? ad : 159);
+  int32_t E = Ep > acc.E ? Ep : acc.E;
+  // X: the frame that stays, T: the one that is shifted
+  uint32_t X[5], T[5];
+  X[0] = P[0] & pbig;
+  T[0] = P[0] & ~pbig;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    X[i + 1] = ch_sel(pbig, P[i + 1], acc.w[i]);
+    T[i + 1] = ch_sel(pbig, acc.w[i], P[i + 1]);
+  }
+  const uint32_t sg = ch_mask<31>(T[4]), m4 = ch_mask<7>(sh), m2 = ch_mask<6>(sh), m1 = ch_mask<5>(sh);
+  uint32_t U[5], V[5], Q[5];
+  U[0] = ch_sel(m4, T[4], T[0]);
+#pragma unroll
+  for (int i = 1; i < 5; ++i) U[i] = ch_sel(m4, sg, T[i]);
+  V[0] = ch_sel(m2, U[2], U[0]);
+  V[1] = ch_sel(m2, U[3], U[1]);
+  V[2] = ch_sel(m2, U[4], U[2]);
+  V[3] = ch_sel(m2, sg, U[3]);
+  V[4] = ch_sel(m2, sg, U[4]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) Q[i] = ch_sel(m1, V[i + 1], V[i]);
+  Q[4] = ch_sel(m1, sg, V[4]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) T[i] = ch_alignbit(Q[i + 1], Q[i], sh);
+  T[4] = (uint32_t)((int32_t)Q[4] >> (sh & 31));
+  // bits of the product below the grid
+  const bool st = a.tz + b.tz - 72 < (d > 0 ? d : 0);
+  uint32_t F[5], c = (uint32_t)((neg != 0) & !st);
+#pragma unroll
+  for (int i = 0; i < 5; ++i) F[i] = ch_addc(X[i], T[i], c, c);
+  // range: exponents; an accumulator with bits below the product's grid; a sum in words 0..3 only
+  uint32_t fb = ch_signbits(F[4]);
+  if (((uint32_t)(E + CH_EMAX) > (uint32_t)(2 * CH_EMAX)) | ((uint32_t)(-33 - d) < (1u << 20)) | (fb > 31u)) return false;
+  uint32_t w0 = F[0] | (uint32_t)st;
+  if (fb - 2u > 11u) {  // the leading bit left 146..157: to 153
+    if (fb < 2u) {
+      const uint32_t r = 6 - fb;
+      const uint32_t lost = w0 << (32 - r);
+      w0 = ch_alignbit(F[1], w0, r) | (uint32_t)(lost != 0);
+#pragma unroll
+      for (int i = 1; i < 4; ++i) F[i] = ch_alignbit(F[i + 1], F[i], r);
+      F[4] = (uint32_t)((int32_t)F[4] >> r);
+    } else {
+      const uint32_t r = 32 - (fb - 6);
+#pragma unroll
+      for (int i = 4; i > 1; --i) F[i] = ch_alignbit(F[i], F[i - 1], r);
+      F[1] = ch_alignbit(F[1], w0, r);
+      w0 = (w0 << (32 - r)) | (w0 & 1u);  // the sticky bit stays at the bottom
+    }
+    E += 6 - (int32_t)fb;
+    fb = 6;
+  }
+  // round to nearest even at bit 47 - fb: bit 15 - fb of word 1, half = 2^14 >> fb
+  uint32_t w1 = F[1] | (w0 < 1u ? w0 : 1u);
+  const uint32_t half = 0x4000u >> fb;
+  const uint32_t lsb = (w1 >> (15u - fb)) & 1u;
+  c = 0;
+  w1 = ch_addc(w1, half - 1u + lsb, 0u, c);
+  acc.w[0] = w1 & (0u - half - half);
+  acc.w[1] = ch_addc(F[2], 0u, c, c);
+  acc.w[2] = ch_addc(F[3], 0u, c, c);
+  acc.w[3] = ch_addc(F[4], 0u, c, c);
+  acc.E = E;
+  return true;
+}
+QB_HD void chain_slow(cacc &acc, q128 a, q128 b) { cacc_set(acc, fma_packed(a, b, cacc_get(acc))); }
+
+// acc = RN(a*b + acc) for packed a, b, with b's unpacked form at hand
+QB_HD void chain_fma(cacc &acc, q128 a, q128 b, const cop &B) {
+  if (!cacc_step(acc, cop_unpack(a), B)) chain_slow(acc, a, b);
+}
+QB_HD void chain_fma(cacc &acc, q128 a, q128 b) { chain_fma(acc, a, b, cop_unpack(b)); }
+
+}  // namespace qb

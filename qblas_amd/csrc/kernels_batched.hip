@@ -23,6 +23,7 @@
 //                   (wide.hpp).
 // Tile shapes are template parameters; the host picks one configuration per call (the
 // autotuner in capi.hip measures them).
+#include "chain.hpp"
 #include "dd.hpp"
 #include "wide.hpp"
 #include "kernels.h"
@@ -126,10 +127,10 @@ __device__ __forceinline__ void ref_gemm_entry(const qblas_gemm_problem &g, int6
   const q128 *bp = B + j * bs_j;
   for (int64_t kk = 0; kk < k; kk += kc) {
     const int64_t ke = (kk + kc < k) ? kk + kc : k;
-    chain ch;
-    chain_init(ch);
+    cacc ch;
+    cacc_init(ch);
     for (int64_t l = kk; l < ke; ++l) chain_fma(ch, bld(ap + l * as_l), bld(bp + l * bs_l));
-    c = fma_packed(alpha, chain_get(ch), mul_packed(kk == 0 ? beta : q_one(), c));
+    c = fma_packed(alpha, cacc_get(ch), mul_packed(kk == 0 ? beta : q_one(), c));
   }
   bst(ci, c);
 }
@@ -275,19 +276,19 @@ __global__ void __launch_bounds__(256) k_gemv_batched_ref(const qblas_gemv_probl
     const q128 *x = (const q128 *)v.x;
     q128 *y = (q128 *)v.y;
     const q128 alpha = qv(v.alpha), beta = qv(v.beta);
-    chain ch;
+    cacc ch;
     if (!colmajor && incx == 1) {
       // two lane chains per row (level2.hpp:35-38 with dot_kernel_vectorized), rows ul*32 + lane/2
       const int64_t i = ul * 32 + (lane >> 1);
       const int par = lane & 1;
       const bool live = i < m;
-      chain_init(ch);
+      cacc_init(ch);
       if (live) {
         const q128 *row = A + i * lda;
         const int64_t pairs = n / 2;
         for (int64_t jj = 0; jj < pairs; ++jj) chain_fma(ch, bld(row + 2 * jj + par), bld(x + 2 * jj + par));
       }
-      const q128 mine = chain_get(ch);
+      const q128 mine = cacc_get(ch);
       const uint64_t olo = (uint64_t)__shfl_xor((unsigned long long)mine.lo, 1);
       const uint64_t ohi = (uint64_t)__shfl_xor((unsigned long long)mine.hi, 1);
       if (live && par == 0) {
@@ -299,20 +300,20 @@ __global__ void __launch_bounds__(256) k_gemv_batched_ref(const qblas_gemv_probl
     } else if (!colmajor) {
       const int64_t i = ul * 64 + lane;
       if (i < m) {
-        chain_init(ch);
+        cacc_init(ch);
         const q128 *row = A + i * lda;
         for (int64_t j = 0; j < n; ++j) chain_fma(ch, bld(row + j), bld(x + j * incx));
         q128 *yi = y + i * incy;
-        bst(yi, fma_packed(alpha, chain_get(ch), mul_packed(beta, bld(yi))));
+        bst(yi, fma_packed(alpha, cacc_get(ch), mul_packed(beta, bld(yi))));
       }
     } else {
       // level2.hpp:63-80: y_i = mul(beta, y_i), then fma(A_ij, mul(alpha, x_j), y_i) over j
       const int64_t i = ul * 64 + lane;
       if (i < m) {
         q128 *yi = y + i * incy;
-        chain_set(ch, mul_packed(beta, bld(yi)));
+        cacc_set(ch, mul_packed(beta, bld(yi)));
         for (int64_t j = 0; j < n; ++j) chain_fma(ch, bld(A + j * lda + i), mul_packed(alpha, bld(x + j * incx)));
-        bst(yi, chain_get(ch));
+        bst(yi, cacc_get(ch));
       }
     }
     u = waves + (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)ticket);  // lane 0's ticket

@@ -10,7 +10,7 @@
 // Every reference chain is inherently sequential, so one lane owns one chain; these kernels are
 // latency-bound by construction.  The other forms (kernels_exact.hip, kernels_dd.hip,
 // kernels_ozaki.hip) trade the reference order for exact or wider accumulation.
-#include "q128.hpp"
+#include "chain.hpp"
 #include "kernels.h"
 
 using namespace qb;
@@ -48,8 +48,8 @@ __device__ __forceinline__ void chunk_range(int64_t n, int T, int t, int64_t &s,
 __global__ void k_dot_ref_chains(const q128 *__restrict__ x, int64_t incx, const q128 *__restrict__ y,
                                  int64_t incy, int64_t n, int T, int contiguous, q128 *__restrict__ part) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  chain ch;
-  chain_init(ch);
+  cacc ch;
+  cacc_init(ch);
   if (contiguous) {
     const int t = tid >> 1, p = tid & 1;
     if (t >= T) return;
@@ -60,14 +60,14 @@ __global__ void k_dot_ref_chains(const q128 *__restrict__ x, int64_t incx, const
       const int64_t k = s + 2 * i + p;
       chain_fma(ch, ld(x + k), ld(y + k));
     }
-    st(part + 2 * t + p, chain_get(ch));
+    st(part + 2 * t + p, cacc_get(ch));
   } else {
     const int t = tid;
     if (t >= T) return;
     int64_t s, e;
     chunk_range(n, T, t, s, e);
     for (int64_t i = s; i < e; ++i) chain_fma(ch, ld(x + i * incx), ld(y + i * incy));
-    st(part + t, chain_get(ch));
+    st(part + t, cacc_get(ch));
   }
 }
 
@@ -111,8 +111,8 @@ __global__ void k_gemv_row_ref(int64_t m, int64_t n, q128 alpha, const q128 *__r
                                const q128 *__restrict__ x, int64_t incx, q128 beta, q128 *__restrict__ y,
                                int64_t incy) {
   const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  chain ch;
-  chain_init(ch);
+  cacc ch;
+  cacc_init(ch);
   if (incx == 1) {
     const int64_t i = tid >> 1;
     const int p = (int)(tid & 1);
@@ -122,7 +122,7 @@ __global__ void k_gemv_row_ref(int64_t m, int64_t n, q128 alpha, const q128 *__r
       const int64_t pairs = n / 2;
       for (int64_t j = 0; j < pairs; ++j) chain_fma(ch, ld(row + 2 * j + p), ld(x + 2 * j + p));
     }
-    const q128 mine = chain_get(ch);
+    const q128 mine = cacc_get(ch);
     // exchange with the partner lane (same row); both lanes of a pair are live or dead together
     const uint64_t olo = (uint64_t)__shfl_xor((unsigned long long)mine.lo, 1);
     const uint64_t ohi = (uint64_t)__shfl_xor((unsigned long long)mine.hi, 1);
@@ -137,7 +137,7 @@ __global__ void k_gemv_row_ref(int64_t m, int64_t n, q128 alpha, const q128 *__r
     const q128 *row = A + i * lda;
     for (int64_t j = 0; j < n; ++j) chain_fma(ch, ld(row + j), ld(x + j * incx));
     q128 *yi = y + i * incy;
-    st(yi, fma_packed(alpha, chain_get(ch), mul_packed(beta, ld(yi))));
+    st(yi, fma_packed(alpha, cacc_get(ch), mul_packed(beta, ld(yi))));
   }
 }
 
@@ -155,10 +155,10 @@ __global__ void k_gemv_col_ref(int64_t m, int64_t n, const q128 *__restrict__ A,
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
     q128 *yi = y + i * incy;
-    chain ch;
-    chain_set(ch, mul_packed(beta, ld(yi)));
+    cacc ch;
+    cacc_set(ch, mul_packed(beta, ld(yi)));
     for (int64_t j = 0; j < n; ++j) chain_fma(ch, ld(A + j * lda + i), ld(ax + j));
-    st(yi, chain_get(ch));
+    st(yi, cacc_get(ch));
   }
 }
 
@@ -174,20 +174,15 @@ __global__ void k_gemv_col_ref(int64_t m, int64_t n, const q128 *__restrict__ A,
 // contiguous dimension), unpack them into LDS, and every lane runs its chain over the step from
 // LDS, in the same order l = kk, kk + 1, ... as the reference.  An operand that is zero,
 // subnormal, Inf or NaN is marked in LDS and taken from memory again for the packed slow path.
+// Bound by VALU issue: about 120 instructions per wave and multiply-add (chain.hpp).  4096^3
+// log-uniform: 244 ms = 563 quad GFLOP/s (577 ms with the 401-instruction step before).
 constexpr int GR_KT = 32;
-constexpr int32_t GR_SPECIAL = INT32_MIN;  // uq.e of an operand the fast path does not take
-__device__ __forceinline__ uq gr_unpack(q128 v) {
-  bool sp;
-  uq u = unpack_fast(v, sp);
-  if (sp) u.e = GR_SPECIAL;
-  return u;
-}
 __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_t kc,
                                                   q128 alpha, const q128 *__restrict__ A, int64_t lda,
                                                   const q128 *__restrict__ B, int64_t ldb, q128 beta,
                                                   q128 *__restrict__ C, int64_t ldc) {
-  __shared__ uq sA[GR_KT][16];
-  __shared__ uq sB[GR_KT][16];
+  __shared__ __attribute__((aligned(16))) cop sA[GR_KT][16];
+  __shared__ __attribute__((aligned(16))) cop sB[GR_KT][16];
   const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
   const int64_t i0 = (int64_t)blockIdx.y * 16, j0 = (int64_t)blockIdx.x * 16;
   const int64_t i = i0 + ti, j = j0 + tj;
@@ -200,8 +195,8 @@ __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64
   const q128 *bp = B + j * bs_j;
   for (int64_t kk = 0; kk < k; kk += kc) {
     const int64_t ke = (kk + kc < k) ? kk + kc : k;
-    chain ch;
-    chain_init(ch);
+    cacc ch;
+    cacc_init(ch);
     for (int64_t l0 = kk; l0 < ke; l0 += GR_KT) {
       const int lt = (int)((ke - l0 < GR_KT) ? ke - l0 : GR_KT);
       __syncthreads();  // the previous step's operands are no longer read
@@ -210,29 +205,20 @@ __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64
         const int e = (int)threadIdx.x + 256 * h;  // 512 = 16 x GR_KT elements of each operand
         // A(i0 + r, l0 + q): l contiguous (RowMajor) -> q fastest; rows contiguous -> r fastest
         const int ra = colmajor ? (e & 15) : (e >> 5), qa = colmajor ? (e >> 4) : (e & 31);
-        if (qa < lt && i0 + ra < m) sA[qa][ra] = gr_unpack(ld(A + (i0 + ra) * as_i + (l0 + qa) * as_l));
+        if (qa < lt && i0 + ra < m) sA[qa][ra] = cop_unpack(ld(A + (i0 + ra) * as_i + (l0 + qa) * as_l));
         // B(l0 + q, j0 + c): columns contiguous (RowMajor) -> c fastest; l contiguous -> q fastest
         const int cb = colmajor ? (e >> 5) : (e & 15), qb = colmajor ? (e & 31) : (e >> 4);
-        if (qb < lt && j0 + cb < n) sB[qb][cb] = gr_unpack(ld(B + (l0 + qb) * bs_l + (j0 + cb) * bs_j));
+        if (qb < lt && j0 + cb < n) sB[qb][cb] = cop_unpack(ld(B + (l0 + qb) * bs_l + (j0 + cb) * bs_j));
       }
       __syncthreads();
       if (live) {
         for (int q = 0; q < lt; ++q) {
-          const uq ua = sA[q][ti], ub = sB[q][tj];
-          bool done = false;
-          if ((ua.e != GR_SPECIAL) & (ub.e != GR_SPECIAL) & !ch.special) {
-            bool ovf = false;
-            const uq r = fma_uq(ua, ub, ch.acc, ovf);
-            if (!ovf) {
-              ch.acc = r;
-              done = true;
-            }
-          }
-          if (!done) chain_set(ch, fma_packed(ld(ap + (l0 + q) * as_l), ld(bp + (l0 + q) * bs_l), chain_get(ch)));
+          if (!cacc_step(ch, sA[q][ti], sB[q][tj]))
+            chain_slow(ch, ld(ap + (l0 + q) * as_l), ld(bp + (l0 + q) * bs_l));
         }
       }
     }
-    c = fma_packed(alpha, chain_get(ch), mul_packed(kk == 0 ? beta : q_one(), c));
+    c = fma_packed(alpha, cacc_get(ch), mul_packed(kk == 0 ? beta : q_one(), c));
   }
   if (live) st(ci, c);
 }

@@ -440,70 +440,6 @@ QB_HD q128 fma_packed(q128 a, q128 b, q128 c) {
 QB_HD q128 add_packed(q128 a, q128 b) { return fma_packed(a, q_one(), b); }
 QB_HD q128 mul_packed(q128 a, q128 b) { return fma_packed(a, b, q_zero(1)); }
 
-// Accumulating FMA for chains kept unpacked: acc = a*b + acc with a, b packed.  Falls back to the
-// packed rules for zeros, subnormals, Inf and NaN; 'accp' mirrors acc in packed form only when
-// the chain has left the finite range (acc_special set), which is sticky.
-struct chain {
-  uq acc;
-  q128 special_val;
-  bool special;  // acc is Inf/NaN: the value is special_val
-};
-
-QB_HD void chain_init(chain &ch) {
-  ch.acc.mh = 0;
-  ch.acc.ml = 0;
-  ch.acc.e = UQ_EZERO;
-  ch.acc.s = 0;
-  ch.special = false;
-  ch.special_val = q_zero(0);
-}
-QB_HD void chain_set(chain &ch, q128 v) {
-  if (q_bexp(v) == 0x7fffu) {
-    ch.special = true;
-    ch.special_val = v;
-    ch.acc.mh = 0;
-    ch.acc.ml = 0;
-    ch.acc.e = UQ_EZERO;
-    ch.acc.s = 0;
-  } else {
-    ch.special = false;
-    ch.acc = unpack_finite(v);
-  }
-}
-QB_HD q128 chain_get(const chain &ch) {
-  if (ch.special) return ch.special_val;
-  return pack(ch.acc);
-}
-// Note on zero accumulators: an unpacked zero keeps its sign in acc.s, so pack() restores -0.
-QB_HD void chain_fma(chain &ch, q128 a, q128 b) {
-  bool spa, spb;
-  const uq A = unpack_fast(a, spa);
-  const uq B = unpack_fast(b, spb);
-  if (!(spa | spb | ch.special)) {
-    bool ovf = false;
-    uq r = fma_uq(A, B, ch.acc, ovf);
-    if (!ovf) {
-      ch.acc = r;
-      return;
-    }
-  }
-  chain_set(ch, fma_packed(a, b, chain_get(ch)));
-}
-// Same with an unpacked, known finite nonzero normal 'b' (e.g. a value staged once).
-QB_HD void chain_fma_ub(chain &ch, q128 a, const uq &B, q128 bpacked) {
-  bool spa;
-  const uq A = unpack_fast(a, spa);
-  if (!(spa | ch.special)) {
-    bool ovf = false;
-    uq r = fma_uq(A, B, ch.acc, ovf);
-    if (!ovf) {
-      ch.acc = r;
-      return;
-    }
-  }
-  chain_set(ch, fma_packed(a, bpacked, chain_get(ch)));
-}
-
 // ------------------------------------------------------------------------------------------
 // conversions
 // ------------------------------------------------------------------------------------------
