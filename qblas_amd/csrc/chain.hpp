@@ -155,34 +155,39 @@ QB_HD q128 cacc_get(const cacc &c) {
   return pack(u);
 }
 
+// columns of the product of two significands: column k at bit 29 k, each one's carry over 29 bits
+// added into the next (the digits are the low 29 bits of columns 0..5 and all of column 6)
+QB_HD void cop_columns(uint64_t (&c)[7], const cop &a, const cop &b) {
+  c[0] = (uint64_t)a.l[0] * b.l[0];
+  c[1] = (uint64_t)a.l[0] * b.l[1] + (c[0] >> 29);
+  c[1] = (uint64_t)a.l[1] * b.l[0] + c[1];
+  c[2] = (uint64_t)a.l[0] * b.l[2] + (c[1] >> 29);
+  c[2] = (uint64_t)a.l[1] * b.l[1] + c[2];
+  c[2] = (uint64_t)a.l[2] * b.l[0] + c[2];
+  c[3] = (uint64_t)a.l[0] * b.l[3] + (c[2] >> 29);
+  c[3] = (uint64_t)a.l[1] * b.l[2] + c[3];
+  c[3] = (uint64_t)a.l[2] * b.l[1] + c[3];
+  c[3] = (uint64_t)a.l[3] * b.l[0] + c[3];
+  c[4] = (uint64_t)a.l[1] * b.l[3] + (c[3] >> 29);
+  c[4] = (uint64_t)a.l[2] * b.l[2] + c[4];
+  c[4] = (uint64_t)a.l[3] * b.l[1] + c[4];
+  c[5] = (uint64_t)a.l[2] * b.l[3] + (c[4] >> 29);
+  c[5] = (uint64_t)a.l[3] * b.l[2] + c[5];
+  c[6] = (uint64_t)a.l[3] * b.l[3] + (c[5] >> 29);
+}
 // acc = RN(a*b + acc).  Returns false, leaving acc as it was, when the packed operation has to do it.
 QB_HD bool cacc_step(cacc &acc, const cop &a, const cop &b) {
-  // product: column k at bit 29 k, carries folded into the next column's addend
-  uint64_t c0 = (uint64_t)a.l[0] * b.l[0];
-  uint64_t c1 = (uint64_t)a.l[0] * b.l[1] + (c0 >> 29);
-  c1 = (uint64_t)a.l[1] * b.l[0] + c1;
-  uint64_t c2 = (uint64_t)a.l[0] * b.l[2] + (c1 >> 29);
-  c2 = (uint64_t)a.l[1] * b.l[1] + c2;
-  c2 = (uint64_t)a.l[2] * b.l[0] + c2;
-  uint64_t c3 = (uint64_t)a.l[0] * b.l[3] + (c2 >> 29);
-  c3 = (uint64_t)a.l[1] * b.l[2] + c3;
-  c3 = (uint64_t)a.l[2] * b.l[1] + c3;
-  c3 = (uint64_t)a.l[3] * b.l[0] + c3;
-  uint64_t c4 = (uint64_t)a.l[1] * b.l[3] + (c3 >> 29);
-  c4 = (uint64_t)a.l[2] * b.l[2] + c4;
-  c4 = (uint64_t)a.l[3] * b.l[1] + c4;
-  uint64_t c5 = (uint64_t)a.l[2] * b.l[3] + (c4 >> 29);
-  c5 = (uint64_t)a.l[3] * b.l[2] + c5;
-  const uint64_t c6 = (uint64_t)a.l[3] * b.l[3] + (c5 >> 29);
+  uint64_t k[7];
+  cop_columns(k, a, b);
   // bits 72.. of the product (29-bit digits of the columns) as the frame, its sign applied as a
   // complement; the missing +1 goes in as the sum's carry when nothing is lost below the grid
   const uint32_t neg = a.neg ^ b.neg;
   uint32_t P[5];
-  P[0] = ((((uint32_t)c2 >> 14) & 0x7fffu) | ((uint32_t)c3 << 15)) ^ neg;
-  P[1] = ((((uint32_t)c3 >> 17) & 0xfffu) | ((uint32_t)c4 << 12)) ^ neg;
-  P[2] = ((((uint32_t)c4 >> 20) & 0x1ffu) | ((uint32_t)c5 << 9)) ^ neg;
-  P[3] = ((((uint32_t)c5 >> 23) & 0x3fu) | ((uint32_t)c6 << 6)) ^ neg;
-  P[4] = ch_alignbit((uint32_t)(c6 >> 32), (uint32_t)c6, 26) ^ neg;
+  P[0] = ((((uint32_t)k[2] >> 14) & 0x7fffu) | ((uint32_t)k[3] << 15)) ^ neg;
+  P[1] = ((((uint32_t)k[3] >> 17) & 0xfffu) | ((uint32_t)k[4] << 12)) ^ neg;
+  P[2] = ((((uint32_t)k[4] >> 20) & 0x1ffu) | ((uint32_t)k[5] << 9)) ^ neg;
+  P[3] = ((((uint32_t)k[5] >> 23) & 0x3fu) | ((uint32_t)k[6] << 6)) ^ neg;
+  P[4] = ch_alignbit((uint32_t)(k[6] >> 32), (uint32_t)k[6], 26) ^ neg;
   const int32_t Ep = a.e + b.e;
   const int32_t d = acc.E - Ep;
   const uint32_t pbig = ch_mask<31>((uint32_t)d);

@@ -7,10 +7,11 @@
 //   dot  : include/quadblas/algorithms/level1.hpp:14-137
 //   gemv : include/quadblas/algorithms/level2.hpp:15-99
 //   gemm : include/quadblas/algorithms/level3.hpp:187-336 (kc from detail/blocking.hpp:17-67)
-// Every reference chain is inherently sequential, so one lane owns one chain; these kernels are
-// latency-bound by construction.  The other forms (kernels_exact.hip, kernels_dd.hip,
+// Every reference chain is a serial order of rounded steps.  Where there are chains enough to fill the
+// chip one lane owns one (chain.hpp); where there are few, a wave does a chain's steps 64 at a time
+// with the same results (chain_scan.hpp).  The other forms (kernels_exact.hip, kernels_dd.hip,
 // kernels_ozaki.hip) trade the reference order for exact or wider accumulation.
-#include "chain.hpp"
+#include "chain_scan.hpp"
 #include "kernels.h"
 
 using namespace qb;
@@ -41,62 +42,52 @@ __device__ __forceinline__ void chunk_range(int64_t n, int T, int t, int64_t &s,
   e = (t == T - 1) ? n : s + chunk;
 }
 
-// Contiguous: chunk t, lane p in {0,1} runs dot_kernel_vectorized's lane-p chain over the
-// chunk's elements start+p, start+p+2, ... for i < len/2 (level1.hpp:20-25).
-// Strided: chunk t runs one serial chain over its elements (level1.hpp:111-114, :130-133).
-// part[] receives 2*T (contiguous) or T (strided) packed partial chains.
-__global__ void k_dot_ref_chains(const q128 *__restrict__ x, int64_t incx, const q128 *__restrict__ y,
-                                 int64_t incy, int64_t n, int T, int contiguous, q128 *__restrict__ part) {
-  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  cacc ch;
-  cacc_init(ch);
-  if (contiguous) {
-    const int t = tid >> 1, p = tid & 1;
-    if (t >= T) return;
-    int64_t s, e;
-    chunk_range(n, T, t, s, e);
-    const int64_t pairs = (e > s) ? (e - s) / 2 : 0;
-    for (int64_t i = 0; i < pairs; ++i) {
-      const int64_t k = s + 2 * i + p;
-      chain_fma(ch, ld(x + k), ld(y + k));
-    }
-    st(part + 2 * t + p, cacc_get(ch));
-  } else {
-    const int t = tid;
-    if (t >= T) return;
-    int64_t s, e;
-    chunk_range(n, T, t, s, e);
-    for (int64_t i = s; i < e; ++i) chain_fma(ch, ld(x + i * incx), ld(y + i * incy));
-    st(part + t, cacc_get(ch));
+// Contiguous: chunk t is two chains, lane p's over elements start+p, start+p+2, ... for i < len/2
+// (dot_kernel_vectorized, level1.hpp:20-25), combined by horizontal_sum (quad_vector.hpp:141-150) and
+// the odd tail's fma (level1.hpp:29-32).  Strided: one serial chain per chunk (level1.hpp:111-114,
+// :130-133).  There are only T or 2T chains, so each gets a whole wave, 64 elements at a time
+// (chain_scan.hpp); a workgroup is one chunk.  part[t] receives the chunk's value, or, with one
+// chunk, out the result ('direct': n < 500 returns the kernel's value without the final
+// "0 + partial" sum, level1.hpp:40-43, :128-134).
+// Bound by the latency of a block of 64 steps.  2^20 elements, T = 16: 0.93 ms (39 ms with one lane
+// per chain and the packed step, 18 ms with chain.hpp's step).
+__global__ void __launch_bounds__(128) k_dot_ref_chunks(const q128 *__restrict__ x, int64_t incx,
+                                                        const q128 *__restrict__ y, int64_t incy, int64_t n, int T,
+                                                        int direct, q128 *__restrict__ part, q128 *__restrict__ out) {
+  __shared__ q128 second;
+  const int t = (int)blockIdx.x, pair = blockDim.x > 64;  // two waves: contiguous
+  const int p = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  int64_t s, e;
+  chunk_range(n, T, t, s, e);
+  const int64_t len = e > s ? e - s : 0, step = 1 + pair;
+  const q128 *xc = x + (s + p) * incx, *yc = y + (s + p) * incy;
+  q128 r = wave_chain(q_zero(0), sc_strided{xc, step * incx}, sc_strided{yc, step * incy}, len / step);
+  if (pair) {
+    if (threadIdx.x == 64) second = r;
+    __syncthreads();
   }
+  if (threadIdx.x != 0) return;
+  if (pair && len) {
+    q128 a = second, b = q_one();
+#pragma unroll 1
+    for (int op = 0; op < 1 + (int)(len & 1); ++op) {
+      cacc acc;
+      cacc_set(acc, r);
+      chain_fma(acc, a, b);
+      r = cacc_get(acc);
+      a = ld(x + e - 1);
+      b = ld(y + e - 1);
+    }
+  }
+  if (T == 1)
+    st(out, direct ? r : add_packed(q_zero(0), r));
+  else
+    st(part + t, r);
 }
-
-// Serial epilogue (one thread): lanes combined by horizontal_sum (quad_vector.hpp:141-150),
-// odd tail fma (level1.hpp:29-32), chunk partials summed from +0 in chunk order (:67-71,
-// :117-120).  'direct' marks the n < 500 paths, which return the kernel's value without the
-// final "0 + partial" sum (level1.hpp:40-43, :128-134).
-__global__ void k_dot_ref_finish(const q128 *__restrict__ x, const q128 *__restrict__ y, int64_t n, int T,
-                                 int contiguous, int direct, const q128 *__restrict__ part,
-                                 q128 *__restrict__ out) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  q128 r = q_zero(0);
-  for (int t = 0; t < T; ++t) {
-    q128 pt;
-    if (contiguous) {
-      int64_t s, e;
-      chunk_range(n, T, t, s, e);
-      if (e > s) {
-        pt = add_packed(ld(part + 2 * t), ld(part + 2 * t + 1));
-        if ((e - s) & 1) pt = fma_packed(ld(x + e - 1), ld(y + e - 1), pt);
-      } else {
-        pt = q_zero(0);
-      }
-    } else {
-      pt = ld(part + t);
-    }
-    r = direct ? pt : add_packed(r, pt);
-  }
-  st(out, r);
+// the chunks' values summed from +0 in chunk order (level1.hpp:67-71, :117-120): one more chain
+__global__ void __launch_bounds__(64) k_dot_ref_sum(int T, const q128 *__restrict__ part, q128 *__restrict__ out) {
+  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1}, sc_const{q_one()}, T);
+  if (threadIdx.x == 0) st(out, r);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -141,6 +132,50 @@ __global__ void k_gemv_row_ref(int64_t m, int64_t n, q128 alpha, const q128 *__r
   }
 }
 
+// y_i = fma(alpha, sum, mul(beta, y_i)) with sum = c0 + c1 (two chains), the odd tail's fma applied;
+// the four operations as one loop, so the step's code is there once
+__device__ __forceinline__ q128 gemv_row_end(q128 c0, q128 c1, int pair, int odd, q128 ta, q128 tx, q128 alpha,
+                                             q128 beta, q128 y) {
+  q128 by = q_zero(1), sum = c0;
+#pragma unroll 1
+  for (int op = 0; op < 4; ++op) {
+    if ((op == 1 && !pair) || (op == 2 && !odd)) continue;
+    const q128 a = op == 0 ? beta : op == 1 ? c1 : op == 2 ? ta : alpha;
+    const q128 b = op == 0 ? y : op == 1 ? q_one() : op == 2 ? tx : sum;
+    cacc acc;
+    cacc_set(acc, (op == 0 || op == 3) ? by : sum);
+    chain_fma(acc, a, b);
+    const q128 r = cacc_get(acc);
+    if (op == 0 || op == 3) by = r;
+    else sum = r;
+  }
+  return by;
+}
+// Few rows: one wave per chain, 64 columns at a time (chain_scan.hpp); rows of a workgroup share x.
+// A pair's chains are neighbouring waves, the first of which ends the row.
+__global__ void __launch_bounds__(256) k_gemv_row_ref_scan(int64_t m, int64_t n, q128 alpha, const q128 *__restrict__ A,
+                                                           int64_t lda, const q128 *__restrict__ x, int64_t incx,
+                                                           q128 beta, q128 *__restrict__ y, int64_t incy) {
+  __shared__ q128 other[4];
+  const int pair = incx == 1;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t c = (int64_t)blockIdx.x * 4 + w;
+  const int64_t i = pair ? c >> 1 : c;
+  const int p = pair ? (int)(c & 1) : 0;
+  q128 r = q_zero(0);
+  if (i < m)
+    r = wave_chain(q_zero(0), sc_strided{A + i * lda + p, 1 + pair}, sc_strided{x + p, pair ? 2 : incx},
+                   pair ? n / 2 : n);
+  if ((threadIdx.x & 63) == 0) other[w] = r;
+  __syncthreads();
+  if (i < m && p == 0 && (threadIdx.x & 63) == 0) {
+    const int odd = pair && (n & 1);
+    q128 *yi = y + i * incy;
+    st(yi, gemv_row_end(r, other[w ^ pair], pair, odd, odd ? ld(A + i * lda + n - 1) : q_zero(0),
+                        odd ? ld(x + n - 1) : q_zero(0), alpha, beta, ld(yi)));
+  }
+}
+
 // ColMajor: ax[j] = mul(alpha, x_j) once per column (level2.hpp:71).
 __global__ void k_scale_vec(int64_t n, q128 alpha, const q128 *__restrict__ x, int64_t incx,
                             q128 *__restrict__ ax) {
@@ -160,6 +195,17 @@ __global__ void k_gemv_col_ref(int64_t m, int64_t n, const q128 *__restrict__ A,
     for (int64_t j = 0; j < n; ++j) chain_fma(ch, ld(A + j * lda + i), ld(ax + j));
     st(yi, cacc_get(ch));
   }
+}
+
+// Few rows: one wave per row; the eight rows of a workgroup share the 128-byte lines of A's columns.
+__global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n, const q128 *__restrict__ A,
+                                                           int64_t lda, const q128 *__restrict__ ax, q128 beta,
+                                                           q128 *__restrict__ y, int64_t incy) {
+  const int64_t i = (int64_t)blockIdx.x * 8 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (i >= m) return;
+  q128 *yi = y + i * incy;
+  const q128 r = wave_chain(mul_packed(beta, ld(yi)), sc_strided{A + i, lda}, sc_strided{ax, 1}, n);
+  if ((threadIdx.x & 63) == 0) st(yi, r);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -298,13 +344,19 @@ hipError_t launch_dot_ref(const q128 *x, int64_t incx, const q128 *y, int64_t in
     Teff = 1;
     direct = 1;
   }
-  const int lanes = contiguous ? 2 * Teff : Teff;
-  const int threads = 64;
-  const int blocks = (lanes + threads - 1) / threads;
-  hipLaunchKernelGGL(k_dot_ref_chains, dim3(blocks), dim3(threads), 0, st, x, incx, y, incy, n, Teff,
-                     contiguous, part);
-  hipLaunchKernelGGL(k_dot_ref_finish, dim3(1), dim3(64), 0, st, x, y, n, Teff, contiguous, direct, part, out);
+  hipLaunchKernelGGL(k_dot_ref_chunks, dim3(Teff), dim3(contiguous ? 128 : 64), 0, st, x, incx, y, incy, n, Teff, direct,
+                     part, out);
+  if (Teff > 1) hipLaunchKernelGGL(k_dot_ref_sum, dim3(1), dim3(64), 0, st, Teff, part, out);
   return hipGetLastError();
+}
+
+// Whether a gemv's chains go to a wave each (chain_scan.hpp) or to a lane each.  A lane's step is a
+// latency of about 0.5 us until the lanes fill the chip; a wave's block of 64 steps costs what about
+// 9 instructions a step cost, and the rest of a block as well.  Measured, uniform entries, us (wave
+// each, lane each): row-major 1500^2 69, 360; 8192^2 809, 2300; 16384 x 2048 (32768 chains) 460, 634;
+// 32768 x 1024 506, 360; column-major 2049 x 777 46, 479; 32768 x 1024 487, 801; 65536 x 1000 906, 799.
+static bool few_chains(int64_t chains, int64_t len) {
+  return chains <= 32768 && chains * ((len + 63) / 64 * 64 + 64) <= 36864 * len;
 }
 
 hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const q128 *A, int64_t lda,
@@ -313,12 +365,22 @@ hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const
   const int threads = 64;
   if (!colmajor) {
     const int64_t lanes = (incx == 1) ? 2 * m : m;
+    if (few_chains(lanes, (incx == 1) ? n / 2 : n)) {
+      hipLaunchKernelGGL(k_gemv_row_ref_scan, dim3((unsigned)((lanes + 3) / 4)), dim3(256), 0, st, m, n, alpha, A, lda,
+                         x, incx, beta, y, incy);
+      return hipGetLastError();
+    }
     const int64_t blocks = (lanes + threads - 1) / threads;
     if (!grid_fits(blocks, threads)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_gemv_row_ref, dim3((unsigned)blocks), dim3(threads), 0, st, m, n, alpha, A, lda, x,
                        incx, beta, y, incy);
   } else {
     hipLaunchKernelGGL(k_scale_vec, dim3(stride_blocks(n, 256)), dim3(256), 0, st, n, alpha, x, incx, ax);
+    if (few_chains(m, n)) {
+      hipLaunchKernelGGL(k_gemv_col_ref_scan, dim3((unsigned)((m + 7) / 8)), dim3(512), 0, st, m, n, A, lda, ax, beta, y,
+                         incy);
+      return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_gemv_col_ref, dim3(stride_blocks(m, threads)), dim3(threads), 0, st, m, n,
                        A, lda, ax, beta, y, incy);
   }
