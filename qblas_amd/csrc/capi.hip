@@ -279,6 +279,7 @@ int ws_acquire(StreamWorkspaces &W, size_t bytes, hipStream_t s, void **out,
 int ws_release(StreamWorkspaces &, hipStream_t) { return QBLAS_OK; }
 
 thread_local StreamWorkspaces t_ws;
+thread_local StreamWorkspaces t_rws;                    // the REFERENCE gemm's blocks of k
 thread_local StreamWorkspaces t_bws;                    // batched calls: prefix sums, OZAKI batch arrays
 thread_local StatusRef t_exact_status;                  // status words of the last EXACT/OZAKI-form call
 thread_local StatusRef t_oz_hdr;                        // header of the last OZAKI-form call
@@ -836,8 +837,23 @@ int dev_gemm(int mode, int layout, int64_t m, int64_t n, int64_t k, q128 alpha, 
   // gemm_simple for m,n,k <= 64 is one chain over all of k; otherwise blocks of kc
   // (level3.hpp:224-229, :244-246).  For k <= kc both are one block.
   const int64_t kc = (m <= 64 && n <= 64 && k <= 64) ? k : (int64_t)g_kc.load();
+  // without the workspace (a capture that has none, memory exhausted) the same result, slower
+  void *part = nullptr;
+  const size_t need = qbk::gemm_ref_ws(m, n, k, kc);
+  if (need) {
+    const std::string err = t_err;
+    // an allocation here must not end a capture that another thread has under way
+    hipStreamCaptureMode cm = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&cm);
+    if (ws_acquire(t_rws, need, s, &part) != QBLAS_OK) {
+      part = nullptr;
+      t_err = err;
+      (void)hipGetLastError();
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&cm);
+  }
   QB_CHECK(qbk::launch_gemm_ref(colmajor, m, n, k, kc, alpha, (const q128 *)A, lda, (const q128 *)B, ldb, beta,
-                                (q128 *)C, ldc, s));
+                                (q128 *)C, ldc, (q128 *)part, s));
   return QBLAS_OK;
 }
 

@@ -31,7 +31,8 @@ hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const
                            q128 *ax /* n, colmajor only */, hipStream_t st);
 hipError_t launch_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_t kc, q128 alpha, const q128 *A,
                            int64_t lda, const q128 *B, int64_t ldb, q128 beta, q128 *C, int64_t ldc,
-                           hipStream_t st);
+                           q128 *part /* gemm_ref_ws bytes, or null */, hipStream_t st);
+size_t gemm_ref_ws(int64_t m, int64_t n, int64_t k, int64_t kc);  // 0: launch_gemm_ref takes null
 hipError_t launch_zero(q128 *p, int64_t n, hipStream_t st);
 hipError_t launch_axpy(int64_t n, q128 alpha, const q128 *x, int64_t incx, q128 *y, int64_t incy, hipStream_t st);
 hipError_t launch_sqrt1(q128 *p, hipStream_t st);  // *p = RN(sqrt(*p))

@@ -11,6 +11,8 @@
 // chip one lane owns one (chain.hpp); where there are few, a wave does a chain's steps 64 at a time
 // with the same results (chain_scan.hpp).  The other forms (kernels_exact.hip, kernels_dd.hip,
 // kernels_ozaki.hip) trade the reference order for exact or wider accumulation.
+#include <algorithm>
+
 #include "chain_scan.hpp"
 #include "kernels.h"
 
@@ -214,7 +216,8 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
 
 // One lane per C element.  k is processed in blocks of kc; each block is a fresh chain t and
 // C = fma(alpha, t, mul(first ? beta : 1, C)) (level3.hpp:297-300 with the micro-kernel's
-// epilogue :102-109; gemm_simple :200-210 is the single-block case).  Layout-aware indexing for
+// epilogue :102-109; gemm_simple :200-210 is the single-block case); the product with 1 changes
+// nothing, so C = fma(alpha, t, C) over the blocks is one more chain, from beta * C.  Layout-aware indexing for
 // both layouts.  A workgroup computes a 16 x 16 tile of C: per step of GR_KT values of l, its 256
 // threads load the tile's 16 x GR_KT elements of A and GR_KT x 16 of B once (coalesced along the
 // contiguous dimension), unpack them into LDS, and every lane runs its chain over the step from
@@ -222,11 +225,15 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
 // subnormal, Inf or NaN is marked in LDS and taken from memory again for the packed slow path.
 // Bound by VALU issue: about 120 instructions per wave and multiply-add (chain.hpp).  4096^3
 // log-uniform: 244 ms = 563 quad GFLOP/s (577 ms with the 401-instruction step before).
+// part == null: the workgroup takes all blocks of k.  Else it takes block kb0 + blockIdx.z and writes its t to
+// part[(blockIdx.z n + j) m + i], for k_gemm_ref_fold: the blocks' chains do not depend on each other,
+// so a C of few tiles still fills the chip: 500 x 333 x 700 427 us (561 without), 64 x 64 x 2000 68 us (874).
 constexpr int GR_KT = 32;
 __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_t kc,
                                                   q128 alpha, const q128 *__restrict__ A, int64_t lda,
                                                   const q128 *__restrict__ B, int64_t ldb, q128 beta,
-                                                  q128 *__restrict__ C, int64_t ldc) {
+                                                  q128 *__restrict__ C, int64_t ldc, int64_t kb0,
+                                                  q128 *__restrict__ part) {
   __shared__ __attribute__((aligned(16))) cop sA[GR_KT][16];
   __shared__ __attribute__((aligned(16))) cop sB[GR_KT][16];
   const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
@@ -236,11 +243,13 @@ __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64
   const int64_t as_i = colmajor ? 1 : lda, as_l = colmajor ? lda : 1;
   const int64_t bs_l = colmajor ? 1 : ldb, bs_j = colmajor ? ldb : 1;
   q128 *ci = C + (colmajor ? j * ldc + i : i * ldc + j);
-  q128 c = live ? ld(ci) : q_zero(0);
   const q128 *ap = A + i * as_i;
   const q128 *bp = B + j * bs_j;
-  for (int64_t kk = 0; kk < k; kk += kc) {
-    const int64_t ke = (kk + kc < k) ? kk + kc : k;
+  const int64_t k0 = part ? (kb0 + blockIdx.z) * kc : 0, k1 = part ? (k0 + kc < k ? k0 + kc : k) : k;
+  cacc c;
+  if (!part) cacc_set(c, live ? mul_packed(beta, ld(ci)) : q_zero(0));
+  for (int64_t kk = k0; kk < k1; kk += kc) {
+    const int64_t ke = (kk + kc < k1) ? kk + kc : k1;
     cacc ch;
     cacc_init(ch);
     for (int64_t l0 = kk; l0 < ke; l0 += GR_KT) {
@@ -264,9 +273,26 @@ __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64
         }
       }
     }
-    c = fma_packed(alpha, cacc_get(ch), mul_packed(kk == 0 ? beta : q_one(), c));
+    if (live) {
+      if (!part) chain_fma(c, alpha, cacc_get(ch));
+      else st(part + ((int64_t)blockIdx.z * n + j) * m + i, cacc_get(ch));
+    }
   }
-  if (live) st(ci, c);
+  if (!part && live) st(ci, cacc_get(c));
+}
+// C = fma(alpha, t, C) over blocks kb0 .. kb0 + nb - 1, C = beta * C before block 0
+__global__ void __launch_bounds__(256) k_gemm_ref_fold(int colmajor, int64_t m, int64_t n, int64_t kb0, int64_t nb,
+                                                       q128 alpha, q128 beta, const q128 *__restrict__ part,
+                                                       q128 *__restrict__ C, int64_t ldc) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= m * n) return;
+  const int64_t j = e / m, i = e - j * m;
+  q128 *ci = C + (colmajor ? j * ldc + i : i * ldc + j);
+  cacc c;
+  cacc_set(c, kb0 == 0 ? mul_packed(beta, ld(ci)) : ld(ci));
+  const cop al = cop_unpack(alpha);
+  for (int64_t b = 0; b < nb; ++b) chain_fma(c, ld(part + b * m * n + e), alpha, al);
+  st(ci, cacc_get(c));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -387,13 +413,34 @@ hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const
   return hipGetLastError();
 }
 
+// Workspace for splitting the blocks of k over workgroups (0: not split): a workgroup of four waves is
+// a tile, and the chip takes 5 of them per CU at a time (LDS), so below about 2048 tiles it is idle in
+// part or for the last wave.  Rounds of at most 64 MB of t.
+size_t gemm_ref_ws(int64_t m, int64_t n, int64_t k, int64_t kc) {
+  const int64_t nb = (k + kc - 1) / kc, tm = (m + 15) / 16, tn = (n + 15) / 16;
+  if (nb < 2 || tm > 2048 || tn > 2048 || tm * tn >= 2048) return 0;
+  const int64_t t = 16 * m * n, fit = std::min<int64_t>((int64_t)(64 << 20) / t, 32768);
+  return (size_t)(t * std::min(nb, fit));
+}
+
 hipError_t launch_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_t kc, q128 alpha, const q128 *A,
-                           int64_t lda, const q128 *B, int64_t ldb, q128 beta, q128 *C, int64_t ldc,
+                           int64_t lda, const q128 *B, int64_t ldb, q128 beta, q128 *C, int64_t ldc, q128 *part,
                            hipStream_t st) {
   if (!grid_fits((n + 15) / 16, 256)) return hipErrorInvalidValue;
-  dim3 grid((unsigned)((n + 15) / 16), (unsigned)((m + 15) / 16));
-  hipLaunchKernelGGL(k_gemm_ref, grid, dim3(256), 0, st, colmajor, m, n, k, kc, alpha, A, lda, B, ldb, beta, C,
-                     ldc);
+  const unsigned tn = (unsigned)((n + 15) / 16), tm = (unsigned)((m + 15) / 16);
+  if (!part) {
+    hipLaunchKernelGGL(k_gemm_ref, dim3(tn, tm), dim3(256), 0, st, colmajor, m, n, k, kc, alpha, A, lda, B, ldb, beta,
+                       C, ldc, (int64_t)0, part);
+    return hipGetLastError();
+  }
+  const int64_t nb = (k + kc - 1) / kc, zb = (int64_t)(gemm_ref_ws(m, n, k, kc) / (size_t)(16 * m * n));
+  for (int64_t z = 0; z < nb; z += zb) {
+    const int64_t c = nb - z < zb ? nb - z : zb;
+    hipLaunchKernelGGL(k_gemm_ref, dim3(tn, tm, (unsigned)c), dim3(256), 0, st, colmajor, m, n, k, kc, alpha, A, lda, B,
+                       ldb, beta, C, ldc, z, part);
+    hipLaunchKernelGGL(k_gemm_ref_fold, dim3((unsigned)((m * n + 255) / 256)), dim3(256), 0, st, colmajor, m, n, z, c,
+                       alpha, beta, part, C, ldc);
+  }
   return hipGetLastError();
 }
 
