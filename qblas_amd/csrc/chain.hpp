@@ -5,41 +5,46 @@
 //
 //   cop   an operand, unpacked once: four 29-bit limbs of the 113-bit significand (so the columns
 //         of a product, sums of at most four 58-bit products, fit 64 bits), exponent, sign as a
-//         mask and the number of trailing zero bits.  Zero, subnormal, Inf and NaN operands carry
-//         the exponent CH_ESPECIAL, which no step's range check passes.
+//         mask and the number of trailing zero bits.  Zero, subnormal, Inf and NaN operands, and
+//         exponents beyond +-CH_OMAX, carry the exponent CH_ESPECIAL, which no step takes.
 //   cacc  the accumulator: a 160-bit two's complement frame W (five 32-bit words, the lowest always
 //         zero between steps) with value W 2^(E-152).  The leading bit lies anywhere in bits
 //         146..158, so a step that moves it by a few bits needs no renormalisation.
 //
 // One step: the product's columns (16 v_mad_u64_u32, each column's carry the next one's addend), its
 // bits 72.. as a frame with leading bit 152/153 at exponent ea + eb; the frame with the lower
-// exponent is shifted right onto the other one's grid (whole words by bit masks, then a funnel),
-// added in two's complement, and rounded in place at the 113th bit below the leading one.  Bits of the product
-// below the grid act through a sticky bit only, which its trailing zeros (the sum of the operands')
-// decide without looking at them: floor(x) plus a sticky bit rounds x correctly, as the grid lies
-// at least 34 bits below the rounding position.  About 120 VALU instructions; 401 with sign and
-// magnitude in 64-bit words and a case per exponent order.
-// Left to the packed operation (chain_slow): special operands or accumulators, exponents near the
-// ends of the range, an accumulator more than 32 bits below the product's grid, and sums that
+// exponent is shifted right onto the other one's grid (the product by whole words with bit masks, then
+// a funnel; the accumulator by the funnel), added in two's complement, and rounded in place at the
+// 113th bit below the leading one.  Bits of the product below the grid act through a sticky bit only,
+// which its trailing zeros (the sum of the operands') decide without looking at them: floor(x) plus a
+// sticky bit rounds x correctly, as the grid lies at least 34 bits below the rounding position.
+// About 85 VALU instructions, 105 with a product 2^32 below the accumulator in the wave; 401 with sign
+// and magnitude in 64-bit words and a case per exponent order.  gemm 2048^3: 21.9 ms on uniform entries
+// (27.7 ms with both operands' shifts in every step).
+// Left to the packed operation (chain_slow): special operands, exponents near the ends of the range, a
+// zero accumulator without cacc_first, one more than 31 bits below the product's grid, and sums that
 // cancel by 26 bits or more.
 #pragma once
 #include "q128.hpp"
 
 namespace qb {
 
-constexpr int32_t CH_ESPECIAL = 1 << 22;  // exponent of an operand or accumulator the step does not take
+constexpr int32_t CH_ESPECIAL = 1 << 22;  // exponent of an operand the step does not take
+constexpr int32_t CH_APACKED = 1 << 24;   // exponent of an accumulator that is held packed
 constexpr int32_t CH_EZERO = -(1 << 24);  // exponent of a zero accumulator
-constexpr int32_t CH_EMAX = 16300;        // |exponent| of a step: every result is then a normal number
+constexpr int32_t CH_OMAX = 8100;         // |exponent| of an operand: a product's lies within 16200
+constexpr int32_t CH_EMAX = 16300;        // |exponent| of an accumulator's frame: every sum is a normal number
+constexpr uint32_t CH_DRANGE = 1u << 17;  // exponent differences of a step: -31 .. 2^17 - 31
 
 struct cop {
   uint32_t l[4];  // significand = sum l[i] 2^(29 i)
   int32_t e;      // value = (-1)^neg significand 2^(e - 112)
   uint32_t neg;   // 0 or ~0
-  int32_t tz;     // trailing zero bits of the significand
+  int32_t tz;     // trailing zero bits of the significand, less 36 (a product's frame begins at bit 72)
   uint32_t pad;
 };
 struct cacc {
-  uint32_t w[4];  // words 1..4 of the frame (word 0 is zero); the packed value if E == CH_ESPECIAL
+  uint32_t w[4];  // words 1..4 of the frame (word 0 is zero); the packed value if E == CH_APACKED
   int32_t E;
 };
 
@@ -73,6 +78,14 @@ QB_HD uint32_t ch_mask(uint32_t x) {
   return 0u - ((x >> B) & 1u);
 #endif
 }
+QB_HD bool ch_any(bool x) {  // of the wave's active lanes: a branch the whole wave takes or skips
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __ballot(x) != 0;
+#else
+  return x;
+#endif
+}
+QB_HD int32_t ch_clamp(int32_t x, int32_t lo, int32_t hi) { return x < lo ? lo : (x > hi ? hi : x); }
 QB_HD uint32_t ch_sel(uint32_t mask, uint32_t a, uint32_t b) { return (mask & a) | (~mask & b); }
 QB_HD uint32_t ch_addc(uint32_t a, uint32_t b, uint32_t ci, uint32_t &co) {
 #if defined(__clang__)
@@ -102,9 +115,10 @@ QB_HD cop cop_unpack(q128 a) {
   r.l[1] = (uint32_t)(a.lo >> 29) & 0x1fffffffu;
   r.l[2] = ch_alignbit((uint32_t)mh, (uint32_t)(a.lo >> 32), 26) & 0x1fffffffu;
   r.l[3] = (uint32_t)(mh >> 23);
-  r.e = (be == 0 || be == 0x7fffu) ? CH_ESPECIAL : (int32_t)be - QBIAS;
+  r.e = (int32_t)be - QBIAS;
+  if ((uint32_t)(r.e + CH_OMAX) > (uint32_t)(2 * CH_OMAX)) r.e = CH_ESPECIAL;
   r.neg = (uint32_t)((int32_t)(uint32_t)(a.hi >> 32) >> 31);
-  r.tz = a.lo ? ch_ctz64(a.lo) : 64 + ch_ctz64(mh);
+  r.tz = (a.lo ? ch_ctz64(a.lo) : 64 + ch_ctz64(mh)) - 36;
   r.pad = 0;
   return r;
 }
@@ -114,12 +128,13 @@ QB_HD void cacc_init(cacc &c) {
   c.E = CH_EZERO;
 }
 QB_HD void cacc_set(cacc &c, q128 v) {
-  if (q_bexp(v) == 0x7fffu) {
+  const int32_t e = (int32_t)q_bexp(v) - QBIAS;
+  if ((e < 50 - CH_EMAX && !q_iszero(v)) || e > CH_EMAX - 50) {
     c.w[0] = (uint32_t)v.lo;
     c.w[1] = (uint32_t)(v.lo >> 32);
     c.w[2] = (uint32_t)v.hi;
     c.w[3] = (uint32_t)(v.hi >> 32);
-    c.E = CH_ESPECIAL;
+    c.E = CH_APACKED;
     return;
   }
   const uq u = unpack_finite(v);
@@ -140,7 +155,7 @@ QB_HD void cacc_set(cacc &c, q128 v) {
 }
 QB_HD q128 cacc_get(const cacc &c) {
   uint64_t lo = ((uint64_t)c.w[1] << 32) | c.w[0], hi = ((uint64_t)c.w[3] << 32) | c.w[2];
-  if (c.E == CH_ESPECIAL) return q_make(lo, hi);
+  if (c.E == CH_APACKED) return q_make(lo, hi);
   if (c.E == CH_EZERO) return q_zero(c.w[0]);
   const uint64_t x = (uint64_t)((int64_t)hi >> 63);
   lo = (lo ^ x) + (x & 1);
@@ -158,77 +173,75 @@ QB_HD q128 cacc_get(const cacc &c) {
 // columns of the product of two significands: column k at bit 29 k, each one's carry over 29 bits
 // added into the next (the digits are the low 29 bits of columns 0..5 and all of column 6)
 QB_HD void cop_columns(uint64_t (&c)[7], const cop &a, const cop &b) {
-  c[0] = (uint64_t)a.l[0] * b.l[0];
-  c[1] = (uint64_t)a.l[0] * b.l[1] + (c[0] >> 29);
-  c[1] = (uint64_t)a.l[1] * b.l[0] + c[1];
-  c[2] = (uint64_t)a.l[0] * b.l[2] + (c[1] >> 29);
-  c[2] = (uint64_t)a.l[1] * b.l[1] + c[2];
-  c[2] = (uint64_t)a.l[2] * b.l[0] + c[2];
-  c[3] = (uint64_t)a.l[0] * b.l[3] + (c[2] >> 29);
-  c[3] = (uint64_t)a.l[1] * b.l[2] + c[3];
-  c[3] = (uint64_t)a.l[2] * b.l[1] + c[3];
-  c[3] = (uint64_t)a.l[3] * b.l[0] + c[3];
-  c[4] = (uint64_t)a.l[1] * b.l[3] + (c[3] >> 29);
-  c[4] = (uint64_t)a.l[2] * b.l[2] + c[4];
-  c[4] = (uint64_t)a.l[3] * b.l[1] + c[4];
-  c[5] = (uint64_t)a.l[2] * b.l[3] + (c[4] >> 29);
-  c[5] = (uint64_t)a.l[3] * b.l[2] + c[5];
-  c[6] = (uint64_t)a.l[3] * b.l[3] + (c[5] >> 29);
+#pragma unroll
+  for (int k = 0; k < 7; ++k) {
+    const int lo = k < 4 ? 0 : k - 3, hi = k < 4 ? k : 3;
+    uint64_t t = k ? c[k - 1] >> 29 : 0;
+#pragma unroll
+    for (int i = lo; i <= hi; ++i) {
+      t += (uint64_t)a.l[i] * b.l[k - i];
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm("" : "+v"(t));  // keep the carry the first addend: reassociated, it costs an addition of its own
+#endif
+    }
+    c[k] = t;
+  }
 }
 // acc = RN(a*b + acc).  Returns false, leaving acc as it was, when the packed operation has to do it.
 QB_HD bool cacc_step(cacc &acc, const cop &a, const cop &b) {
   uint64_t k[7];
   cop_columns(k, a, b);
-  // bits 72.. of the product (29-bit digits of the columns) as the frame, its sign applied as a
-  // complement; the missing +1 goes in as the sum's carry when nothing is lost below the grid
-  const uint32_t neg = a.neg ^ b.neg;
+  // bits 72.. of the product (29-bit digits of the columns) as the frame
   uint32_t P[5];
-  P[0] = ((((uint32_t)k[2] >> 14) & 0x7fffu) | ((uint32_t)k[3] << 15)) ^ neg;
-  P[1] = ((((uint32_t)k[3] >> 17) & 0xfffu) | ((uint32_t)k[4] << 12)) ^ neg;
-  P[2] = ((((uint32_t)k[4] >> 20) & 0x1ffu) | ((uint32_t)k[5] << 9)) ^ neg;
-  P[3] = ((((uint32_t)k[5] >> 23) & 0x3fu) | ((uint32_t)k[6] << 6)) ^ neg;
-  P[4] = ch_alignbit((uint32_t)(k[6] >> 32), (uint32_t)k[6], 26) ^ neg;
+  P[0] = (((uint32_t)k[2] >> 14) & 0x7fffu) | ((uint32_t)k[3] << 15);
+  P[1] = (((uint32_t)k[3] >> 17) & 0xfffu) | ((uint32_t)k[4] << 12);
+  P[2] = (((uint32_t)k[4] >> 20) & 0x1ffu) | ((uint32_t)k[5] << 9);
+  P[3] = (((uint32_t)k[5] >> 23) & 0x3fu) | ((uint32_t)k[6] << 6);
+  P[4] = ch_alignbit((uint32_t)(k[6] >> 32), (uint32_t)k[6], 26);
   const int32_t Ep = a.e + b.e;
   const int32_t d = acc.E - Ep;
-  const uint32_t pbig = ch_mask<31>((uint32_t)d);
-  const int32_t ad = d < 0 ? -d : d;
-  const uint32_t sh = (uint32_t)(ad < 159 ? ad : 159);
-  int32_t E = Ep > acc.E ? Ep : acc.E;
-  // X: the frame that stays, T: the one that is shifted
-  uint32_t X[5], T[5];
-  X[0] = P[0] & pbig;
-  T[0] = P[0] & ~pbig;
+  // d > 0: the product moves right onto the accumulator's grid, by a funnel, after whole words where a
+  // lane has a product 2^32 and more below (none has with entries of one scale)
+  const int32_t sh = ch_clamp(d, 0, 159);
+  if (ch_any(sh >= 32)) {
+    const uint32_t m4 = ch_mask<7>((uint32_t)sh), m2 = ch_mask<6>((uint32_t)sh), m1 = ch_mask<5>((uint32_t)sh);
+    uint32_t Q[5];
+    Q[0] = ch_sel(m4, P[4], P[0]);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    X[i + 1] = ch_sel(pbig, P[i + 1], acc.w[i]);
-    T[i + 1] = ch_sel(pbig, acc.w[i], P[i + 1]);
+    for (int i = 1; i < 5; ++i) Q[i] = P[i] & ~m4;
+    P[0] = ch_sel(m2, Q[2], Q[0]);
+    P[1] = ch_sel(m2, Q[3], Q[1]);
+    P[2] = ch_sel(m2, Q[4], Q[2]);
+    P[3] = Q[3] & ~m2;
+    P[4] = Q[4] & ~m2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) P[i] = ch_sel(m1, P[i + 1], P[i]);
+    P[4] &= ~m1;
   }
-  const uint32_t sg = ch_mask<31>(T[4]), m4 = ch_mask<7>(sh), m2 = ch_mask<6>(sh), m1 = ch_mask<5>(sh);
-  uint32_t U[5], V[5], Q[5];
-  U[0] = ch_sel(m4, T[4], T[0]);
+  // its sign is applied as a complement; the missing +1 goes in as the sum's carry when no bit of the
+  // product lies below the grid
+  const uint32_t neg = a.neg ^ b.neg;
 #pragma unroll
-  for (int i = 1; i < 5; ++i) U[i] = ch_sel(m4, sg, T[i]);
-  V[0] = ch_sel(m2, U[2], U[0]);
-  V[1] = ch_sel(m2, U[3], U[1]);
-  V[2] = ch_sel(m2, U[4], U[2]);
-  V[3] = ch_sel(m2, sg, U[3]);
-  V[4] = ch_sel(m2, sg, U[4]);
+  for (int i = 0; i < 4; ++i) P[i] = ch_alignbit(P[i + 1], P[i], (uint32_t)sh) ^ neg;
+  P[4] = (P[4] >> (sh & 31)) ^ neg;
+  const bool st = a.tz + b.tz < sh;
+  // d < 0: the accumulator moves onto the product's grid, by at most 31 bits (word 0 takes them)
+  uint32_t A[5] = {0, acc.w[0], acc.w[1], acc.w[2], acc.w[3]};
+  if (ch_any(d < 0)) {
+    const uint32_t sa = (uint32_t)(d < 0 ? -d : 0);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) Q[i] = ch_sel(m1, V[i + 1], V[i]);
-  Q[4] = ch_sel(m1, sg, V[4]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) T[i] = ch_alignbit(Q[i + 1], Q[i], sh);
-  T[4] = (uint32_t)((int32_t)Q[4] >> (sh & 31));
-  // bits of the product below the grid
-  const bool st = a.tz + b.tz - 72 < (d > 0 ? d : 0);
+    for (int i = 0; i < 4; ++i) A[i] = ch_alignbit(A[i + 1], A[i], sa);
+    A[4] = (uint32_t)((int32_t)A[4] >> (sa & 31));
+  }
   uint32_t F[5], c = (uint32_t)((neg != 0) & !st);
 #pragma unroll
-  for (int i = 0; i < 5; ++i) F[i] = ch_addc(X[i], T[i], c, c);
-  // range: exponents; an accumulator with bits below the product's grid; a sum in words 0..3 only
+  for (int i = 0; i < 5; ++i) F[i] = ch_addc(P[i], A[i], c, c);
+  int32_t E = Ep > acc.E ? Ep : acc.E;
   uint32_t fb = ch_signbits(F[4]);
-  if (((uint32_t)(E + CH_EMAX) > (uint32_t)(2 * CH_EMAX)) | ((uint32_t)(-33 - d) < (1u << 20)) | (fb > 31u)) return false;
   uint32_t w0 = F[0] | (uint32_t)st;
-  if (fb - 2u > 11u) {  // the leading bit left 146..157: to 153
+  if (((uint32_t)(d + 31) > CH_DRANGE) | (fb - 2u > 11u)) {
+    // special or far apart; a sum in words 0..3 only; else the leading bit left 146..157: to 153
+    if (((uint32_t)(d + 31) > CH_DRANGE) | (fb > 31u)) return false;
     if (fb < 2u) {
       const uint32_t r = 6 - fb;
       const uint32_t lost = w0 << (32 - r);
@@ -244,26 +257,32 @@ QB_HD bool cacc_step(cacc &acc, const cop &a, const cop &b) {
       w0 = (w0 << (32 - r)) | (w0 & 1u);  // the sticky bit stays at the bottom
     }
     E += 6 - (int32_t)fb;
+    if ((uint32_t)(E + CH_EMAX) > (uint32_t)(2 * CH_EMAX)) return false;
     fb = 6;
   }
-  // round to nearest even at bit 47 - fb: bit 15 - fb of word 1, half = 2^14 >> fb
-  uint32_t w1 = F[1] | (w0 < 1u ? w0 : 1u);
-  const uint32_t half = 0x4000u >> fb;
-  const uint32_t lsb = (w1 >> (15u - fb)) & 1u;
-  c = 0;
-  w1 = ch_addc(w1, half - 1u + lsb, 0u, c);
-  acc.w[0] = w1 & (0u - half - half);
+  // round to nearest even at bit 47 - fb, bit 15 - fb of word 1: half less one unit is added, and one
+  // unit more if anything lies below word 1 or the result is odd
+  c = (uint32_t)((w0 | ((F[1] >> (15u - fb)) & 1u)) != 0);
+  acc.w[0] = ch_addc(F[1], 0x3fffu >> fb, c, c) & ~(0x7fffu >> fb);
   acc.w[1] = ch_addc(F[2], 0u, c, c);
   acc.w[2] = ch_addc(F[3], 0u, c, c);
   acc.w[3] = ch_addc(F[4], 0u, c, c);
   acc.E = E;
   return true;
 }
+// before a chain's first step: a zero accumulator takes the product's grid, so the step is an ordinary one
+QB_HD void cacc_first(cacc &acc, const cop &a, const cop &b) {
+  if (acc.E == CH_EZERO && a.e != CH_ESPECIAL && b.e != CH_ESPECIAL) {
+    acc.w[0] = 0;  // -0 + x = x
+    acc.E = a.e + b.e;
+  }
+}
 QB_HD void chain_slow(cacc &acc, q128 a, q128 b) { cacc_set(acc, fma_packed(a, b, cacc_get(acc))); }
 
 // acc = RN(a*b + acc) for packed a, b, with b's unpacked form at hand
 QB_HD void chain_fma(cacc &acc, q128 a, q128 b, const cop &B) {
-  if (!cacc_step(acc, cop_unpack(a), B)) chain_slow(acc, a, b);
+  const cop A = cop_unpack(a);
+  if (!cacc_step(acc, A, B)) chain_slow(acc, a, b);
 }
 QB_HD void chain_fma(cacc &acc, q128 a, q128 b) { chain_fma(acc, a, b, cop_unpack(b)); }
 

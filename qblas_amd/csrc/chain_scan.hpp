@@ -108,7 +108,9 @@ QB_HD void sstate_step(sstate &s, q128 a, q128 b) {
       for (int i = 0; i < 4; ++i) acc.w[i] = ch_addc(s.w[i] ^ s.neg, 0u, c, c);
       acc.E = s.b + 8 - SC_LOW;
     }
-    if (cacc_step(acc, cop_unpack(a), cop_unpack(b))) {
+    const cop A = cop_unpack(a), B = cop_unpack(b);
+    cacc_first(acc, A, B);
+    if (cacc_step(acc, A, B)) {
       sstate_from_sum(s, acc.w, acc.E - 8);
       return;
     }
@@ -142,7 +144,7 @@ QB_HD sprod sc_product(q128 qa, q128 qb) {
   r.F[3] = (((uint32_t)c[5] >> 18) & 0x7ffu) | ((uint32_t)c[6] << 11);
   r.F[4] = ch_alignbit((uint32_t)(c[6] >> 32), (uint32_t)c[6], 21);
   r.neg = a.neg ^ b.neg;
-  r.tz = a.tz + b.tz;
+  r.tz = a.tz + b.tz + 72;
   r.Ep = a.e + b.e;
   r.bad = r.Ep < -SC_EMAX || r.Ep > SC_EMAX;  // CH_ESPECIAL operands among them
   if (a.e == CH_ESPECIAL || b.e == CH_ESPECIAL) {

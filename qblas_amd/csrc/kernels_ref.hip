@@ -223,11 +223,11 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
 // contiguous dimension), unpack them into LDS, and every lane runs its chain over the step from
 // LDS, in the same order l = kk, kk + 1, ... as the reference.  An operand that is zero,
 // subnormal, Inf or NaN is marked in LDS and taken from memory again for the packed slow path.
-// Bound by VALU issue: about 120 instructions per wave and multiply-add (chain.hpp).  4096^3
-// log-uniform: 244 ms = 563 quad GFLOP/s (577 ms with the 401-instruction step before).
+// Bound by VALU issue: 85 to 105 instructions per wave and multiply-add (chain.hpp).  4096^3
+// log-uniform: 222 ms = 619 quad GFLOP/s (577 ms with a 401-instruction step); 2048^3 uniform 21.9 ms.
 // part == null: the workgroup takes all blocks of k.  Else it takes block kb0 + blockIdx.z and writes its t to
 // part[(blockIdx.z n + j) m + i], for k_gemm_ref_fold: the blocks' chains do not depend on each other,
-// so a C of few tiles still fills the chip: 500 x 333 x 700 427 us (561 without), 64 x 64 x 2000 68 us (874).
+// so a C of few tiles still fills the chip: 500 x 333 x 700 340 us (440 without), 64 x 64 x 2000 70 us (740).
 constexpr int GR_KT = 32;
 __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_t kc,
                                                   q128 alpha, const q128 *__restrict__ A, int64_t lda,
@@ -267,6 +267,7 @@ __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64
       }
       __syncthreads();
       if (live) {
+        if (l0 == kk) cacc_first(ch, sA[0][ti], sB[0][tj]);
         for (int q = 0; q < lt; ++q) {
           if (!cacc_step(ch, sA[q][ti], sB[q][tj]))
             chain_slow(ch, ld(ap + (l0 + q) * as_l), ld(bp + (l0 + q) * bs_l));

@@ -104,7 +104,9 @@ int main(int argc, char **argv) {
         operands(kind, i, a, b);
         ref = fma_packed(a, b, ref);
         ++steps;
-        if (!cacc_step(acc, cop_unpack(a), cop_unpack(b))) {
+        const cop A = cop_unpack(a), B = cop_unpack(b);
+        if (i == 0) cacc_first(acc, A, B);
+        if (!cacc_step(acc, A, B)) {
           ++slow;
           chain_slow(acc, a, b);
         }
