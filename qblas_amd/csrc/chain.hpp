@@ -279,11 +279,96 @@ QB_HD void cacc_first(cacc &acc, const cop &a, const cop &b) {
 }
 QB_HD void chain_slow(cacc &acc, q128 a, q128 b) { cacc_set(acc, fma_packed(a, b, cacc_get(acc))); }
 
+QB_HD q128 chain_mul(q128 a, q128 b) {  // mul_packed(a, b)
+  const cop A = cop_unpack(a), B = cop_unpack(b);
+  cacc z;
+  cacc_init(z);
+  z.w[0] = 1;  // -0
+  cacc_first(z, A, B);
+  if (!cacc_step(z, A, B)) chain_slow(z, a, b);
+  return cacc_get(z);
+}
 // acc = RN(a*b + acc) for packed a, b, with b's unpacked form at hand
 QB_HD void chain_fma(cacc &acc, q128 a, q128 b, const cop &B) {
   const cop A = cop_unpack(a);
   if (!cacc_step(acc, A, B)) chain_slow(acc, a, b);
 }
 QB_HD void chain_fma(cacc &acc, q128 a, q128 b) { chain_fma(acc, a, b, cop_unpack(b)); }
+
+// y_i = fma(alpha, sum, mul(beta, y_i)) with sum = c0 + c1 (two chains), the odd tail's fma applied;
+// the four operations as one loop, so the step's code is there once
+QB_HD q128 gemv_row_end(q128 c0, q128 c1, int pair, int odd, q128 ta, q128 tx, q128 alpha,
+                                             q128 beta, q128 y) {
+  q128 by = q_zero(1), sum = c0;
+#pragma unroll 1
+  for (int op = 0; op < 4; ++op) {
+    if ((op == 1 && !pair) || (op == 2 && !odd)) continue;
+    const q128 a = op == 0 ? beta : op == 1 ? c1 : op == 2 ? ta : alpha;
+    const q128 b = op == 0 ? y : op == 1 ? q_one() : op == 2 ? tx : sum;
+    cacc acc;
+    cacc_set(acc, (op == 0 || op == 3) ? by : sum);
+    chain_fma(acc, a, b);
+    const q128 r = cacc_get(acc);
+    if (op == 0 || op == 3) by = r;
+    else sum = r;
+  }
+  return by;
+}
+#if defined(__HIPCC__)
+// One chain per lane along a row of a matrix, all lanes of a wave against the same vector:
+//   ch = RN(a[s sa] x(s per + par) + ch)   for s = 0..steps-1
+// with per = 1, or 2 when lanes of odd and even par (0 or 1) take every other element.  The wave unpacks
+// 32 elements of x at a time into its own LDS; every lane of the wave calls (live: it has a chain), and
+// steps, per and x are the same in all of them.  Elements of a are loaded four steps at a time, a group
+// ahead, and pass through the lane's LDS slots, so the step's code is there once: a row's lane pair then
+// asks for a whole 128-byte line at once.  With a load per step the lines of a wave's 32 rows were
+// fetched again and again (13.8 GB for the 9.0 GB of a batch of 2048 gemv problems).
+constexpr int LC_GROUP = 4;
+struct chain_lds {
+  cop u[32];
+  q128 p[32];
+  uint4 a[LC_GROUP][64];
+};
+template <typename X>
+__device__ __forceinline__ void lane_chain(cacc &ch, bool live, const q128 *__restrict__ a, int64_t sa, int64_t steps,
+                                           int per, int par, const X x, chain_lds &lds) {
+  const int lane = (int)(threadIdx.x & 63), span = 32 / per;
+  uint4 v[LC_GROUP];
+#pragma unroll
+  for (int g = 0; g < LC_GROUP; ++g) {
+    v[g] = make_uint4(0, 0, 0, 0);
+    if (live && g < steps) v[g] = *reinterpret_cast<const uint4 *>(a + g * sa);
+  }
+  for (int64_t s0 = 0; s0 < steps; s0 += span) {
+    const int cnt = (int)((steps - s0 < span) ? steps - s0 : span);
+    __builtin_amdgcn_wave_barrier();  // the wave's reads of the span before are done
+    if (lane < cnt * per) {
+      const q128 e = x(s0 * per + lane);
+      lds.p[lane] = e;
+      lds.u[lane] = cop_unpack(e);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (!live) continue;
+    for (int q0 = 0; q0 < cnt; q0 += LC_GROUP) {
+#pragma unroll
+      for (int g = 0; g < LC_GROUP; ++g) lds.a[g][lane] = v[g];
+      a += LC_GROUP * sa;
+#pragma unroll
+      for (int g = 0; g < LC_GROUP; ++g)
+        if (s0 + q0 + LC_GROUP + g < steps) v[g] = *reinterpret_cast<const uint4 *>(a + g * sa);
+      const int ge = cnt - q0 < LC_GROUP ? cnt - q0 : LC_GROUP;
+      for (int g = 0; g < ge; ++g) {
+        const uint4 w = lds.a[g][lane];
+        const q128 e = q_make(((uint64_t)w.y << 32) | w.x, ((uint64_t)w.w << 32) | w.z);
+        const int k = (q0 + g) * per + par;
+        const cop E = cop_unpack(e);
+        if (s0 + q0 + g == 0) cacc_first(ch, E, lds.u[k]);
+        if (!cacc_step(ch, E, lds.u[k])) chain_slow(ch, e, lds.p[k]);
+      }
+    }
+  }
+}
+#endif  // __HIPCC__
 
 }  // namespace qb

@@ -260,6 +260,7 @@ __global__ void __launch_bounds__(256) k_gemm_batched_dd(const qblas_gemm_proble
 __global__ void __launch_bounds__(256) k_gemv_batched_ref(const qblas_gemv_problem *__restrict__ P, int64_t count,
                                                           const int64_t *__restrict__ start, int colmajor,
                                                           uint32_t *__restrict__ queue) {
+  __shared__ __attribute__((aligned(16))) chain_lds lds[4];
   const int lane = threadIdx.x & 63;
   const int64_t total = start[count];
   const int64_t waves = (int64_t)gridDim.x * 4;
@@ -276,45 +277,31 @@ __global__ void __launch_bounds__(256) k_gemv_batched_ref(const qblas_gemv_probl
     const q128 *x = (const q128 *)v.x;
     q128 *y = (q128 *)v.y;
     const q128 alpha = qv(v.alpha), beta = qv(v.beta);
+    // RowMajor, incx == 1: two lane chains per row (level2.hpp:35-38 with dot_kernel_vectorized), rows
+    // ul*32 + lane/2; else one chain per row, rows ul*64 + lane.  ColMajor (level2.hpp:63-80):
+    // y_i = mul(beta, y_i), then fma(A_ij, mul(alpha, x_j), y_i) over j
+    const int per = (!colmajor && incx == 1) ? 2 : 1, par = lane & (per - 1);
+    const int64_t i = ul * (64 / per) + lane / per;
+    const bool live = i < m;
+    q128 *yi = y + i * incy;
     cacc ch;
-    if (!colmajor && incx == 1) {
-      // two lane chains per row (level2.hpp:35-38 with dot_kernel_vectorized), rows ul*32 + lane/2
-      const int64_t i = ul * 32 + (lane >> 1);
-      const int par = lane & 1;
-      const bool live = i < m;
-      cacc_init(ch);
-      if (live) {
-        const q128 *row = A + i * lda;
-        const int64_t pairs = n / 2;
-        for (int64_t jj = 0; jj < pairs; ++jj) chain_fma(ch, bld(row + 2 * jj + par), bld(x + 2 * jj + par));
-      }
-      const q128 mine = cacc_get(ch);
-      const uint64_t olo = (uint64_t)__shfl_xor((unsigned long long)mine.lo, 1);
-      const uint64_t ohi = (uint64_t)__shfl_xor((unsigned long long)mine.hi, 1);
-      if (live && par == 0) {
-        q128 sum = add_packed(mine, q_make(olo, ohi));
-        if (n & 1) sum = fma_packed(bld(A + i * lda + n - 1), bld(x + n - 1), sum);
-        q128 *yi = y + i * incy;
-        bst(yi, fma_packed(alpha, sum, mul_packed(beta, bld(yi))));
-      }
-    } else if (!colmajor) {
-      const int64_t i = ul * 64 + lane;
-      if (i < m) {
-        cacc_init(ch);
-        const q128 *row = A + i * lda;
-        for (int64_t j = 0; j < n; ++j) chain_fma(ch, bld(row + j), bld(x + j * incx));
-        q128 *yi = y + i * incy;
-        bst(yi, fma_packed(alpha, cacc_get(ch), mul_packed(beta, bld(yi))));
-      }
-    } else {
-      // level2.hpp:63-80: y_i = mul(beta, y_i), then fma(A_ij, mul(alpha, x_j), y_i) over j
-      const int64_t i = ul * 64 + lane;
-      if (i < m) {
-        q128 *yi = y + i * incy;
-        cacc_set(ch, mul_packed(beta, bld(yi)));
-        for (int64_t j = 0; j < n; ++j) chain_fma(ch, bld(A + j * lda + i), mul_packed(alpha, bld(x + j * incx)));
-        bst(yi, cacc_get(ch));
-      }
+    cacc_init(ch);
+    if (colmajor && live) cacc_set(ch, chain_mul(beta, bld(yi)));
+    lane_chain(ch, live, A + (colmajor ? i : i * lda + par), colmajor ? lda : per, n / per, per, par,
+               [=](int64_t j) {
+                 const q128 v = bld(x + j * incx);
+                 return colmajor ? chain_mul(alpha, v) : v;
+               },
+               lds[threadIdx.x >> 6]);
+    q128 r = cacc_get(ch);
+    const uint64_t olo = (uint64_t)__shfl_xor((unsigned long long)r.lo, 1);
+    const uint64_t ohi = (uint64_t)__shfl_xor((unsigned long long)r.hi, 1);
+    if (live && par == 0) {
+      const int odd = per == 2 && (n & 1);
+      if (!colmajor)
+        r = gemv_row_end(r, q_make(olo, ohi), per == 2, odd, odd ? bld(A + i * lda + n - 1) : q_zero(0),
+                         odd ? bld(x + n - 1) : q_zero(0), alpha, beta, bld(yi));
+      bst(yi, r);
     }
     u = waves + (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)ticket);  // lane 0's ticket
   }

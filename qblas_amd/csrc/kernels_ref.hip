@@ -100,58 +100,25 @@ __global__ void __launch_bounds__(64) k_dot_ref_sum(int T, const q128 *__restric
 // on the row, level2.hpp:35-38); the pair is combined with a lane exchange, the odd tail applied,
 // then y_i = fma(alpha, sum, mul(beta, y_i)) (level2.hpp:48).
 // RowMajor, incx != 1: one chain per row (level2.hpp:41-44).
-__global__ void k_gemv_row_ref(int64_t m, int64_t n, q128 alpha, const q128 *__restrict__ A, int64_t lda,
-                               const q128 *__restrict__ x, int64_t incx, q128 beta, q128 *__restrict__ y,
-                               int64_t incy) {
-  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(64) k_gemv_row_ref(int64_t m, int64_t n, q128 alpha, const q128 *__restrict__ A,
+                                                     int64_t lda, const q128 *__restrict__ x, int64_t incx, q128 beta,
+                                                     q128 *__restrict__ y, int64_t incy) {
+  __shared__ __attribute__((aligned(16))) chain_lds lds;
+  const int pair = incx == 1, lane = (int)threadIdx.x, p = lane & pair;
+  const int64_t i = (int64_t)blockIdx.x * (64 >> pair) + (lane >> pair);
+  const bool live = i < m;
+  const q128 *row = A + i * lda;
   cacc ch;
   cacc_init(ch);
-  if (incx == 1) {
-    const int64_t i = tid >> 1;
-    const int p = (int)(tid & 1);
-    const bool live = i < m;
-    if (live) {
-      const q128 *row = A + i * lda;
-      const int64_t pairs = n / 2;
-      for (int64_t j = 0; j < pairs; ++j) chain_fma(ch, ld(row + 2 * j + p), ld(x + 2 * j + p));
-    }
-    const q128 mine = cacc_get(ch);
-    // exchange with the partner lane (same row); both lanes of a pair are live or dead together
-    const uint64_t olo = (uint64_t)__shfl_xor((unsigned long long)mine.lo, 1);
-    const uint64_t ohi = (uint64_t)__shfl_xor((unsigned long long)mine.hi, 1);
-    if (!live || p != 0) return;
-    q128 sum = add_packed(mine, q_make(olo, ohi));
-    if (n & 1) sum = fma_packed(ld(A + i * lda + n - 1), ld(x + n - 1), sum);
-    q128 *yi = y + i * incy;
-    st(yi, fma_packed(alpha, sum, mul_packed(beta, ld(yi))));
-  } else {
-    const int64_t i = tid;
-    if (i >= m) return;
-    const q128 *row = A + i * lda;
-    for (int64_t j = 0; j < n; ++j) chain_fma(ch, ld(row + j), ld(x + j * incx));
-    q128 *yi = y + i * incy;
-    st(yi, fma_packed(alpha, cacc_get(ch), mul_packed(beta, ld(yi))));
-  }
-}
-
-// y_i = fma(alpha, sum, mul(beta, y_i)) with sum = c0 + c1 (two chains), the odd tail's fma applied;
-// the four operations as one loop, so the step's code is there once
-__device__ __forceinline__ q128 gemv_row_end(q128 c0, q128 c1, int pair, int odd, q128 ta, q128 tx, q128 alpha,
-                                             q128 beta, q128 y) {
-  q128 by = q_zero(1), sum = c0;
-#pragma unroll 1
-  for (int op = 0; op < 4; ++op) {
-    if ((op == 1 && !pair) || (op == 2 && !odd)) continue;
-    const q128 a = op == 0 ? beta : op == 1 ? c1 : op == 2 ? ta : alpha;
-    const q128 b = op == 0 ? y : op == 1 ? q_one() : op == 2 ? tx : sum;
-    cacc acc;
-    cacc_set(acc, (op == 0 || op == 3) ? by : sum);
-    chain_fma(acc, a, b);
-    const q128 r = cacc_get(acc);
-    if (op == 0 || op == 3) by = r;
-    else sum = r;
-  }
-  return by;
+  lane_chain(ch, live, row + p, 1 + pair, n >> pair, 1 + pair, p, [=](int64_t j) { return ld(x + j * incx); }, lds);
+  const q128 mine = cacc_get(ch);
+  const uint64_t olo = (uint64_t)__shfl_xor((unsigned long long)mine.lo, 1);
+  const uint64_t ohi = (uint64_t)__shfl_xor((unsigned long long)mine.hi, 1);
+  if (!live || p != 0) return;
+  const int odd = pair && (n & 1);
+  q128 *yi = y + i * incy;
+  st(yi, gemv_row_end(mine, q_make(olo, ohi), pair, odd, odd ? ld(row + n - 1) : q_zero(0),
+                      odd ? ld(x + n - 1) : q_zero(0), alpha, beta, ld(yi)));
 }
 // Few rows: one wave per chain, 64 columns at a time (chain_scan.hpp); rows of a workgroup share x.
 // A pair's chains are neighbouring waves, the first of which ends the row.
@@ -183,22 +150,23 @@ __global__ void k_scale_vec(int64_t n, q128 alpha, const q128 *__restrict__ x, i
                             q128 *__restrict__ ax) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride)
-    st(ax + j, mul_packed(alpha, ld(x + j * incx)));
+    st(ax + j, chain_mul(alpha, ld(x + j * incx)));
 }
 // ColMajor: y_i = mul(beta, y_i) (level2.hpp:63-66), then y_i = fma(A_ij, ax_j, y_i) for
 // j = 0..n-1 (level2.hpp:69-80); lane i owns row i, so loads of A columns coalesce.
-__global__ void k_gemv_col_ref(int64_t m, int64_t n, const q128 *__restrict__ A, int64_t lda,
-                               const q128 *__restrict__ ax, q128 beta, q128 *__restrict__ y, int64_t incy) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
+__global__ void __launch_bounds__(64) k_gemv_col_ref(int64_t m, int64_t n, const q128 *__restrict__ A, int64_t lda,
+                                                     const q128 *__restrict__ ax, q128 beta, q128 *__restrict__ y,
+                                                     int64_t incy) {
+  __shared__ __attribute__((aligned(16))) chain_lds lds;
+  for (int64_t i0 = (int64_t)blockIdx.x * 64; i0 < m; i0 += (int64_t)gridDim.x * 64) {
+    const int64_t i = i0 + threadIdx.x;
     q128 *yi = y + i * incy;
     cacc ch;
-    cacc_set(ch, mul_packed(beta, ld(yi)));
-    for (int64_t j = 0; j < n; ++j) chain_fma(ch, ld(A + j * lda + i), ld(ax + j));
-    st(yi, cacc_get(ch));
+    cacc_set(ch, i < m ? chain_mul(beta, ld(yi)) : q_zero(0));
+    lane_chain(ch, i < m, A + i, lda, n, 1, 0, [=](int64_t j) { return ld(ax + j); }, lds);
+    if (i < m) st(yi, cacc_get(ch));
   }
 }
-
 // Few rows: one wave per row; the eight rows of a workgroup share the 128-byte lines of A's columns.
 __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n, const q128 *__restrict__ A,
                                                            int64_t lda, const q128 *__restrict__ ax, q128 beta,
@@ -206,7 +174,7 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
   const int64_t i = (int64_t)blockIdx.x * 8 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (i >= m) return;
   q128 *yi = y + i * incy;
-  const q128 r = wave_chain(mul_packed(beta, ld(yi)), sc_strided{A + i, lda}, sc_strided{ax, 1}, n);
+  const q128 r = wave_chain(chain_mul(beta, ld(yi)), sc_strided{A + i, lda}, sc_strided{ax, 1}, n);
   if ((threadIdx.x & 63) == 0) st(yi, r);
 }
 
@@ -227,7 +195,8 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
 // log-uniform: 222 ms = 619 quad GFLOP/s (577 ms with a 401-instruction step); 2048^3 uniform 21.9 ms.
 // part == null: the workgroup takes all blocks of k.  Else it takes block kb0 + blockIdx.z and writes its t to
 // part[(blockIdx.z n + j) m + i], for k_gemm_ref_fold: the blocks' chains do not depend on each other,
-// so a C of few tiles still fills the chip: 500 x 333 x 700 340 us (440 without), 64 x 64 x 2000 70 us (740).
+// so a C of few tiles still fills the chip: 500 x 333 x 700 427 us against 561, 64 x 64 x 2000 68 us
+// against 874 (both with the step of 105 instructions; now 340 us and 72 us).
 constexpr int GR_KT = 32;
 __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_t kc,
                                                   q128 alpha, const q128 *__restrict__ A, int64_t lda,
@@ -377,13 +346,13 @@ hipError_t launch_dot_ref(const q128 *x, int64_t incx, const q128 *y, int64_t in
   return hipGetLastError();
 }
 
-// Whether a gemv's chains go to a wave each (chain_scan.hpp) or to a lane each.  A lane's step is a
-// latency of about 0.5 us until the lanes fill the chip; a wave's block of 64 steps costs what about
-// 9 instructions a step cost, and the rest of a block as well.  Measured, uniform entries, us (wave
-// each, lane each): row-major 1500^2 69, 360; 8192^2 809, 2300; 16384 x 2048 (32768 chains) 460, 634;
-// 32768 x 1024 506, 360; column-major 2049 x 777 46, 479; 32768 x 1024 487, 801; 65536 x 1000 906, 799.
+// Whether a gemv's chains go to a wave each (chain_scan.hpp) or to a lane each (lane_chain).  A lane's
+// step is a latency of about 0.5 us until the lanes fill the chip; a wave's block of 64 steps costs a
+// fixed amount and about 9 instructions a step.  Measured, uniform entries, us (wave each, lane each):
+// row-major 1500^2 69, 359; 8192^2 797, 1932; 16384 x 2048 (32768 chains) 457, 519; 65536 x 1000 980, 316;
+// column-major 2049 x 777 63, 366; 8192^2 1061, 3738; 32768 x 1024 476, 510; 4608 x 16 20, 16.
 static bool few_chains(int64_t chains, int64_t len) {
-  return chains <= 32768 && chains * ((len + 63) / 64 * 64 + 64) <= 36864 * len;
+  return chains <= 32768 && chains * ((len + 63) / 64 * 64 + 128) <= 36864 * len;
 }
 
 hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const q128 *A, int64_t lda,

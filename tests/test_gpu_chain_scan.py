@@ -76,9 +76,9 @@ def test_gemv(O, Q, cuda, kind, layout, m, n, incx):
         assert np.array_equal(plain(from_dev(dy)), plain(want))
 
 
-# chains (64 ceil(len / 64) + 64) <= 36864 len: 4608 chains of 16 are the last that get a wave each
-@pytest.mark.parametrize("layout,m,n,incx", [(1, 4608, 16, 1), (1, 4609, 16, 1), (0, 4608, 16, 2), (0, 4609, 16, 2),
-                                             (0, 2304, 32, 1), (0, 2305, 33, 1)])
+# chains (64 ceil(len / 64) + 128) <= 36864 len: 3072 chains of 16 are the last that get a wave each
+@pytest.mark.parametrize("layout,m,n,incx", [(1, 3072, 16, 1), (1, 3073, 16, 1), (0, 3072, 16, 2), (0, 3073, 16, 2),
+                                             (0, 1536, 32, 1), (0, 1537, 33, 1), (0, 5000, 45, 1), (1, 3075, 33, 2)])
 def test_gemv_either_side_of_the_rule(O, Q, cuda, layout, m, n, incx):
     print(f"gemv layout={layout} {m}x{n} incx={incx}", flush=True)
     lda = n if layout == 0 else m
@@ -89,3 +89,9 @@ def test_gemv_either_side_of_the_rule(O, Q, cuda, layout, m, n, incx):
     Q.dev_gemv(Q.MODE_REFERENCE, layout, m, n, 1.5, dA.data_ptr(), lda, dx.data_ptr(), incx, -0.5, dy.data_ptr(), 1)
     cuda.cuda.synchronize()
     assert np.array_equal(from_dev(dy), want)
+
+
+@pytest.mark.parametrize("kind", ("cancel", "sparse", "subnormal", "nan"))
+@pytest.mark.parametrize("layout,m,n,incx", [(0, 1600, 31, 1), (0, 3300, 17, 2), (1, 3200, 15, 1)])
+def test_gemv_lane_per_chain(O, Q, cuda, kind, layout, m, n, incx):
+    test_gemv(O, Q, cuda, kind, layout, m, n, incx)
