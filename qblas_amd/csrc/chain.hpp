@@ -369,6 +369,54 @@ __device__ __forceinline__ void lane_chain(cacc &ch, bool live, const q128 *__re
     }
   }
 }
+
+// The chains t = sum over l in [kk, ke) of A(i, l) B(l, j) of a TM x TN tile of C at (i0, j0), one per thread of 256,
+// rows fastest.  Per step of KT values of l the workgroup loads the tile's TM x KT elements of A and
+// KT x TN of B once (coalesced along the contiguous dimension), unpacks them into LDS, and every thread
+// runs its chain over the step from LDS, in the order l = kk, kk + 1, ...  A special operand is taken
+// from memory again.  Every thread of the workgroup calls; threads outside m x n return zero.
+template <int TM, int TN, int KT>
+__device__ __forceinline__ q128 tile_chain(int colmajor, int64_t m, int64_t n, const q128 *__restrict__ A, int64_t lda,
+                                           const q128 *__restrict__ B, int64_t ldb, int64_t i0, int64_t j0, int64_t kk,
+                                           int64_t ke, cop *sA, cop *sB) {
+  static_assert(TM * TN == 256, "256 threads");
+  const int64_t as_i = colmajor ? 1 : lda, as_l = colmajor ? lda : 1;
+  const int64_t bs_l = colmajor ? 1 : ldb, bs_j = colmajor ? ldb : 1;
+  const int ti = (int)threadIdx.x % TM, tj = (int)threadIdx.x / TM;
+  const bool live = i0 + ti < m && j0 + tj < n;
+  const q128 *ap = A + (i0 + ti) * as_i;
+  const q128 *bp = B + (j0 + tj) * bs_j;
+  auto load = [](const q128 *p) {
+    const uint4 v = *reinterpret_cast<const uint4 *>(p);
+    return q_make(((uint64_t)v.y << 32) | v.x, ((uint64_t)v.w << 32) | v.z);
+  };
+  cacc ch;
+  cacc_init(ch);
+  for (int64_t l0 = kk; l0 < ke; l0 += KT) {
+    const int lt = (int)((ke - l0 < KT) ? ke - l0 : KT);
+    __syncthreads();  // the previous step's operands are no longer read
+#pragma unroll
+    for (int e0 = 0; e0 < TM * KT; e0 += 256) {
+      const int e = e0 + (int)threadIdx.x;  // rows contiguous: r fastest; l contiguous: q fastest
+      const int r = colmajor ? e % TM : e / KT, q = colmajor ? e / TM : e % KT;
+      if (e < TM * KT && q < lt && i0 + r < m) sA[q * TM + r] = cop_unpack(load(A + (i0 + r) * as_i + (l0 + q) * as_l));
+    }
+#pragma unroll
+    for (int e0 = 0; e0 < TN * KT; e0 += 256) {
+      const int e = e0 + (int)threadIdx.x;
+      const int c = colmajor ? e / KT : e % TN, q = colmajor ? e % KT : e / TN;
+      if (e < TN * KT && q < lt && j0 + c < n) sB[q * TN + c] = cop_unpack(load(B + (l0 + q) * bs_l + (j0 + c) * bs_j));
+    }
+    __syncthreads();
+    if (live) {
+      if (l0 == kk) cacc_first(ch, sA[ti], sB[tj]);
+      for (int q = 0; q < lt; ++q)
+        if (!cacc_step(ch, sA[q * TM + ti], sB[q * TN + tj]))
+          chain_slow(ch, load(ap + (l0 + q) * as_l), load(bp + (l0 + q) * bs_l));
+    }
+  }
+  return cacc_get(ch);
+}
 #endif  // __HIPCC__
 
 }  // namespace qb

@@ -186,11 +186,7 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
 // C = fma(alpha, t, mul(first ? beta : 1, C)) (level3.hpp:297-300 with the micro-kernel's
 // epilogue :102-109; gemm_simple :200-210 is the single-block case); the product with 1 changes
 // nothing, so C = fma(alpha, t, C) over the blocks is one more chain, from beta * C.  Layout-aware indexing for
-// both layouts.  A workgroup computes a 16 x 16 tile of C: per step of GR_KT values of l, its 256
-// threads load the tile's 16 x GR_KT elements of A and GR_KT x 16 of B once (coalesced along the
-// contiguous dimension), unpack them into LDS, and every lane runs its chain over the step from
-// LDS, in the same order l = kk, kk + 1, ... as the reference.  An operand that is zero,
-// subnormal, Inf or NaN is marked in LDS and taken from memory again for the packed slow path.
+// both layouts.  A workgroup computes a 16 x 16 tile of C (tile_chain).
 // Bound by VALU issue: 85 to 105 instructions per wave and multiply-add (chain.hpp).  4096^3
 // log-uniform: 222 ms = 619 quad GFLOP/s (577 ms with a 401-instruction step); 2048^3 uniform 21.9 ms.
 // part == null: the workgroup takes all blocks of k.  Else it takes block kb0 + blockIdx.z and writes its t to
@@ -203,49 +199,22 @@ __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64
                                                   const q128 *__restrict__ B, int64_t ldb, q128 beta,
                                                   q128 *__restrict__ C, int64_t ldc, int64_t kb0,
                                                   q128 *__restrict__ part) {
-  __shared__ __attribute__((aligned(16))) cop sA[GR_KT][16];
-  __shared__ __attribute__((aligned(16))) cop sB[GR_KT][16];
+  __shared__ __attribute__((aligned(16))) cop sA[GR_KT * 16];
+  __shared__ __attribute__((aligned(16))) cop sB[GR_KT * 16];
   const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
   const int64_t i0 = (int64_t)blockIdx.y * 16, j0 = (int64_t)blockIdx.x * 16;
   const int64_t i = i0 + ti, j = j0 + tj;
   const bool live = i < m && j < n;  // every thread takes part in the loads and barriers
-  const int64_t as_i = colmajor ? 1 : lda, as_l = colmajor ? lda : 1;
-  const int64_t bs_l = colmajor ? 1 : ldb, bs_j = colmajor ? ldb : 1;
   q128 *ci = C + (colmajor ? j * ldc + i : i * ldc + j);
-  const q128 *ap = A + i * as_i;
-  const q128 *bp = B + j * bs_j;
   const int64_t k0 = part ? (kb0 + blockIdx.z) * kc : 0, k1 = part ? (k0 + kc < k ? k0 + kc : k) : k;
   cacc c;
-  if (!part) cacc_set(c, live ? mul_packed(beta, ld(ci)) : q_zero(0));
+  if (!part) cacc_set(c, live ? chain_mul(beta, ld(ci)) : q_zero(0));
   for (int64_t kk = k0; kk < k1; kk += kc) {
     const int64_t ke = (kk + kc < k1) ? kk + kc : k1;
-    cacc ch;
-    cacc_init(ch);
-    for (int64_t l0 = kk; l0 < ke; l0 += GR_KT) {
-      const int lt = (int)((ke - l0 < GR_KT) ? ke - l0 : GR_KT);
-      __syncthreads();  // the previous step's operands are no longer read
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int e = (int)threadIdx.x + 256 * h;  // 512 = 16 x GR_KT elements of each operand
-        // A(i0 + r, l0 + q): l contiguous (RowMajor) -> q fastest; rows contiguous -> r fastest
-        const int ra = colmajor ? (e & 15) : (e >> 5), qa = colmajor ? (e >> 4) : (e & 31);
-        if (qa < lt && i0 + ra < m) sA[qa][ra] = cop_unpack(ld(A + (i0 + ra) * as_i + (l0 + qa) * as_l));
-        // B(l0 + q, j0 + c): columns contiguous (RowMajor) -> c fastest; l contiguous -> q fastest
-        const int cb = colmajor ? (e >> 5) : (e & 15), qb = colmajor ? (e & 31) : (e >> 4);
-        if (qb < lt && j0 + cb < n) sB[qb][cb] = cop_unpack(ld(B + (l0 + qb) * bs_l + (j0 + cb) * bs_j));
-      }
-      __syncthreads();
-      if (live) {
-        if (l0 == kk) cacc_first(ch, sA[0][ti], sB[0][tj]);
-        for (int q = 0; q < lt; ++q) {
-          if (!cacc_step(ch, sA[q][ti], sB[q][tj]))
-            chain_slow(ch, ld(ap + (l0 + q) * as_l), ld(bp + (l0 + q) * bs_l));
-        }
-      }
-    }
+    const q128 t = tile_chain<16, 16, GR_KT>(colmajor, m, n, A, lda, B, ldb, i0, j0, kk, ke, sA, sB);
     if (live) {
-      if (!part) chain_fma(c, alpha, cacc_get(ch));
-      else st(part + ((int64_t)blockIdx.z * n + j) * m + i, cacc_get(ch));
+      if (!part) chain_fma(c, alpha, t);
+      else st(part + ((int64_t)blockIdx.z * n + j) * m + i, t);
     }
   }
   if (!part && live) st(ci, cacc_get(c));
