@@ -30,6 +30,8 @@
 //    queued and recomputed by the EXACT form's exact accumulation (correctly rounded); an entry
 //    whose products lie too far apart for the windows takes the full-range path (wide.hpp).
 // So the result of every entry has relative error <= 2^-105.9 or is correctly rounded.
+#include <algorithm>
+
 #include "wide.hpp"
 #include "kernels.h"
 
@@ -109,7 +111,7 @@ __global__ void k_oz_init(int32_t *eA, uint32_t *fA, int64_t Mp, int32_t *eB, ui
     eB[g] = OZ_EZERO;
     fB[g] = 0;
   }
-  if (g < OZ_HDR / 4) hdr[g] = 0u;
+  if (hdr && g < OZ_HDR / 4) hdr[g] = 0u;
 }
 
 __device__ __forceinline__ int oz_ilogb(q128 x, uint32_t &fl) {
@@ -165,6 +167,77 @@ __global__ void __launch_bounds__(256) k_oz_scale(const q128 *__restrict__ X, in
     for (; c < c1; ++c) e = max(e, oz_ilogb(ldq_c(X + r * sr + c * sc), fl));
     if (e != OZ_EZERO) atomicMax(E + r, e);
     if (fl) atomicOr(F + r, fl);
+  }
+}
+
+// Both operands of a small product in one launch: blockIdx.y 0 is A, 1 is B, and a row's whole range of
+// c belongs to one workgroup, so E and F are written, not initialised and then joined by atomics.  A
+// launch costs about as much as these operands' loads: 150 x 200 x 333, 7 us instead of 22 us of three
+// kernels and their gaps.  contig: 4 rows, a wave each; else 16 rows (lane % 16), the other 16 lanes
+// along c.
+struct oz_operand {
+  const q128 *X;
+  int64_t R, C, sr, sc;
+  int32_t *E;
+  uint32_t *F;
+};
+constexpr int64_t OZ_SMALL_R = 4096, OZ_SMALL_C = 1024;
+__global__ void __launch_bounds__(256) k_oz_scale_small(oz_operand a, oz_operand b) {
+  __shared__ int s_e[4][16];
+  __shared__ uint32_t s_f[4][16];
+  const oz_operand o = blockIdx.y ? b : a;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  int e = OZ_EZERO;
+  uint32_t fl = 0;
+  if (o.sc == 1) {
+    const int64_t r = (int64_t)blockIdx.x * 4 + wv;
+    if (r >= o.R) return;  // whole waves; no barrier in this branch
+    const q128 *row = o.X + r * o.sr;
+    for (int64_t c = lane; c < o.C; c += 256) {
+      q128 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = c + 64 * u < o.C ? ldq_c(row + c + 64 * u) : q_zero(0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e = max(e, oz_ilogb(v[u], fl));
+    }
+    e = wave_max(e);
+    fl = wave_or(fl);
+    if (lane == 0) {
+      o.E[r] = e;
+      o.F[r] = fl;
+    }
+    return;
+  }
+  const int64_t r0 = (int64_t)blockIdx.x * 16, r = r0 + (lane & 15);
+  if (r0 >= o.R) return;  // the whole workgroup
+  if (r < o.R) {
+    const q128 *row = o.X + r * o.sr;
+    for (int64_t c = wv * 4 + (lane >> 4); c < o.C; c += 64) {
+      q128 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = c + 16 * u < o.C ? ldq_c(row + (c + 16 * u) * o.sc) : q_zero(0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e = max(e, oz_ilogb(v[u], fl));
+    }
+  }
+#pragma unroll
+  for (int m = 16; m <= 32; m <<= 1) {
+    e = max(e, __shfl_xor(e, m));
+    fl |= __shfl_xor(fl, m);
+  }
+  if (lane < 16) {
+    s_e[wv][lane] = e;
+    s_f[wv][lane] = fl;
+  }
+  __syncthreads();
+  if (threadIdx.x < 16 && r < o.R) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      e = max(e, s_e[w][lane]);
+      fl |= s_f[w][lane];
+    }
+    o.E[r] = e;
+    o.F[r] = fl;
   }
 }
 
@@ -863,6 +936,23 @@ static void oz_scale(const q128 *X, int64_t R, int64_t Cn, int64_t sr, int64_t s
   k_oz_scale<<<grid, 256, 0, st>>>(X, R, Cn, sr, sc, contig, cchunk, E, F);
 }
 
+// Exponents and flags of A's m rows and B's n columns; hdr, if not null, is cleared
+static void oz_scale_both(int64_t m, int64_t n, int64_t k, const q128 *A, int64_t asr, int64_t asc, const q128 *B,
+                          int64_t bsr, int64_t bsc, int32_t *eA, uint32_t *fA, int32_t *eB, uint32_t *fB,
+                          uint32_t *hdr, hipStream_t st) {
+  if (m <= OZ_SMALL_R && n <= OZ_SMALL_R && k <= OZ_SMALL_C) {
+    if (hdr) k_oz_init<<<1, 256, 0, st>>>(eA, fA, 0, eB, fB, 0, hdr);
+    const oz_operand a{A, m, k, asr, asc, eA, fA}, b{B, n, k, bsc, bsr, eB, fB};  // B columns: r = j, c = l
+    const int64_t ga = (m + (asc == 1 ? 3 : 15)) / (asc == 1 ? 4 : 16), gb = (n + (bsr == 1 ? 3 : 15)) / (bsr == 1 ? 4 : 16);
+    k_oz_scale_small<<<dim3((unsigned)(ga > gb ? ga : gb), 2), 256, 0, st>>>(a, b);
+    return;
+  }
+  const int64_t mx = std::max<int64_t>(std::max(m, n), OZ_HDR / 4);
+  k_oz_init<<<(unsigned)((mx + 255) / 256), 256, 0, st>>>(eA, fA, m, eB, fB, n, hdr);
+  oz_scale(A, m, k, asr, asc, eA, fA, st);
+  oz_scale(B, n, k, bsc, bsr, eB, fB, st);
+}
+
 // Exact recomputation of the queued entries (header word 1 counts them, list holds (i, j)).  When
 // B's columns are strided, a transposed copy of B (at Bt) is made first if the queue is long; the
 // copy and the repair read the queue length on the device, so nothing is synchronized.
@@ -886,11 +976,11 @@ static hipError_t oz_repair_queue(int64_t m, int64_t n, int64_t k, const q128 *A
 
 void ozaki_probe_scales(const void *wsv, int64_t m, int64_t n, const int32_t **eA, const uint32_t **fA,
                         const int32_t **eB, const uint32_t **fB);
-// Header and scaling exponents of a call: the probe's when it ran on the same operands (probe_ws),
-// else computed here into the call's own arrays (*eA.. point there on entry).
-static void oz_prepare(int64_t Mp, int64_t Np, int64_t m, int64_t n, int64_t k, const q128 *A, int64_t asr,
-                       int64_t asc, const q128 *B, int64_t bsr, int64_t bsc, const void *probe_ws, int32_t **eA,
-                       uint32_t **fA, int32_t **eB, uint32_t **fB, uint32_t *hdr, hipStream_t st) {
+// Scaling exponents of a call, the probe's when it ran on the same operands (probe_ws), else computed
+// here into the call's own arrays (*eA.. point there on entry); hdr, if not null, is cleared.
+static void oz_prepare(int64_t m, int64_t n, int64_t k, const q128 *A, int64_t asr, int64_t asc, const q128 *B,
+                       int64_t bsr, int64_t bsc, const void *probe_ws, int32_t **eA, uint32_t **fA, int32_t **eB,
+                       uint32_t **fB, uint32_t *hdr, hipStream_t st) {
   if (probe_ws) {
     const int32_t *pa, *pb;
     const uint32_t *qa, *qb;
@@ -899,13 +989,10 @@ static void oz_prepare(int64_t Mp, int64_t Np, int64_t m, int64_t n, int64_t k, 
     *fA = const_cast<uint32_t *>(qa);
     *eB = const_cast<int32_t *>(pb);
     *fB = const_cast<uint32_t *>(qb);
-    k_oz_init<<<1, 256, 0, st>>>(*eA, *fA, 0, *eB, *fB, 0, hdr);  // header only
+    if (hdr) k_oz_init<<<1, 256, 0, st>>>(*eA, *fA, 0, *eB, *fB, 0, hdr);  // header only
     return;
   }
-  const int64_t ninit = (Mp > Np ? Mp : Np) > OZ_HDR / 4 ? (Mp > Np ? Mp : Np) : OZ_HDR / 4;
-  k_oz_init<<<(unsigned)((ninit + 255) / 256), 256, 0, st>>>(*eA, *fA, Mp, *eB, *fB, Np, hdr);
-  oz_scale(A, m, k, asr, asc, *eA, *fA, st);
-  oz_scale(B, n, k, bsc, bsr, *eB, *fB, st);  // B columns: r = j, c = l
+  oz_scale_both(m, n, k, A, asr, asc, B, bsr, bsc, *eA, *fA, *eB, *fB, hdr, st);
 }
 
 hipError_t launch_gemm_ozaki(int colmajor, int64_t m, int64_t n, int64_t k, int S, q128 alpha, const q128 *A,
@@ -923,7 +1010,7 @@ hipError_t launch_gemm_ozaki(int colmajor, int64_t m, int64_t n, int64_t k, int 
   uint32_t *fA = (uint32_t *)(ws + L.fA), *fB = (uint32_t *)(ws + L.fB);
   uint32_t *hdr = (uint32_t *)ws;
   if (ev) (void)hipEventRecord(ev[0], st);
-  oz_prepare(L.Mp, L.Np, m, n, k, A, asr, asc, B, bsr, bsc, probe_ws, &eA, &fA, &eB, &fB, hdr, st);
+  oz_prepare(m, n, k, A, asr, asc, B, bsr, bsc, probe_ws, &eA, &fA, &eB, &fB, hdr, st);
   switch (S) {
 #define QB_OZ_CASE(s) \
   case s: oz_launch_slices<s>(L, A, m, k, asr, asc, B, n, bsr, bsc, eA, eB, ws, st); break;
@@ -971,7 +1058,6 @@ hipError_t launch_ozaki_probe(int colmajor, int64_t m, int64_t n, int64_t k, con
                               const q128 *B, int64_t ldb, int samples, void *wsv, hipStream_t st, int *out) {
   char *ws = (char *)wsv;
   auto al = [](size_t v) { return (v + 255) / 256 * 256; };
-  uint32_t *hdr = (uint32_t *)ws;
   int32_t *eA = (int32_t *)(ws + OZ_HDR);
   uint32_t *fA = (uint32_t *)(ws + al(OZ_HDR + (size_t)m * 4));
   int32_t *eB = (int32_t *)(ws + al(OZ_HDR + (size_t)m * 4) + al((size_t)m * 4));
@@ -980,9 +1066,7 @@ hipError_t launch_ozaki_probe(int colmajor, int64_t m, int64_t n, int64_t k, con
   const int64_t bsr = colmajor ? 1 : ldb, bsc = colmajor ? ldb : 1;
   const int64_t ninit = (m > n ? m : n) > OZ_HDR / 4 ? (m > n ? m : n) : OZ_HDR / 4;
   if (!grid_fits((ninit + 3) / 4, 256)) return hipErrorInvalidValue;
-  k_oz_init<<<(unsigned)((ninit + 255) / 256), 256, 0, st>>>(eA, fA, m, eB, fB, n, hdr);
-  oz_scale(A, m, k, asr, asc, eA, fA, st);
-  oz_scale(B, n, k, bsc, bsr, eB, fB, st);
+  oz_scale_both(m, n, k, A, asr, asc, B, bsr, bsc, eA, fA, eB, fB, nullptr, st);
   if (samples > OZ_PROBE_MAX) samples = OZ_PROBE_MAX;
   k_oz_probe<<<(unsigned)(samples < 256 ? samples : 256), OZR_BS, 0, st>>>(
       m, n, k, A, asr, asc, B, bsr, bsc, eA, eB, samples, out ? out : (int *)(ws + ozaki_probe_out_offset(m, n)));
@@ -1685,10 +1769,20 @@ __device__ __forceinline__ i32x4v crt_pack16(const i32x16v &d, int p, uint32_t m
 // dword of one modulus.
 // Groups 0..15 use slots 0..31 (k < 16), groups 16..31 slots 32..63.
 constexpr int CRT_RS = 17;  // LDS row stride (elements) of the residue kernel
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) k_crt_residues(const q128 *__restrict__ X, int64_t R, int64_t K, int64_t sr,
-                                                      int64_t sc, const int32_t *__restrict__ E, int t,
-                                                      const crt_tab *__restrict__ T, int64_t Rb, int64_t Kb,
-                                                      int64_t plane, int8_t *__restrict__ out) {
+// Both operands in one launch: workgroups 0 .. ga - 1 are A's, the rest B's.  split: a wave takes one half
+// of a fragment position, not both: for few positions, where a wave's latency is the launch's (150 x 200 x
+// 333: 14 us with the header cleared here, 42 us as two launches of whole positions and a clear).  The
+// first workgroup clears the call's header.
+struct crt_operand {
+  const q128 *X;
+  int64_t R, sr, sc;
+  const int32_t *E;
+  int64_t Rb, plane;
+  int8_t *out;
+};
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
+k_crt_residues(crt_operand oa, crt_operand ob, unsigned ga, int64_t K, int64_t Kb, int t, int split,
+               const crt_tab *__restrict__ T, uint32_t *__restrict__ hdr) {
   __shared__ __attribute__((aligned(16))) uint32_t s_lo[4][32 * CRT_RS][4];
   __shared__ uint32_t s_hi[4][32 * CRT_RS];
   __shared__ i32x4v s_cst[32];  // moduli 32..63: p, mdiv, half - off, 16 off
@@ -1704,7 +1798,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
   __syncthreads();  // every wave of the block is still here
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63, n = lane & 31,
             h = lane >> 5;
-  const int64_t pos = (int64_t)blockIdx.x * 4 + wave;
+  if (blockIdx.x == 0 && threadIdx.x < OZ_HDR / 4) hdr[threadIdx.x] = 0u;
+  const bool second = blockIdx.x >= ga;
+  const q128 *__restrict__ X = second ? ob.X : oa.X;
+  const int32_t *__restrict__ E = second ? ob.E : oa.E;
+  int8_t *__restrict__ out = second ? ob.out : oa.out;
+  const int64_t R = second ? ob.R : oa.R, sr = second ? ob.sr : oa.sr, sc = second ? ob.sc : oa.sc,
+                Rb = second ? ob.Rb : oa.Rb, plane = second ? ob.plane : oa.plane;
+  const int64_t unit = (int64_t)(blockIdx.x - (second ? ga : 0u)) * 4 + wave;
+  const int64_t pos = unit >> split;
+  const int half0 = split ? (int)(unit & 1) : 0, half1 = split ? half0 + 1 : 2;
   if (pos >= Rb * Kb) return;  // whole waves; only wave-local LDS below
   const int64_t rb = pos / Kb, kb = pos - rb * Kb;
   const bool kcontig = (sc == 1);
@@ -1738,9 +1841,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
       ev[i] = in ? E[row] : OZ_EZERO;
     }
   };
-  load_half(0);
+  load_half(half0);
 #pragma nounroll
-  for (int half = 0; half < 2; ++half) {
+  for (int half = half0; half < half1; ++half) {
     {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -1757,7 +1860,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
         s_hi[wave][e] = W[4] ^ 0x80808080u;
       }
     }
-    if (half == 0) load_half(1);
+    if (half + 1 < half1) load_half(half + 1);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -2093,9 +2196,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                                                     const uint32_t *__restrict__ fB, q128 alpha, q128 beta,
                                                     q128 *__restrict__ C, int64_t csr, int64_t csc,
                                                     uint32_t *__restrict__ hdr, uint32_t *__restrict__ list,
-                                                    uint32_t *__restrict__ xrec) {
+                                                    uint32_t *__restrict__ xrec, int quarters) {
   constexpr int RW = (XW + 3) & ~3;
-  const int64_t blk = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // a wave takes a whole block (quarters = 4), or one row quarter of it (1): few blocks, where a wave's
+  // latency is the launch's (150 x 200: 19 us whole, 8 us by quarters)
+  const int64_t unit = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t blk = quarters == 4 ? unit : unit >> 2;
+  const int rq0 = quarters == 4 ? 0 : (int)(unit & 3), rq1 = rq0 + quarters;
   if (blk >= Mb * Nb) return;  // whole waves
   const int lane = threadIdx.x & 63, n = lane & 31, kh = lane >> 5;
   const int64_t bm = blk / Nb, bn = blk - bm * Nb;
@@ -2150,12 +2257,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       ch[it] = in ? reinterpret_cast<const uint32_t *>(C + row * csr + col * csc)[3] : 0u;
     }
   };
-  load_entries(0, eAr, fAr, chi);
-  load_rows(0);
+  load_entries(rq0, eAr, fAr, chi);
+  load_rows(rq0);
   // Each quarter waits once, at its top, for everything loaded so far; its swaps free w, and the
   // next quarter's loads are issued before its reconstruction, so they land meanwhile
 #pragma nounroll
-  for (int rq = 0; rq < 4; ++rq) {
+  for (int rq = rq0; rq < rq1; ++rq) {
     uint32_t Q[2][2][16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -2168,7 +2275,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       Q[0][1][j] = s2[0];
       Q[1][1][j] = s2[1];
     }
-    if (rq < 3) {
+    if (rq + 1 < rq1) {
       load_entries(rq + 1, eAn, fAn, chn);
       load_rows(rq + 1);
     }
@@ -2495,14 +2602,16 @@ hipError_t launch_gemm_crt(int colmajor, int64_t m, int64_t n, int64_t k, int t,
   crt_tab *tab = tab_in ? (crt_tab *)tab_in : (crt_tab *)(ws + L.tab);
   int8_t *RA = (int8_t *)(ws + L.rA), *RB = (int8_t *)(ws + L.rB), *RC = (int8_t *)(ws + L.rC);
   const int64_t wgs = (int64_t)nq * (L.Mb / CRT_TA) * (L.Nb / CRT_TB);
-  if (!oz_grids_fit(L.Mp, L.Np, L.Kb) || !grid_fits((L.Mb * L.Kb + 3) / 4, 256) ||
-      !grid_fits((L.Nb * L.Kb + 3) / 4, 256) || !grid_fits(wgs, 512) || !grid_fits((L.Mb * L.Nb + 3) / 4, 256))
+  if (!oz_grids_fit(L.Mp, L.Np, L.Kb) || !grid_fits(((L.Mb + L.Nb) * L.Kb + 3) / 4 + 2, 256) || !grid_fits(wgs, 512) || !grid_fits((L.Mb * L.Nb + 3) / 4, 256))
     return hipErrorInvalidValue;
   if (ev) (void)hipEventRecord(ev[0], st);
-  oz_prepare(L.Mp, L.Np, m, n, k, A, asr, asc, B, bsr, bsc, probe_ws, &eA, &fA, &eB, &fB, hdr, st);
+  oz_prepare(m, n, k, A, asr, asc, B, bsr, bsc, probe_ws, &eA, &fA, &eB, &fB, nullptr, st);
   if (!tab_in) k_crt_tables<<<1, 64, 0, st>>>(nq, tab);
-  k_crt_residues<<<(unsigned)((L.Mb * L.Kb + 3) / 4), 256, 0, st>>>(A, m, k, asr, asc, eA, t, tab, L.Mb, L.Kb, L.pA, RA);
-  k_crt_residues<<<(unsigned)((L.Nb * L.Kb + 3) / 4), 256, 0, st>>>(B, n, k, bsc, bsr, eB, t, tab, L.Nb, L.Kb, L.pB, RB);
+  // 3072 waves fill the chip (3 per SIMD)
+  const int split = (L.Mb + L.Nb) * L.Kb <= 1536;
+  const unsigned ga = (unsigned)(((L.Mb * L.Kb << split) + 3) / 4), gb = (unsigned)(((L.Nb * L.Kb << split) + 3) / 4);
+  k_crt_residues<<<ga + gb, 256, 0, st>>>(crt_operand{A, m, asr, asc, eA, L.Mb, L.pA, RA},
+                                          crt_operand{B, n, bsc, bsr, eB, L.Nb, L.pB, RB}, ga, k, L.Kb, t, split, tab, hdr);
   if (ev) (void)hipEventRecord(ev[1], st);
   k_crt_gemm<<<(unsigned)min(wgs, (int64_t)crt_cu_count()), 512, 0, st>>>(RA, RB, L.Mb, L.Nb, L.Kb, L.pA, L.pB, L.pC, tab,
                                                                      RC, wgs);
@@ -2511,7 +2620,8 @@ hipError_t launch_gemm_crt(int colmajor, int64_t m, int64_t n, int64_t k, int t,
   if (e != hipSuccess) return e;
   const int kc = ceil_log2(k < 1 ? 1 : k);
   const int xbits = kc + 2 * t - 3;  // |X| < K 2^(2t-4) < 2^xbits; two's complement needs xbits + 1
-  const unsigned fgrid = (unsigned)((L.Mb * L.Nb + 3) / 4);
+  const int quarters = L.Mb * L.Nb <= 512 ? 1 : 4;  // 2048 waves fill the chip (2 per SIMD)
+  const unsigned fgrid = (unsigned)((L.Mb * L.Nb * (4 / quarters) + 3) / 4);
   uint32_t *list = (uint32_t *)(ws + L.list), *xrec = (uint32_t *)(ws + L.xrec);
   const bool fast = q_iszero(beta) && alpha.lo == 0 && (alpha.hi << 1) == (0x3fffull << 49);
   const int64_t mn = m * n;
@@ -2519,10 +2629,10 @@ hipError_t launch_gemm_crt(int colmajor, int64_t m, int64_t n, int64_t k, int t,
 #define QB_CRT_FIN(XW)                                                                                              \
   if (fast) {                                                                                                     \
     k_crt_finish<XW, true><<<fgrid, 256, 0, st>>>(m, n, k, t, kc, L.Mb, L.Nb, L.pC, RC, tab, eA, fA, eB, fB, alpha, beta, \
-                                                  C, csr, csc, hdr, list, xrec);                                  \
+                                                  C, csr, csc, hdr, list, xrec, quarters);                        \
   } else {                                                                                                        \
     k_crt_finish<XW, false><<<fgrid, 256, 0, st>>>(m, n, k, t, kc, L.Mb, L.Nb, L.pC, RC, tab, eA, fA, eB, fB, alpha,     \
-                                                   beta, C, csr, csc, hdr, list, xrec);                           \
+                                                   beta, C, csr, csc, hdr, list, xrec, quarters);                 \
     k_crt_finish_ab<XW><<<stride_blocks(mn, 256), 256, 0, st>>>(m, n, t, kc, xrec, eA, fA, eB, fB, alpha,    \
                                                                       beta, C, csr, csc, hdr, list);              \
   }
