@@ -187,37 +187,43 @@ QB_HD void cop_columns(uint64_t (&c)[7], const cop &a, const cop &b) {
     c[k] = t;
   }
 }
-// acc = RN(a*b + acc).  Returns false, leaving acc as it was, when the packed operation has to do it.
-QB_HD bool cacc_step(cacc &acc, const cop &a, const cop &b) {
-  uint64_t k[7];
-  cop_columns(k, a, b);
-  // bits 72.. of the product (29-bit digits of the columns) as the frame
-  uint32_t P[5];
+// P >> (sh & ~31), zeros from above, for sh < 160: taken by the wave only when a lane needs it
+QB_HD void ch_shift_words(uint32_t (&P)[5], uint32_t sh) {
+  if (!ch_any(sh >= 32)) return;
+  const uint32_t m4 = ch_mask<7>(sh), m2 = ch_mask<6>(sh), m1 = ch_mask<5>(sh);
+  uint32_t Q[5];
+  Q[0] = ch_sel(m4, P[4], P[0]);
+#pragma unroll
+  for (int i = 1; i < 5; ++i) Q[i] = P[i] & ~m4;
+  P[0] = ch_sel(m2, Q[2], Q[0]);
+  P[1] = ch_sel(m2, Q[3], Q[1]);
+  P[2] = ch_sel(m2, Q[4], Q[2]);
+  P[3] = Q[3] & ~m2;
+  P[4] = Q[4] & ~m2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) P[i] = ch_sel(m1, P[i + 1], P[i]);
+  P[4] &= ~m1;
+}
+// bits 72.. of a product as a frame, its leading bit at 152 or 153
+QB_HD void ch_frame(uint32_t (&P)[5], const uint64_t (&k)[7]) {
   P[0] = (((uint32_t)k[2] >> 14) & 0x7fffu) | ((uint32_t)k[3] << 15);
   P[1] = (((uint32_t)k[3] >> 17) & 0xfffu) | ((uint32_t)k[4] << 12);
   P[2] = (((uint32_t)k[4] >> 20) & 0x1ffu) | ((uint32_t)k[5] << 9);
   P[3] = (((uint32_t)k[5] >> 23) & 0x3fu) | ((uint32_t)k[6] << 6);
   P[4] = ch_alignbit((uint32_t)(k[6] >> 32), (uint32_t)k[6], 26);
+}
+// acc = RN(a*b + acc).  Returns false, leaving acc as it was, when the packed operation has to do it.
+QB_HD bool cacc_step(cacc &acc, const cop &a, const cop &b) {
+  uint64_t k[7];
+  cop_columns(k, a, b);
+  uint32_t P[5];
+  ch_frame(P, k);
   const int32_t Ep = a.e + b.e;
   const int32_t d = acc.E - Ep;
   // d > 0: the product moves right onto the accumulator's grid, by a funnel, after whole words where a
   // lane has a product 2^32 and more below (none has with entries of one scale)
   const int32_t sh = ch_clamp(d, 0, 159);
-  if (ch_any(sh >= 32)) {
-    const uint32_t m4 = ch_mask<7>((uint32_t)sh), m2 = ch_mask<6>((uint32_t)sh), m1 = ch_mask<5>((uint32_t)sh);
-    uint32_t Q[5];
-    Q[0] = ch_sel(m4, P[4], P[0]);
-#pragma unroll
-    for (int i = 1; i < 5; ++i) Q[i] = P[i] & ~m4;
-    P[0] = ch_sel(m2, Q[2], Q[0]);
-    P[1] = ch_sel(m2, Q[3], Q[1]);
-    P[2] = ch_sel(m2, Q[4], Q[2]);
-    P[3] = Q[3] & ~m2;
-    P[4] = Q[4] & ~m2;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) P[i] = ch_sel(m1, P[i + 1], P[i]);
-    P[4] &= ~m1;
-  }
+  ch_shift_words(P, (uint32_t)sh);
   // its sign is applied as a complement; the missing +1 goes in as the sum's carry when no bit of the
   // product lies below the grid
   const uint32_t neg = a.neg ^ b.neg;

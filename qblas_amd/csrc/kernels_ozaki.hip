@@ -32,6 +32,7 @@
 // So the result of every entry has relative error <= 2^-105.9 or is correctly rounded.
 #include <algorithm>
 
+#include "finish_top.hpp"
 #include "wide.hpp"
 #include "kernels.h"
 
@@ -48,6 +49,7 @@ constexpr int OZ_KPASS_BLOCKS = 128;    // k blocks (of 32) per int32 accumulati
 constexpr int OZ_PW = 8;                // signed 32-bit words of a pass sum V (and of N + bias)
 constexpr int OZ_PREC = 8;              // words per pass-sum record (32 bytes)
 constexpr int OZ_FINW = 9;              // words of |sum of passes| in the finish
+constexpr int OZ_FINW_ONE = 6;          // and with one diagonal range (S <= 19: |V| < 2^169, up to 2^21 passes)
 constexpr int32_t OZ_EZERO = INT32_MIN; // row/column exponent of an all-zero row/column
 constexpr uint32_t OZF_NONFINITE = 1u;
 constexpr int OZ_REPAIR_BLOCKS = 1024;
@@ -600,28 +602,32 @@ k_oz_gemm(const int8_t *__restrict__ As, const int8_t *__restrict__ Bs, int64_t 
 // ------------------------------------------------------------------------------------------
 // 4. finish and certification
 // ------------------------------------------------------------------------------------------
+// a / b, a >= 0, b > 0, in 32 bits where they fit (a 64-bit division is about 100 instructions)
+__device__ __forceinline__ int64_t div_small(int64_t a, int64_t b) {
+  return ((a | b) >> 32) == 0 ? (int64_t)((uint32_t)a / (uint32_t)b) : a / b;
+}
 __device__ __forceinline__ bool q_finite_nonzero(q128 x) { return q_bexp(x) != 0x7fffu && !q_iszero(x); }
 
-// Entry (i, j): res = alpha * (sum of its pass records) 2^(E_i+F_j-8(S+1)) + beta y rounded once;
-// true when res is certified (else the entry goes to the exact repair).  kfac = ceil(log2(K (S+1)/4)).
-__device__ __forceinline__ bool oz_finish_value(int64_t i, int64_t j, int S, int kfac, int npass,
-                                                const uint32_t *__restrict__ part, int64_t Mp, int64_t Np,
-                                                const int32_t *__restrict__ eA, const uint32_t *__restrict__ fA,
-                                                const int32_t *__restrict__ eB, const uint32_t *__restrict__ fB,
-                                                q128 alpha, q128 beta, q128 yv, q128 &res) {
+// One entry: res = alpha * (sum of its pass records) 2^(E_i+F_j-8(S+1)) + beta y rounded once, with ei,
+// fi and ej, fj the row's and column's exponent and flags and the records at p, p + step, ...  NW: words
+// the sum of passes needs.  true when res is certified (else the entry goes to the exact repair).
+// kfac = ceil(log2(K (S+1)/4)).
+template <int NW>
+__device__ __forceinline__ bool oz_finish_value(int S, int kfac, int npass, const uint32_t *__restrict__ p, int64_t step,
+                                                int ei, uint32_t fi, int ej, uint32_t fj, q128 alpha, q128 beta, q128 yv,
+                                                q128 &res) {
   const bool ab_ok = (q_bexp(alpha) != 0x7fffu) && (q_bexp(beta) != 0x7fffu) && (q_bexp(yv) != 0x7fffu);
   bool done = false;
-  const bool fin = !((fA[i] | fB[j]) & OZF_NONFINITE);
+  const bool fin = !((fi | fj) & OZF_NONFINITE);
   if (ab_ok && fin && q_iszero(alpha)) {
     // alpha*AB is a zero; beta*y decides unless it is zero too (then the sign of the exact sum matters)
     res = mul_packed(beta, yv);
     done = !q_iszero(res);
-  } else if (ab_ok && fin && eA[i] != OZ_EZERO && eB[j] != OZ_EZERO) {
-    uint32_t V[OZ_FINW];
+  } else if (ab_ok && fin && ei != OZ_EZERO && ej != OZ_EZERO) {
+    uint32_t V[NW];
 #pragma unroll
-    for (int w = 0; w < OZ_FINW; ++w) V[w] = 0;
-    for (int z = 0; z < npass; ++z) {
-      const uint32_t *p = part + ((int64_t)z * Mp * Np + i * Np + j) * OZ_PREC;
+    for (int w = 0; w < NW; ++w) V[w] = 0;
+    for (int z = 0; z < npass; ++z, p += step) {
       const i32x4v v0 = *reinterpret_cast<const i32x4v *>(p);
       const i32x4v v1 = *reinterpret_cast<const i32x4v *>(p + 4);
       const uint32_t x[OZ_PW] = {(uint32_t)v0.x, (uint32_t)v0.y, (uint32_t)v0.z, (uint32_t)v0.w, (uint32_t)v1.x,
@@ -629,19 +635,17 @@ __device__ __forceinline__ bool oz_finish_value(int64_t i, int64_t j, int S, int
       const uint32_t ext = (x[OZ_PW - 1] >> 31) ? 0xffffffffu : 0u;
       uint32_t c = 0;
 #pragma unroll
-      for (int w = 0; w < OZ_FINW; ++w) V[w] = addc32(V[w], w < OZ_PW ? x[w] : ext, c, c);
+      for (int w = 0; w < NW; ++w) V[w] = addc32(V[w], w < OZ_PW ? x[w] : ext, c, c);
     }
-    const uint32_t sgn = V[OZ_FINW - 1] >> 31;
-    if (sgn) {
-      uint32_t c = 1;
+    const uint32_t sgn = V[NW - 1] >> 31;
+    uint32_t c = sgn;
 #pragma unroll
-      for (int w = 0; w < OZ_FINW; ++w) V[w] = addc32(~V[w], 0u, c, c);
-    }
-    if (!rzero<OZ_FINW>(V)) {
-      const int Ei = eA[i] + 3, Fj = eB[j] + 3;
+    for (int w = 0; w < NW; ++w) V[w] = addc32(V[w] ^ (0u - sgn), 0u, c, c);
+    if (!rzero<NW>(V)) {
+      const int Ei = ei + 3, Fj = ej + 3;
       const int lsb = Ei + Fj - 8 * (S + 1);
       int terr;
-      res = finish_reg_top<OZ_FINW>(V, lsb, sgn, alpha, beta, yv, terr);
+      res = finish_top<NW>(V, lsb, sgn, alpha, beta, yv, terr);
       if (q_finite_nonzero(res)) {
         const int ea = unpack_finite(alpha).e;
         const int bexp = ea + 1 + kfac + Ei + Fj - 8 * S;  // |alpha (AB - P)| < 2^bexp
@@ -655,6 +659,7 @@ __device__ __forceinline__ bool oz_finish_value(int64_t i, int64_t j, int S, int
 }
 
 // One thread per output (i, j), j fastest.
+template <int NW>
 __global__ void __launch_bounds__(256) k_oz_finish(int64_t M, int64_t N, int S, int kfac, int npass,
                                                    const uint32_t *__restrict__ part, int64_t Mp, int64_t Np,
                                                    const int32_t *__restrict__ eA, const uint32_t *__restrict__ fA,
@@ -663,10 +668,11 @@ __global__ void __launch_bounds__(256) k_oz_finish(int64_t M, int64_t N, int S, 
                                                    int64_t csc, uint32_t *__restrict__ hdr, uint32_t *__restrict__ list) {
   const int64_t stride = (int64_t)gridDim.x * 256;
   for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < M * N; g += stride) {
-    const int64_t i = g / N, j = g - i * N;
+    const int64_t i = div_small(g, N), j = g - i * N;
     q128 *cp = C + i * csr + j * csc;
     q128 res;
-    if (oz_finish_value(i, j, S, kfac, npass, part, Mp, Np, eA, fA, eB, fB, alpha, beta, ldq_c(cp), res)) {
+    if (oz_finish_value<NW>(S, kfac, npass, part + (i * Np + j) * OZ_PREC, Mp * Np * OZ_PREC, eA[i], fA[i], eB[j], fB[j],
+                            alpha, beta, ldq_c(cp), res)) {
       stq_c(cp, res);
     } else {
       const uint32_t slot = atomicAdd(hdr + 1, 1u);
@@ -1039,9 +1045,13 @@ hipError_t launch_gemm_ozaki(int colmajor, int64_t m, int64_t n, int64_t k, int 
   while ((double)(1ull << (kfac < 62 ? kfac : 62)) < kb && kfac < 80) ++kfac;
   const int64_t mn = m * n;
   if (gate && (e = gate->fn(gate->arg, st)) != hipSuccess) return e;
-  k_oz_finish<<<stride_blocks(mn, 256), 256, 0, st>>>(m, n, S, kfac, (int)L.npass, (const uint32_t *)(ws + L.part),
-                                                            L.Mp, L.Np, eA, fA, eB, fB, alpha, beta, C, csr, csc, hdr,
-                                                            (uint32_t *)(ws + L.list));
+#define QB_OZ_FIN(NW)                                                                                                  \
+  k_oz_finish<NW><<<stride_blocks(mn, 256), 256, 0, st>>>(m, n, S, kfac, (int)L.npass, (const uint32_t *)(ws + L.part), \
+                                                          L.Mp, L.Np, eA, fA, eB, fB, alpha, beta, C, csr, csc, hdr,  \
+                                                          (uint32_t *)(ws + L.list))
+  if (S <= OZ_ONE_RANGE_MAX) QB_OZ_FIN(OZ_FINW_ONE);
+  else QB_OZ_FIN(OZ_FINW);
+#undef QB_OZ_FIN
   if (ev) (void)hipEventRecord(ev[3], st);
   return oz_repair_queue(m, n, k, A, asr, asc, B, bsr, bsc, eA, eB, alpha, beta, C, csr, csc, hdr,
                          (uint32_t *)(ws + L.list), (q128 *)(ws + L.bt), st, ev);
@@ -1126,7 +1136,8 @@ enum {
   BO_TILES,     // 64x64 product tiles times k passes
   BO_ENT,       // outputs m n
   BO_SCA,       // scaling items of A: rows (RowMajor) or groups of 64 rows (ColMajor)
-  BO_SCB        // of B: groups of 64 columns (RowMajor) or columns (ColMajor)
+  BO_SCB,       // of B: groups of 64 columns (RowMajor) or columns (ColMajor)
+  BO_FIN        // workgroups of the finish: 256 outputs each, of one problem
 };
 
 struct bo_geom {
@@ -1175,14 +1186,17 @@ __device__ __forceinline__ int64_t bo_find_from(const int64_t *__restrict__ off,
   return p;
 }
 
-// off[0][*] = 0, off[p + 1][f] = sum of count f over problems 0..p; one block, 1024 problems a chunk
+// off[0][*] = 0, off[p + 1][f] = sum of count f over problems 0..p; one block, 1024 problems a chunk:
+// prefix sums of all counts by shuffles in each wave, then over the 16 waves' totals (a scan through LDS
+// a count at a time, 20 barriers each, took 70 us for 4096 problems, this 38)
 __global__ void __launch_bounds__(1024) k_bo_scan(const qblas_gemm_problem *__restrict__ P, int64_t count,
                                                   int colmajor, int64_t *__restrict__ off) {
-  __shared__ int64_t s[1024];
-  int64_t base[BO_F];
-#pragma unroll
-  for (int f = 0; f < BO_F; ++f) base[f] = 0;
-  if (threadIdx.x < BO_F) off[threadIdx.x] = 0;
+  __shared__ int64_t s_tot[16][BO_F], s_base[17][BO_F];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x < BO_F) {
+    off[threadIdx.x] = 0;
+    s_base[16][threadIdx.x] = 0;  // the chunks before
+  }
   for (int64_t b = 0; b < count; b += 1024) {
     const int64_t p = b + threadIdx.x;
     int64_t v[BO_F];
@@ -1199,20 +1213,31 @@ __global__ void __launch_bounds__(1024) k_bo_scan(const qblas_gemm_problem *__re
       v[BO_ENT] = G.m * G.n;
       v[BO_SCA] = colmajor ? (G.m + 63) / 64 : G.m;
       v[BO_SCB] = colmajor ? G.n : (G.n + 63) / 64;
+      v[BO_FIN] = (G.m * G.n + 255) / 256;
     }
 #pragma unroll
     for (int f = 0; f < BO_F; ++f) {
-      s[threadIdx.x] = v[f];
-      __syncthreads();
-      for (int o = 1; o < 1024; o <<= 1) {
-        const int64_t t = (threadIdx.x >= o) ? s[threadIdx.x - o] : 0;
-        __syncthreads();
-        s[threadIdx.x] += t;
-        __syncthreads();
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int64_t t = __shfl_up((long long)v[f], o);
+        v[f] += lane >= o ? t : 0;
       }
-      if (p < count) off[(p + 1) * BO_F + f] = base[f] + s[threadIdx.x];
-      base[f] += s[1023];
-      __syncthreads();
+      if (lane == 63) s_tot[wave][f] = v[f];
+    }
+    __syncthreads();
+    if (threadIdx.x < BO_F) {
+      int64_t t = s_base[16][threadIdx.x];
+#pragma unroll
+      for (int w = 0; w < 16; ++w) {
+        s_base[w][threadIdx.x] = t;
+        t += s_tot[w][threadIdx.x];
+      }
+      s_base[16][threadIdx.x] = t;
+    }
+    __syncthreads();
+    if (p < count) {
+#pragma unroll
+      for (int f = 0; f < BO_F; ++f) off[(p + 1) * BO_F + f] = s_base[wave][f] + v[f];
     }
   }
 }
@@ -1332,29 +1357,35 @@ k_bo_gemm(const qblas_gemm_problem *__restrict__ P, int64_t count, const int64_t
                                G.Kb, G.Mp, G.Np, tm, tn, kp, 0, part + o[BO_PART] * OZ_PREC);
 }
 
-// one thread per output of every problem; uncertified entries queue (problem, i, j)
+// one thread per output, a workgroup's 256 of one problem, whose descriptor and offsets it reads by scalar
+// loads (the constant address space: no store of the kernel goes there); uncertified entries queue
+// (problem, i, j).  Bound by VALU issue (444 instructions a wave) and by the records and C (64 bytes an
+// entry): 4096 problems of 8..256, 71 million entries, 1.30 ms; 2.11 ms with the 12-word epilogue and every
+// lane reading its own descriptor.
 __global__ void __launch_bounds__(256) k_bo_finish(const qblas_gemm_problem *__restrict__ P, int64_t count,
-                                                   const int64_t *__restrict__ off, int colmajor, int S, int64_t total,
+                                                   const int64_t *__restrict__ off, int colmajor, int S,
                                                    const uint32_t *__restrict__ part, const int32_t *__restrict__ eA,
                                                    const uint32_t *__restrict__ fA, const int32_t *__restrict__ eB,
                                                    const uint32_t *__restrict__ fB, uint32_t *__restrict__ hdr,
                                                    uint32_t *__restrict__ list) {
   if (hdr[OZ_HDR_STALE]) return;  // nothing queued: the repair has nothing to do either
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (g >= total) return;
-  const int64_t p = bo_find_from(off, count, BO_ENT, (int64_t)blockIdx.x * 256, g);
-  const qblas_gemm_problem &pr = P[p];
-  const bo_geom G = bo_geometry(pr, colmajor);
-  const int64_t *o = off + p * BO_F;
-  const int64_t u = g - o[BO_ENT];
-  const int64_t i = u / G.n, j = u - i * G.n;
-  int kfac = 0;  // ceil(log2(K (S+1) / 4))
-  while ((4ll << kfac) < G.k * (S + 1)) ++kfac;
-  q128 *cp = (q128 *)pr.C + i * G.csr + j * G.csc;
+  const int64_t p = bo_find(off, count, BO_FIN, blockIdx.x);  // uniform
+  const auto *pr = (const __attribute__((address_space(4))) qblas_gemm_problem *)(uintptr_t)(P + p);
+  const auto *o = (const __attribute__((address_space(4))) int64_t *)(uintptr_t)(off + p * BO_F);
+  // a problem has fewer than 2^32 entries (one thread each)
+  const uint32_t u = (uint32_t)((int64_t)blockIdx.x - o[BO_FIN]) * 256u + threadIdx.x;
+  const uint32_t n = (uint32_t)pr->n, i = u / n, j = u - i * n;
+  if (i >= (uint32_t)pr->m) return;
+  const int64_t ldc = pr->ldc, k = pr->k, kb = k * (S + 1);
+  const int kfac = kb <= 4 ? 0 : 62 - clz64((uint64_t)(kb - 1));  // ceil(log2(K (S+1) / 4))
+  const int npass = (int)(((k + 31) / 32 + OZ_KPASS_BLOCKS - 1) / OZ_KPASS_BLOCKS);
+  const int64_t Np = (pr->n + OZ_TILE - 1) / OZ_TILE * OZ_TILE, Mp = (pr->m + OZ_TILE - 1) / OZ_TILE * OZ_TILE;
+  q128 *cp = (q128 *)pr->C + (colmajor ? j * ldc + i : i * ldc + j);
+  const int64_t ri = o[BO_ROWS] + i, cj = o[BO_COLS] + j;
+  const q128 alpha = q_make(pr->alpha[0], pr->alpha[1]), beta = q_make(pr->beta[0], pr->beta[1]);
   q128 res;
-  if (oz_finish_value(i, j, S, kfac, (int)G.npk, part + o[BO_PART] * OZ_PREC, G.Mp, G.Np, eA + o[BO_ROWS],
-                      fA + o[BO_ROWS], eB + o[BO_COLS], fB + o[BO_COLS], q_make(pr.alpha[0], pr.alpha[1]),
-                      q_make(pr.beta[0], pr.beta[1]), ldq_c(cp), res)) {
+  if (oz_finish_value<OZ_FINW_ONE>(S, kfac, npass, part + (o[BO_PART] + i * Np + j) * OZ_PREC, Mp * Np * OZ_PREC, eA[ri],
+                                   fA[ri], eB[cj], fB[cj], alpha, beta, ldq_c(cp), res)) {
     stq_c(cp, res);
   } else {
     const uint32_t slot = atomicAdd(hdr + 1, 1u);
@@ -1472,7 +1503,7 @@ static void bo_launch(int colmajor, int64_t count, const qblas_gemm_problem *P, 
   k_bo_slice<S><<<(unsigned)((ta + 255) / 256), 256, 0, st>>>(P, count, off, colmajor, 0, ta, eA, sA, hdr);
   k_bo_slice<S><<<(unsigned)((tb + 255) / 256), 256, 0, st>>>(P, count, off, colmajor, 1, tb, eB, sB, hdr);
   k_bo_gemm<S><<<(unsigned)tot[BO_TILES], 256, 0, st>>>(P, count, off, colmajor, sA, sB, part, hdr);
-  k_bo_finish<<<(unsigned)((tot[BO_ENT] + 255) / 256), 256, 0, st>>>(P, count, off, colmajor, S, tot[BO_ENT], part,
+  k_bo_finish<<<(unsigned)tot[BO_FIN], 256, 0, st>>>(P, count, off, colmajor, S, part,
                                                                        eA, fA, eB, fB, hdr, list);
   uint32_t *wq = list + 4 * tot[BO_ENT];
   k_bo_repair<<<OZ_REPAIR_BLOCKS, OZR_BS, 0, st>>>(P, count, off, colmajor, eA, eB, hdr, list, wq);
@@ -1490,7 +1521,7 @@ hipError_t launch_gemm_ozaki_batched(int colmajor, int64_t count, const qblas_ge
   // grids: one workgroup per tile, one thread per entry and per (fragment position, lane), one
   // wave per scaling item; queued entries are numbered in 32 bits
   const int64_t ni = tot[BO_ROWS] > tot[BO_COLS] ? tot[BO_ROWS] : tot[BO_COLS];
-  if (!grid_fits(tot[BO_TILES], 256) || !grid_fits((tot[BO_ENT] + 255) / 256, 256) ||
+  if (!grid_fits(tot[BO_TILES], 256) || !grid_fits(tot[BO_FIN], 256) ||
       !grid_fits(tot[BO_FRAGA] / 4 + 1, 256) || !grid_fits(tot[BO_FRAGB] / 4 + 1, 256) ||
       !grid_fits((tot[BO_SCA] + 3) / 4, 256) || !grid_fits((tot[BO_SCB] + 3) / 4, 256) ||
       !grid_fits((ni + 255) / 256 + 1, 256) || count > 0xffffffffll)
@@ -2444,7 +2475,7 @@ __global__ void __launch_bounds__(256) k_crt_finish_ab(int64_t M, int64_t N, int
   constexpr int RW = (XW + 3) & ~3;
   const int64_t stride = (int64_t)gridDim.x * 256;
   for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < M * N; g += stride) {
-    const int64_t i = g / N, j = g - i * N;
+    const int64_t i = div_small(g, N), j = g - i * N;
     q128 *cp = C + i * csr + j * csc;
     const q128 yv = ldq_c(cp);
     const bool ab_ok = (q_bexp(alpha) != 0x7fffu) && (q_bexp(beta) != 0x7fffu) && (q_bexp(yv) != 0x7fffu);
@@ -2474,7 +2505,7 @@ __global__ void __launch_bounds__(256) k_crt_finish_ab(int64_t M, int64_t N, int
       if (!rzero<XW>(X)) {
         const int Ei = eA[i] + 3, Fj = eB[j] + 3;
         int terr;
-        res = finish_reg_top<XW>(X, Ei + Fj - 2 * t, sgn, alpha, beta, yv, terr);
+        res = finish_top<XW>(X, Ei + Fj - 2 * t, sgn, alpha, beta, yv, terr);
         if (q_finite_nonzero(res)) {
           const int bexp = unpack_finite(alpha).e + 1 + kc + Ei + Fj - t - 2;
           const int eb = (terr == INT_MIN) ? bexp : max(bexp, terr) + 1;  // with the epilogue's cut
