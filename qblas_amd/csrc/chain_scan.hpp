@@ -19,6 +19,8 @@
 // binades bmin .. bmin + 13 fit 128 bits.  A product of zero leaves S as it is; steps that are done
 // count as such products.
 #pragma once
+#include <utility>
+
 #include "chain.hpp"
 
 namespace qb {
@@ -256,7 +258,7 @@ QB_HD bool sc_inside(uint32_t S3, int32_t k) {
 #if defined(__HIPCC__)
 template <int CTRL, int ROWS>
 __device__ __forceinline__ uint32_t sc_dpp(uint32_t x) {  // 0 where there is no source lane
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, ROWS == 0xf);
 }
 template <int CTRL, int ROWS>
 __device__ __forceinline__ void sc_scan_step(uint32_t (&v)[4]) {
@@ -272,13 +274,21 @@ __device__ __forceinline__ void sc_scan_step(double &v) {
   const uint32_t lo = sc_dpp<CTRL, ROWS>((uint32_t)u), hi = sc_dpp<CTRL, ROWS>((uint32_t)(u >> 32));
   v += __longlong_as_double(((uint64_t)hi << 32) | lo);
 }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void sc_scan_step(uint32_t &v) {
+  v += sc_dpp<CTRL, ROWS>(v);
+}
 // inclusive prefix sum over the wave: rows of 16 lanes by shifts, then the rows' totals
 template <typename X>
-__device__ __forceinline__ void sc_scan(X &v) {
+__device__ __forceinline__ void sc_scan_row(X &v) {
   sc_scan_step<0x111, 0xf>(v);
   sc_scan_step<0x112, 0xf>(v);
   sc_scan_step<0x114, 0xf>(v);
   sc_scan_step<0x118, 0xf>(v);
+}
+template <typename X>
+__device__ __forceinline__ void sc_scan(X &v) {
+  sc_scan_row(v);
   sc_scan_step<0x142, 0xa>(v);  // row_bcast:15
   sc_scan_step<0x143, 0xc>(v);  // row_bcast:31
 }
@@ -308,20 +318,16 @@ struct sc_const {
   __device__ __forceinline__ q128 operator()(int64_t) const { return v; }
 };
 
-// S = RN(S + a(i) b(i)) for i = 0..n-1 by one whole wave; every lane returns the result.  init, a, b
-// and n are the same in all lanes.
+// S = RN(S + a(i) b(i)) for i = pos..n-1 by one whole wave.  s (in scalar registers), a, b, pos and n are
+// the same in all lanes.
 template <typename LA, typename LB>
-__device__ __forceinline__ q128 wave_chain(q128 init, const LA a, const LB b, int64_t n) {
+__device__ __forceinline__ void wave_steps(sstate &s, const LA a, const LB b, int64_t pos, int64_t n) {
   const int lane = (int)(threadIdx.x & 63);
-  sstate s;  // the same in all lanes, in scalar registers
-  sstate_set(s, init);
-  sstate_uniform(s);
   q128 qa = q_zero(0), qb_ = q_zero(0);
-  if (lane < n) {
-    qa = a(lane);
-    qb_ = b(lane);
+  if (pos + lane < n) {
+    qa = a(pos + lane);
+    qb_ = b(pos + lane);
   }
-  int64_t pos = 0;
   while (pos < n) {
     const int cnt = (int)((n - pos < 64) ? n - pos : 64);
     // the next block's operands (read again below if this block ends early)
@@ -337,7 +343,11 @@ __device__ __forceinline__ q128 wave_chain(q128 init, const LA a, const LB b, in
     while (lo < cnt) {
       int cut = lo;  // steps before it are final after this pass; step `cut` is done by itself
       if (s.kind == 2 && s.b == QBIAS + 1) {  // Inf or NaN
-        if (q_isnan(sstate_get(s))) return q_nan();
+        if (q_isnan(sstate_get(s))) {
+          sstate_set(s, q_nan());
+          sstate_uniform(s);
+          return;
+        }
         // an infinity stays until an operand is not finite
         const int64_t at = pos + lane;
         const uint64_t odd =
@@ -411,6 +421,279 @@ __device__ __forceinline__ q128 wave_chain(q128 init, const LA a, const LB b, in
         qb_ = b(i);
       }
     }
+  }
+}
+// a whole chain of n steps from init; every lane returns the result
+template <typename LA, typename LB>
+__device__ __forceinline__ q128 wave_chain(q128 init, const LA a, const LB b, int64_t n) {
+  sstate s;
+  sstate_set(s, init);
+  sstate_uniform(s);
+  wave_steps(s, a, b, 0, n);
+  return sstate_get(s);
+}
+
+// The same by a workgroup of SG_WAVES waves, SG_PER consecutive steps a lane and SG_STEPS at a time, for a
+// launch of fewer chains than the chip has CUs.  Each wave does its steps as above from the predicted sum
+// before them; the exact sums before a wave are the state and the totals of the waves before it, and the
+// rounding done again at climbs and ties goes through one list in step order, by the first wave.  A wave does
+// not know the binade that the one before ends in, so its first product counts as a climb.  The window of
+// binades lies below the largest of the sums at the waves' ends (the state's rule where that would cut the
+// state itself).  Where a sum leaves the window, or the state is not of kind 0, the next 64 steps are one
+// wave's work, which every wave does for itself.  Every barrier is met by all waves: what decides is the same
+// in all of them.
+constexpr int SG_WAVES = 8;  // at most 16: a row of lanes holds a value of each
+constexpr int SG_PER = 4;    // two prefix sums for 256 steps of a wave
+constexpr int SG_SPAN = 64 * SG_PER;
+constexpr int SG_STEPS = SG_SPAN * SG_WAVES;
+struct sg_lds {
+  double dsum[16];         // the waves' sums of products, in double precision
+  uint4 total[16];         // of rounded products
+  uint32_t fixes[16];      // roundings to be done again
+  uint4 list[SG_STEPS];    // of each: sum + product below the grid, doubled (sg_fix)
+  uint32_t corr[SG_STEPS]; // the correction of the sums from there on
+  uint4 end[16];           // the sum after the wave's last good step
+  int cut[16];             // good steps
+};
+// sc_fix as a step E -> ((A + E + add + ((A + E) & odd ? 1 : 0)) & grid) - after on the corrections so far, E, in
+// halves of 2^(bmin - 112): A is the exact sum before the step plus the product's floor; what lies below A
+// takes the tie's place of the odd bit
+struct sg_fix {
+  uint32_t A, odd, after;
+  int32_t k;
+};
+__device__ __forceinline__ sg_fix sg_make_fix(const slane &l, uint32_t S0) {
+  const uint64_t z = ((uint64_t)(S0 - l.v[0]) << 32) + (((uint64_t)l.x1 << 32) | l.x0);
+  const bool low = l.lost || ((uint32_t)z & 0x7fffffffu) != 0;
+  sg_fix r;
+  r.A = (uint32_t)(z >> 31);
+  r.k = l.k + 1;
+  r.odd = low ? 0u : 1u << r.k;
+  r.after = S0 << 1;
+  return r;
+}
+// The fixes of lanes F0 .. F0 + 7, z = A + E of the first one in, (E + after) of the last one out; the next
+// one's z is (E + after) + C.  Inline assembly: the condition of the AND is the addition's carry, which the
+// compiler makes with two compares and a select, and a lane is written by its number.
+template <int F0, int... F>
+__device__ __forceinline__ void sg_fix_eight(uint32_t &z, uint32_t &kept, uint32_t C, uint32_t odd, uint32_t add,
+                                             uint32_t grid, std::integer_sequence<int, F...>) {
+  (([&] {
+     uint32_t r = z;
+     if (F0 + F > 0) r += sc_lane(C, F0 + F);
+     asm("s_and_b32 %0, %1, %2\n\ts_addc_u32 %0, %1, %3"
+         : "=&s"(z)
+         : "s"(r), "s"(sc_lane(odd, F0 + F)), "s"(sc_lane(add, F0 + F))
+         : "scc");
+     z &= sc_lane(grid, F0 + F);
+     asm("v_writelane_b32 %0, %1, %2" : "+v"(kept) : "s"(z), "n"(F0 + F));
+   }()),
+   ...);
+}
+template <int... G>
+__device__ __forceinline__ void sg_fix_lanes(uint32_t &z, uint32_t &kept, uint32_t C, uint32_t odd, uint32_t add,
+                                             uint32_t grid, int cnt, std::integer_sequence<int, G...>) {
+  (void)((8 * G < cnt &&
+          (sg_fix_eight<8 * G>(z, kept, C, odd, add, grid, std::make_integer_sequence<int, 8>{}), true)) &&
+         ...);
+}
+template <typename LA, typename LB>
+__device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, int64_t n, sg_lds &lds) {
+  const int lane = (int)(threadIdx.x & 63), wl = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (threadIdx.x < 16) {  // waves that the workgroup does not have
+    lds.dsum[wl] = 0.0;
+    lds.total[wl] = make_uint4(0, 0, 0, 0);
+    lds.fixes[wl] = 0;
+    lds.cut[wl] = SG_SPAN;
+  }
+  __syncthreads();
+  sstate s;
+  sstate_set(s, init);
+  sstate_uniform(s);
+  int64_t pos = 0;
+  q128 qa[SG_PER], qb_[SG_PER];
+  auto fetch = [&](int64_t at) {
+    const int64_t i = at + SG_PER * (int)threadIdx.x;
+#pragma unroll
+    for (int r = 0; r < SG_PER; ++r) {
+      qa[r] = qb_[r] = q_zero(0);
+      if (i + r < n) {
+        qa[r] = a(i + r);
+        qb_[r] = b(i + r);
+      }
+    }
+  };
+  fetch(0);
+  for (bool single = true; pos < n;) {  // the first sums climb and fall through many binades
+    if (single || s.kind != 0) {
+      const int64_t to = n - pos < 64 ? n : pos + 64;
+      wave_steps(s, a, b, pos, to);
+      if (s.kind == 2 && q_isnan(sstate_get(s))) return q_nan();
+      pos = to;
+      fetch(pos);
+      single = false;
+      continue;
+    }
+    sprod p[SG_PER];
+    double d[SG_PER];  // sums of the lane's products
+    bool any = false;  // the lane has a product
+#pragma unroll
+    for (int r = 0; r < SG_PER; ++r) {
+      p[r] = sc_product(qa[r], qb_[r]);
+      if (pos + SG_PER * (int)threadIdx.x + r >= n) sc_clear(p[r]);
+      any |= p[r].Ep != -SC_BIG;
+      const double v = sc_value(p[r], s.b);
+      d[r] = r ? d[r ? r - 1 : 0] + v : v;
+    }
+    fetch(pos + SG_STEPS);  // the next steps' operands (read again below if these end early)
+    double dt = d[SG_PER - 1];
+    sc_scan(dt);
+    if (lane == 63) lds.dsum[wv] = dt;
+    __syncthreads();
+    // the sum before the wave, and the largest binade at a wave's end
+    double before = lds.dsum[wl];
+    sc_scan_row(before);
+    before += sc_first(s);
+    int32_t top = sc_binade(before, s.b);
+    if (top == SC_BIG) top = s.b;
+#pragma unroll
+    for (int i = 1; i < 16; i <<= 1) top = max(top, __shfl_xor(top, i));
+    top = max(__builtin_amdgcn_readfirstlane(top), s.b);
+    int32_t bmin = top + 2 - SC_WIN;
+    if (bmin > s.b) bmin = s.b - SC_LOW;
+    const uint64_t bu = __double_as_longlong(before);
+    const int wp = wv ? wv - 1 : 0;  // the wave before
+    const double d0 =
+        wv ? __longlong_as_double(((uint64_t)sc_lane((uint32_t)(bu >> 32), wp) << 32) | sc_lane((uint32_t)bu, wp)) : sc_first(s);
+    // the sums before the lane: exact differences do not matter, only that a lane's own are used throughout
+    const double dl = (dt - d[SG_PER - 1]) + d0;
+    int32_t bi[SG_PER], last = 0;
+#pragma unroll
+    for (int r = 0; r < SG_PER; ++r) {
+      bi[r] = sc_binade(dl + d[r], s.b);
+      last = p[r].Ep != -SC_BIG ? bi[r] : last;
+    }
+    const uint64_t lanes_below = (1ull << lane) - 1;
+    const uint64_t below = __ballot(any) & lanes_below;
+    int32_t bp = __builtin_amdgcn_ds_bpermute(4 * (63 - clz64(below)), last);
+    if (below == 0) bp = -SC_BIG;  // unknown: a climb
+    slane l[SG_PER];
+    uint32_t V[SG_PER][4];  // sums of the lane's rounded products
+    int at = 0, mine = 0, all = 0;  // fixes before the lane, of the lane, of the wave
+#pragma unroll
+    for (int r = 0; r < SG_PER; ++r) {
+      l[r] = sc_round(p[r], bi[r], bp, bmin);
+      bp = p[r].Ep != -SC_BIG ? bi[r] : bp;
+      uint32_t c = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) V[r][i] = r ? ch_addc(V[r ? r - 1 : 0][i], l[r].v[i], c, c) : l[r].v[i];
+      const uint64_t fm = __ballot(l[r].fix);
+      at += __popcll(fm & lanes_below);
+      all += __popcll(fm);
+    }
+    uint32_t S[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[i] = V[SG_PER - 1][i];
+    sc_scan(S);
+    if (lane == 63) {
+      lds.total[wv] = make_uint4(S[0], S[1], S[2], S[3]);
+      lds.fixes[wv] = (uint32_t)all;
+    }
+    __syncthreads();
+    uint32_t fx = lds.fixes[wl];
+    sc_scan_row(fx);
+    at += wv ? (int)sc_lane(fx, wp) : 0;
+    const int fixes = (int)sc_lane(fx, 15);
+    {
+      const uint4 t = lds.total[wl];
+      uint32_t B[4] = {t.x, t.y, t.z, t.w};
+      sc_scan_row(B);
+      // the state in units of 2^(bmin - 112): s.b - bmin is 0..SC_WIN - 2, the leading bit of w at 112 + SC_LOW
+      const int up = s.b - bmin - SC_LOW;
+      uint64_t lo = ((uint64_t)s.w[1] << 32) | s.w[0], hi = ((uint64_t)s.w[3] << 32) | s.w[2];
+      if (up >= 0) {
+        hi = shl_fill(hi, lo, up);
+        lo <<= up;
+      } else {  // the bits below the leading 113 are zero
+        lo = shr_fill(hi, lo, -up);
+        hi >>= -up;
+      }
+      const uint32_t w[4] = {(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+      uint32_t c = s.neg & 1u, c2 = 0, c3 = 1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // the sum before the lane
+        const uint32_t base = ch_addc(w[i] ^ s.neg, wv ? sc_lane(B[i], wp) : 0u, c, c);
+        S[i] = ch_addc(S[i], base, c2, c2);
+        S[i] = ch_addc(S[i], ~V[SG_PER - 1][i], c3, c3);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < SG_PER; ++r) {
+      if (l[r].fix) {
+        const sg_fix f = sg_make_fix(l[r], S[0] + V[r][0]);
+        lds.list[at + mine] = make_uint4(f.A, f.odd, f.after, (uint32_t)f.k);
+        ++mine;
+      }
+    }
+    __syncthreads();
+    if (wv == 0) {  // one by one, in scalar registers
+      uint32_t E = 0;
+      for (int f0 = 0; f0 < fixes; f0 += 64) {
+        const int cnt = fixes - f0 < 64 ? fixes - f0 : 64;
+        const uint4 u = lds.list[f0 + (lane < cnt ? lane : 0)];
+        const uint32_t add = (1u << (u.w - 1)) - (u.y ? 1u : 0u), grid = 0u - (1u << u.w);
+        const uint32_t C = u.x - (uint32_t)__shfl_up((int)u.z, 1);
+        uint32_t z = sc_lane(u.x, 0) + E, kept = 0;  // kept: (E + after) of the lane's fix
+        sg_fix_lanes(z, kept, C, u.y, add, grid, cnt, std::make_integer_sequence<int, 8>{});
+        E = z - sc_lane(u.z, 63);
+        if (lane < cnt) lds.corr[f0 + lane] = (uint32_t)((int32_t)(kept - u.z) >> 1);
+      }
+    }
+    __syncthreads();
+    // the sums of the lane's steps, checked: `good` of them are final, the last of those in S
+    uint32_t corr = at ? lds.corr[at - 1] : 0u;
+    uint32_t G[4];
+    int good = 0;
+    bool still = true;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) G[i] = 0;
+#pragma unroll
+    for (int r = 0; r < SG_PER; ++r) {
+      if (l[r].fix) corr = lds.corr[at++];
+      const uint32_t x = (uint32_t)((int32_t)corr >> 31);
+      uint32_t c = 0, c2 = 0, X[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        X[i] = ch_addc(S[i], V[r][i], c, c);
+        X[i] = ch_addc(X[i], i ? x : corr, c2, c2);
+      }
+      still = still && !p[r].bad && (p[r].Ep == -SC_BIG || (l[r].live && sc_inside(X[3], l[r].k)));
+      good += still ? 1 : 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) G[i] = still ? X[i] : G[i];
+    }
+    const uint64_t badm = ~__ballot(good == SG_PER);
+    const int bl = badm ? __ffsll((unsigned long long)badm) - 1 : 64;  // the first lane that fails
+    const int bg = bl < 64 ? (int)sc_lane((uint32_t)good, bl & 63) : 0;
+    const int el = bg ? bl : bl - 1;  // the lane of the last good step
+    if (lane == (el < 0 ? 0 : el)) {
+      lds.end[wv] = make_uint4(G[0], G[1], G[2], G[3]);
+      lds.cut[wv] = SG_PER * bl + bg;
+    }
+    __syncthreads();
+    const uint64_t early = __ballot(lane < SG_WAVES && lds.cut[wl] < SG_SPAN);
+    const int w = early ? __ffsll((unsigned long long)early) - 1 : SG_WAVES - 1;
+    const int cut = __builtin_amdgcn_readfirstlane(lds.cut[w]);
+    const int done = SG_SPAN * w + cut;
+    if (done) {
+      const uint4 t = lds.end[cut ? w : w - 1];
+      const uint32_t T[4] = {t.x, t.y, t.z, t.w};
+      sstate_from_sum(s, T, bmin);
+      sstate_uniform(s);
+    }
+    pos += done;
+    single = done < SG_STEPS;
   }
   return sstate_get(s);
 }

@@ -44,6 +44,22 @@ __device__ __forceinline__ void chunk_range(int64_t n, int T, int t, int64_t &s,
   e = (t == T - 1) ? n : s + chunk;
 }
 
+// a contiguous chunk's value from its two chains' and, of an odd length, its last element (at e - 1)
+__device__ __forceinline__ q128 dot_pair_end(q128 r, q128 a, const q128 *__restrict__ x, const q128 *__restrict__ y,
+                                             int64_t e, int odd) {
+  q128 b = q_one();
+#pragma unroll 1
+  for (int op = 0; op < 1 + odd; ++op) {
+    cacc acc;
+    cacc_set(acc, r);
+    chain_fma(acc, a, b);
+    r = cacc_get(acc);
+    a = ld(x + e - 1);
+    b = ld(y + e - 1);
+  }
+  return r;
+}
+
 // Contiguous: chunk t is two chains, lane p's over elements start+p, start+p+2, ... for i < len/2
 // (dot_kernel_vectorized, level1.hpp:20-25), combined by horizontal_sum (quad_vector.hpp:141-150) and
 // the odd tail's fma (level1.hpp:29-32).  Strided: one serial chain per chunk (level1.hpp:111-114,
@@ -51,8 +67,7 @@ __device__ __forceinline__ void chunk_range(int64_t n, int T, int t, int64_t &s,
 // (chain_scan.hpp); a workgroup is one chunk.  part[t] receives the chunk's value, or, with one
 // chunk, out the result ('direct': n < 500 returns the kernel's value without the final
 // "0 + partial" sum, level1.hpp:40-43, :128-134).
-// Bound by the latency of a block of 64 steps.  2^20 elements, T = 16: 0.93 ms (39 ms with one lane
-// per chain and the packed step, 18 ms with chain.hpp's step).
+// Bound by the latency of a block of 64 steps, about 1.8 us.
 __global__ void __launch_bounds__(128) k_dot_ref_chunks(const q128 *__restrict__ x, int64_t incx,
                                                         const q128 *__restrict__ y, int64_t incy, int64_t n, int T,
                                                         int direct, q128 *__restrict__ part, q128 *__restrict__ out) {
@@ -69,22 +84,38 @@ __global__ void __launch_bounds__(128) k_dot_ref_chunks(const q128 *__restrict__
     __syncthreads();
   }
   if (threadIdx.x != 0) return;
-  if (pair && len) {
-    q128 a = second, b = q_one();
-#pragma unroll 1
-    for (int op = 0; op < 1 + (int)(len & 1); ++op) {
-      cacc acc;
-      cacc_set(acc, r);
-      chain_fma(acc, a, b);
-      r = cacc_get(acc);
-      a = ld(x + e - 1);
-      b = ld(y + e - 1);
-    }
-  }
+  if (pair && len) r = dot_pair_end(r, second, x, y, e, (int)(len & 1));
   if (T == 1)
     st(out, direct ? r : add_packed(q_zero(0), r));
   else
     st(part + t, r);
+}
+// Long chunks: a workgroup per chain (group_chain), whose values k_dot_ref_group_sum puts together.  2048 steps
+// take 5 us of VALU issue and barriers and about 60 cycles more for each climb or tie.  2^20 elements, T = 16:
+// 0.29 ms (0.94 ms with a wave per chain; log-uniform 0.16 ms, 0.78 ms).
+__global__ void __launch_bounds__(64 * SG_WAVES) k_dot_ref_group(const q128 *__restrict__ x, int64_t incx,
+                                                                 const q128 *__restrict__ y, int64_t incy, int64_t n,
+                                                                 int T, int pair, q128 *__restrict__ part) {
+  __shared__ sg_lds lds;
+  const int t = (int)blockIdx.x >> pair, p = (int)blockIdx.x & pair;
+  int64_t s, e;
+  chunk_range(n, T, t, s, e);
+  const int64_t step = 1 + pair;
+  const q128 r = group_chain(q_zero(0), sc_strided{x + (s + p) * incx, step * incx},
+                             sc_strided{y + (s + p) * incy, step * incy}, (e - s) / step, lds);
+  if (threadIdx.x == 0) st(part + blockIdx.x, r);
+}
+__global__ void __launch_bounds__(64) k_dot_ref_group_sum(const q128 *__restrict__ x, const q128 *__restrict__ y,
+                                                          int64_t n, int T, int pair, q128 *__restrict__ part,
+                                                          q128 *__restrict__ out) {
+  for (int t = threadIdx.x; pair && t < T; t += 64) {
+    int64_t s, e;
+    chunk_range(n, T, t, s, e);
+    st(part + 2 * t, dot_pair_end(ld(part + 2 * t), ld(part + 2 * t + 1), x, y, e, (int)((e - s) & 1)));
+  }
+  __syncthreads();
+  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1 + pair}, sc_const{q_one()}, T);
+  if (threadIdx.x == 0) st(out, r);
 }
 // the chunks' values summed from +0 in chunk order (level1.hpp:67-71, :117-120): one more chain
 __global__ void __launch_bounds__(64) k_dot_ref_sum(int T, const q128 *__restrict__ part, q128 *__restrict__ out) {
@@ -301,6 +332,11 @@ __global__ void k_fill_2d(int kind, uint64_t seed, int64_t rows, int64_t cols, i
 // launchers
 // ------------------------------------------------------------------------------------------
 
+// Whether a dot's chains get a workgroup each instead of a wave (a workgroup's registers take a CU).  Measured,
+// us (workgroup, wave): 32 chains of 512 41, 32; 1024 47, 56; 4096 60, 160; 32768 288, 949; 256 chains of 512
+// 52, 43; 1024 54, 60 (48, 45 log-uniform); 1536 70, 83 (53, 57); 4096 95, 164.
+static bool group_chains(int64_t chains, int64_t len) { return chains <= 256 && len >= 1280; }
+
 hipError_t launch_dot_ref(const q128 *x, int64_t incx, const q128 *y, int64_t incy, int64_t n, int T,
                           q128 *part, q128 *out, hipStream_t st) {
   const int contiguous = (incx == 1 && incy == 1);
@@ -308,6 +344,12 @@ hipError_t launch_dot_ref(const q128 *x, int64_t incx, const q128 *y, int64_t in
   if (n < 500) {  // level1.hpp:40-43 (contiguous) and :128-134 (strided): one chain set, no sum
     Teff = 1;
     direct = 1;
+  }
+  if (group_chains(Teff << contiguous, (n / Teff) >> contiguous)) {
+    hipLaunchKernelGGL(k_dot_ref_group, dim3((unsigned)(Teff << contiguous)), dim3(64 * SG_WAVES), 0, st, x, incx, y,
+                       incy, n, Teff, contiguous, part);
+    hipLaunchKernelGGL(k_dot_ref_group_sum, dim3(1), dim3(64), 0, st, x, y, n, Teff, contiguous, part, out);
+    return hipGetLastError();
   }
   hipLaunchKernelGGL(k_dot_ref_chunks, dim3(Teff), dim3(contiguous ? 128 : 64), 0, st, x, incx, y, incy, n, Teff, direct,
                      part, out);

@@ -58,6 +58,14 @@ def test_dot(O, Q, cuda, kind, n, inc, T):
     assert np.array_equal(plain(from_dev(out)), plain(O.to_pair(O.dot(n, x, inc, y, inc, T))))
 
 
+# chains of a workgroup each: 1280 steps are the fewest, 2048 are done at a time; 256 chains are the most
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n,inc,T", [(1279, 2, 1), (1280, 2, 1), (2112, 3, 1), (2113, 2, 1), (2560, 1, 1), (4225, 1, 1), (8323, 1, 2), (21503, 2, 5),
+                                     (66000, 1, 3), (327685, 1, 128), (327697, 2, 256)])
+def test_dot_workgroup_per_chain(O, Q, cuda, kind, n, inc, T):
+    test_dot(O, Q, cuda, kind, n, inc, T)
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("layout,m,n,incx", [(0, 3, 129, 1), (0, 5, 64, 2), (0, 7, 1001, 1), (1, 9, 65, 1), (1, 17, 1000, 2), (1, 8, 63, 1)])
 def test_gemv(O, Q, cuda, kind, layout, m, n, incx):
