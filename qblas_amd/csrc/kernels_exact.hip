@@ -6,6 +6,7 @@
 //   k_dot_exact_partial    grid-stride lanes, block-uniform window anchor, products into lazy LDS
 //                          digits (exact_dev.hpp), wave and block reductions into one lo/hi window
 //                          pair per block.
+//   k_dot_exact_small      a short dot whole, in one workgroup.
 //   k_exact_dot_combine    sums the block partials on a common base in registers (column sums per
 //                          workgroup); the last workgroup ripples the carries once and rounds.
 //   k_vec_split            the gemv vector prepared once: 29-bit limbs and a tag per element.
@@ -29,18 +30,20 @@ namespace qbk {
 // ------------------------------------------------------------------------------------------
 constexpr int XD_BS = 256;
 
-__global__ void __launch_bounds__(XD_BS) k_dot_exact_partial(const q128 *__restrict__ x, int64_t incx,
-                                                             const q128 *__restrict__ y, int64_t incy, int64_t n,
-                                                             part_t *__restrict__ parts, uint32_t *__restrict__ hdr) {
-  __shared__ int s_mn[XD_BS / 64], s_mx[XD_BS / 64];
-  __shared__ uint32_t s_fl[XD_BS / 64];
-  __shared__ unsigned long long s_dig[XD_BS / 64][DIG][64];
+// The block's share of the products: its digits in s_dig[0][k][0] and its flags, for thread 0; returns the
+// anchor to every thread.  Every thread of BS calls.
+template <int BS>
+__device__ __forceinline__ int dot_exact_block(const q128 *__restrict__ x, int64_t incx, const q128 *__restrict__ y,
+                                               int64_t incy, int64_t n, uint32_t *__restrict__ hdr,
+                                               unsigned long long (&s_dig)[BS / 64][DIG][64], uint32_t &flags) {
+  __shared__ int s_mn[BS / 64], s_mx[BS / 64];
+  __shared__ uint32_t s_fl[BS / 64];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (blockIdx.x == 0 && threadIdx.x < 4) hdr[threadIdx.x] = 0;  // status, counts, ticket of the combine
   unsigned long long *d = &s_dig[wv][0][lane];
   dig_clear(d);
-  const int64_t stride = (int64_t)gridDim.x * XD_BS;
-  const int64_t i0 = (int64_t)blockIdx.x * XD_BS + threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * BS;
+  const int64_t i0 = (int64_t)blockIdx.x * BS + threadIdx.x;
   // the first two element pairs are loaded before the anchor is known (they set it) and are the
   // first ones accumulated
   const q128 zq = q_zero(0);
@@ -57,12 +60,12 @@ __global__ void __launch_bounds__(XD_BS) k_dot_exact_partial(const q128 *__restr
   __syncthreads();
   int bmn = s_mn[0], bmx = s_mx[0];
 #pragma unroll
-  for (int w = 1; w < XD_BS / 64; ++w) {
+  for (int w = 1; w < BS / 64; ++w) {
     bmn = min(bmn, s_mn[w]);
     bmx = max(bmx, s_mx[w]);
   }
   const int A = (bmn == EXP_NONE) ? 0 : ((bmn + bmx) >> 1) - WIN2_CENTER;
-  uint32_t flags = 0;
+  flags = 0;
   if (h0) dig_accumulate(d, A, a0, b0, flags);
   if (h1) dig_accumulate(d, A, a1, b1, flags);
   int64_t i = i0 + 2 * stride;
@@ -78,11 +81,11 @@ __global__ void __launch_bounds__(XD_BS) k_dot_exact_partial(const q128 *__restr
   } else {
     for (; i < n; i += stride) dig_accumulate(d, A, ldq_nt(x + i * incx), ldq_nt(y + i * incy), flags);
   }
-  // block reduction in the digit domain: digit k of the block is the int64 sum of the 256 lanes'
-  // digit k (each lane's digit takes < 2^29 + 1 per product: no overflow for any practical n);
-  // DP threads per digit each add 256 / DP of them, then a shuffle reduction over the DP threads
-  constexpr int DP = 8;
-  static_assert(DIG * DP <= XD_BS && 64 % DP == 0, "digit sums: DP threads per digit within one wave");
+  // block reduction in the digit domain: digit k of the block is the int64 sum of the lanes' digit
+  // k (each lane's digit takes < 2^29 + 1 per product: no overflow for any practical n);
+  // DP threads per digit each add BS / DP of them, then a shuffle reduction over the DP threads
+  constexpr int DP = BS / 32;
+  static_assert(DIG * DP <= BS && 64 % DP == 0, "digit sums: DP threads per digit within one wave");
   flags = wave_or(flags);
   if (lane == 0) s_fl[wv] = flags;
   __syncthreads();  // every lane's digits are final
@@ -90,7 +93,7 @@ __global__ void __launch_bounds__(XD_BS) k_dot_exact_partial(const q128 *__restr
     const int k = threadIdx.x / DP, q = threadIdx.x % DP;
     int64_t sum = 0;
 #pragma unroll
-    for (int w = 0; w < XD_BS / 64; ++w) {
+    for (int w = 0; w < BS / 64; ++w) {
 #pragma unroll
       for (int j = 0; j < 64 / DP; ++j) sum += (int64_t)s_dig[w][k][q + DP * j];
     }
@@ -99,17 +102,53 @@ __global__ void __launch_bounds__(XD_BS) k_dot_exact_partial(const q128 *__restr
     if (q == 0) s_dig[0][k][0] = (unsigned long long)sum;  // only this thread reads that slot
   }
   __syncthreads();
+#pragma unroll
+  for (int w = 0; w < BS / 64; ++w) flags |= s_fl[w];
+  return A;
+}
+
+__global__ void __launch_bounds__(XD_BS) k_dot_exact_partial(const q128 *__restrict__ x, int64_t incx,
+                                                             const q128 *__restrict__ y, int64_t incy, int64_t n,
+                                                             part_t *__restrict__ parts, uint32_t *__restrict__ hdr) {
+  __shared__ unsigned long long s_dig[XD_BS / 64][DIG][64];
+  uint32_t flags;
+  const int A = dot_exact_block<XD_BS>(x, incx, y, incy, n, hdr, s_dig, flags);
   if (threadIdx.x == 0) {
     uint32_t Wl[WW], Wh[WW];
     dig_to_windows(&s_dig[0][0][0], Wl, Wh);
-#pragma unroll
-    for (int w = 1; w < XD_BS / 64; ++w) flags |= s_fl[w];
     // a zero window is marked by the anchor EXP_NONE, so the combine reads 8 bytes per record
     // to find the range of the nonzero ones
     part_t *p = parts + 2 * (int64_t)blockIdx.x;
     put_parts(p, A, flags, Wl, Wh);
     if (win_is_zero(Wl)) p[0].A = EXP_NONE;
     if (win_is_zero(Wh)) p[1].A = EXP_NONE;
+  }
+}
+
+// A short dot in one launch of one workgroup, which rounds its digits itself: n = 1001 takes 6.9 us a call,
+// 12.8 with the partial and combine kernels, whose time is two launches' latency.
+constexpr int XS_BS = 512;
+constexpr int64_t XS_MAX = 2048;  // 4 products a lane; above it the partial kernel has more than one block
+__global__ void __launch_bounds__(XS_BS) k_dot_exact_small(const q128 *__restrict__ x, int64_t incx,
+                                                           const q128 *__restrict__ y, int64_t incy, int64_t n,
+                                                           q128 *__restrict__ out, uint32_t *__restrict__ hdr) {
+  __shared__ unsigned long long s_dig[XS_BS / 64][DIG][64];
+  __shared__ kul_t K;
+  uint32_t flags;
+  const int A = dot_exact_block<XS_BS>(x, incx, y, incy, n, hdr, s_dig, flags);
+  if (flags & FL_LOST) {  // the same in every thread
+    kul_clear_all(K);
+    __syncthreads();
+    const q128 r = wide_item(K, n, x, incx, y, incy, false, q_one(), q_zero(0), q_zero(0), hdr);
+    if (threadIdx.x == 0) {
+      stq_c(out, r);
+      hdr[2] = 1;
+    }
+  } else if (threadIdx.x == 0) {
+    uint32_t Wl[WW], Wh[WW], M[SW], sign;
+    dig_to_windows(&s_dig[0][0][0], Wl, Wh);
+    s_from_windows(M, sign, Wl, Wh);
+    stq_c(out, finish_reg(M, A, sign, 0u, flags, false, q_one(), q_zero(0), q_zero(0)));
   }
 }
 
@@ -693,6 +732,10 @@ size_t gemv_exact_ws(int colmajor, int64_t m, int64_t n) {
 hipError_t launch_dot_exact(const q128 *x, int64_t incx, const q128 *y, int64_t incy, int64_t n, void *ws,
                             q128 *out, hipStream_t st) {
   uint32_t *hdr = (uint32_t *)ws;
+  if (n <= XS_MAX) {
+    hipLaunchKernelGGL(k_dot_exact_small, dim3(1), dim3(XS_BS), 0, st, x, incx, y, incy, n, out, hdr);
+    return hipGetLastError();
+  }
   const int blocks = dot_exact_blocks(n);
   part_t *parts = (part_t *)((char *)ws + 256);
   col_rec *recs = (col_rec *)(parts + 2 * blocks);
