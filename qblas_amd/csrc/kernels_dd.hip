@@ -85,7 +85,7 @@ constexpr int DOT_BS = 256;
 
 __global__ void __launch_bounds__(DOT_BS) k_dot_dd_partial(const q128 *__restrict__ x, int64_t incx,
                                                            const q128 *__restrict__ y, int64_t incy, int64_t n,
-                                                           dd *__restrict__ part) {
+                                                           dd *__restrict__ part, q128 *__restrict__ out) {
   const int64_t stride = (int64_t)gridDim.x * DOT_BS;
   int64_t i = (int64_t)blockIdx.x * DOT_BS + threadIdx.x;
   dd acc0 = dd_zero(), acc1 = dd_zero();
@@ -100,7 +100,9 @@ __global__ void __launch_bounds__(DOT_BS) k_dot_dd_partial(const q128 *__restric
     for (; i < n; i += stride) acc0 = dd_fma(q_to_dd(ldq(x + i * incx)), q_to_dd(ldq(y + i * incy)), acc0);
   }
   const dd s = block_sum_dd<DOT_BS>(dd_add(acc0, acc1));
-  if (threadIdx.x == 0) st_dd(part + blockIdx.x, s);
+  if (threadIdx.x != 0) return;
+  if (out) stq(out, dd_to_q(s));
+  else st_dd(part + blockIdx.x, s);
 }
 
 __global__ void __launch_bounds__(256) k_dot_dd_final(const dd *__restrict__ part, int nparts,
@@ -351,7 +353,10 @@ hipError_t launch_dot_dd(const q128 *x, int64_t incx, const q128 *y, int64_t inc
                          hipStream_t st) {
   const int blocks = dot_dd_blocks(n);
   dd *part = (dd *)ws;
-  hipLaunchKernelGGL(k_dot_dd_partial, dim3(blocks), dim3(DOT_BS), 0, st, x, incx, y, incy, n, part);
+  // one block's sum is the result (the final kernel would add zeros to it): one launch, not two
+  hipLaunchKernelGGL(k_dot_dd_partial, dim3(blocks), dim3(DOT_BS), 0, st, x, incx, y, incy, n, part,
+                     blocks == 1 ? out : nullptr);
+  if (blocks == 1) return hipGetLastError();
   hipLaunchKernelGGL(k_dot_dd_final, dim3(1), dim3(256), 0, st, part, blocks, out);
   return hipGetLastError();
 }

@@ -686,51 +686,64 @@ __global__ void __launch_bounds__(256) k_oz_finish(int64_t M, int64_t N, int S, 
 // 5. exact repair of the queued entries
 // ------------------------------------------------------------------------------------------
 // One workgroup per queued entry (grid-stride over the queue): exact accumulation of
-// sum_l A_il B_lj in two windows per lane with a block-uniform anchor placing the largest
-// possible product (from the row and column maxima) at the top of the high window, then the
-// exact alpha*S + beta*C rounded once.  An entry with a product below the low window is
-// recomputed on the full-range path by the same workgroup.
+// sum_l A_il B_lj in each lane's LDS digits (exact_dev.hpp) with an anchor placing the largest
+// possible product (from the row and column maxima) at the top of their range, then the exact
+// alpha*S + beta*C rounded once.  An entry with a product below the range is recomputed on the
+// full-range path.  Bound by VALU issue, about 125 instructions a product; the rounding, 1400
+// instructions of one lane, waits until the workgroup has summed up to OZR_SLOTS entries and is
+// done for all of them at once, one a lane.  4096^3 log-uniform with 33817 queued entries: 0.51 ms
+// (1.2 ms with two register windows a lane, summed over the lanes and rounded entry by entry).
 constexpr int OZR_BS = 256;
 
-// Exact sum_l A_il B_lj by one workgroup: two windows per lane (anchor An), wave and block
-// reductions; thread 0 returns with the block's windows and flags.
+constexpr int OZR_SLOTS = 64;  // the lanes of the wave that rounds
+struct ozr_lds {
+  unsigned long long dig[OZR_BS / 64][DIG][64];
+  unsigned long long slot[DIG][OZR_SLOTS];  // digit sums of the entries
+  uint32_t flags[OZR_SLOTS];
+};
+static_assert(OZR_SLOTS == 64, "slots are digits of stride 64");
+
+// every thread, before the slots are used again
+__device__ __forceinline__ void oz_clear_slots(ozr_lds &lds) {
+  __syncthreads();  // the slots are read
+  if (threadIdx.x < OZR_SLOTS) lds.flags[threadIdx.x] = 0;
+  __syncthreads();
+}
+// Exact sum_l A_il B_lj by the workgroup into slot u (digits of anchor An); every thread calls, and the
+// slot is complete for all of them on return.
 __device__ __forceinline__ void oz_block_dot(int64_t K, const q128 *__restrict__ ar, int64_t asc,
-                                             const q128 *__restrict__ bc, int64_t bsr, int An, uint32_t (&Wl)[WW],
-                                             uint32_t (&Wh)[WW], uint32_t &flags, uint32_t (*s_w)[2 * WW + 1]) {
+                                             const q128 *__restrict__ bc, int64_t bsr, int An, int u, ozr_lds &lds) {
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-  for (int k = 0; k < WW; ++k) {
-    Wl[k] = 0;
-    Wh[k] = 0;
+  unsigned long long *d = &lds.dig[wv][0][lane];
+  dig_clear(d);
+  uint32_t flags = 0;
+  int64_t l = threadIdx.x;
+  for (; l + OZR_BS < K; l += 2 * OZR_BS) {  // two pairs in flight
+    const q128 a0 = ldq_c(ar + l * asc), b0 = ldq_c(bc + l * bsr);
+    const q128 a1 = ldq_c(ar + (l + OZR_BS) * asc), b1 = ldq_c(bc + (l + OZR_BS) * bsr);
+    dig_accumulate(d, An, a0, b0, flags);
+    dig_accumulate(d, An, a1, b1, flags);
   }
-  flags = 0;
-  for (int64_t l = threadIdx.x; l < K; l += OZR_BS) accumulate(Wl, Wh, An, ldq_c(ar + l * asc), ldq_c(bc + l * bsr), flags);
-  wave_sum_win(Wl);
-  wave_sum_win(Wh);
-  flags = wave_or(flags);
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < WW; ++k) {
-      s_w[wv][k] = Wl[k];
-      s_w[wv][WW + k] = Wh[k];
-    }
-    s_w[wv][2 * WW] = flags;
+  if (l < K) dig_accumulate(d, An, ldq_c(ar + l * asc), ldq_c(bc + l * bsr), flags);
+  if (__ballot(flags != 0)) {
+    flags = wave_or(flags);
+    if (lane == 0) atomicOr(&lds.flags[u], flags);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  constexpr int DP = 8;  // threads per digit
+  static_assert(DIG * DP <= OZR_BS && 64 % DP == 0, "digit sums: DP threads per digit within one wave");
+  if (threadIdx.x < DIG * DP) {
+    const int k = threadIdx.x / DP, q = threadIdx.x % DP;
+    int64_t sum = 0;
 #pragma unroll
-    for (int w = 1; w < OZR_BS / 64; ++w) {
-      uint32_t X[WW], Y[WW];
+    for (int w = 0; w < OZR_BS / 64; ++w)
 #pragma unroll
-      for (int k = 0; k < WW; ++k) {
-        X[k] = s_w[w][k];
-        Y[k] = s_w[w][WW + k];
-      }
-      win_add_win(Wl, X);
-      win_add_win(Wh, Y);
-      flags |= s_w[w][2 * WW];
-    }
+      for (int j = 0; j < 64 / DP; ++j) sum += (int64_t)lds.dig[w][k][q + DP * j];
+#pragma unroll
+    for (int m = 1; m < DP; m <<= 1) sum += __shfl_xor(sum, m);
+    if (q == 0) lds.slot[k][u] = (unsigned long long)sum;
   }
+  __syncthreads();
 }
 
 // window anchor placing the largest possible product (from the row and column maxima) at the top
@@ -739,26 +752,21 @@ __device__ __forceinline__ int oz_anchor(int ei, int ej) {
   return (ei == OZ_EZERO || ej == OZ_EZERO) ? 0 : ei + ej - 224 - (WIN_BAND + WIN_OMAX);
 }
 
-// One entry by the whole workgroup: *cp = RN(alpha sum_l ar[l asc] bc[l bsr] + beta *cp).  An entry
-// with a product outside the windows of anchor An is left unwritten: its queue index e goes to
-// the full-range queue wq (header word 2 counts it) for k_oz_wide / k_bo_wide.
-__device__ __forceinline__ void oz_repair_entry(int64_t K, const q128 *__restrict__ ar, int64_t asc,
-                                                const q128 *__restrict__ bc, int64_t bsr, int An, q128 alpha,
-                                                q128 beta, q128 *__restrict__ cp, uint32_t *__restrict__ hdr,
-                                                uint32_t (*s_w)[2 * WW + 1], uint32_t e, uint32_t *__restrict__ wq) {
-  uint32_t Wl[WW], Wh[WW], flags;
-  oz_block_dot(K, ar, asc, bc, bsr, An, Wl, Wh, flags, s_w);
-  if (threadIdx.x == 0) {
-    if (flags & FL_LOST) {
-      wq[atomicAdd(hdr + 2, 1u)] = e;
-    } else {
-      uint32_t Mw[SW];
-      uint32_t sign;
-      s_from_windows(Mw, sign, Wl, Wh);
-      stq_c(cp, finish_reg(Mw, An, sign, 0u, flags, true, alpha, beta, ldq_c(cp)));
-    }
+// One thread: *cp = RN(alpha S + beta *cp) of the sum in slot u.  An entry with a product outside the
+// digits of anchor An is left unwritten: its queue index e goes to the full-range queue wq (header
+// word 2 counts it) for k_oz_wide / k_bo_wide.
+__device__ __forceinline__ void oz_repair_round(const ozr_lds &lds, int u, int An, q128 alpha, q128 beta,
+                                                q128 *__restrict__ cp, uint32_t *__restrict__ hdr, uint32_t e,
+                                                uint32_t *__restrict__ wq) {
+  const uint32_t flags = lds.flags[u];
+  if (flags & FL_LOST) {
+    wq[atomicAdd(hdr + 2, 1u)] = e;
+    return;
   }
-  __syncthreads();
+  uint32_t Wl[WW], Wh[WW], Mw[SW], sign;
+  dig_to_windows(&lds.slot[0][u], Wl, Wh);
+  s_from_windows(Mw, sign, Wl, Wh);
+  stq_c(cp, finish_reg(Mw, An, sign, 0u, flags, true, alpha, beta, ldq_c(cp)));
 }
 
 // Queued entries at least this many: B's strided columns are read from a transposed copy (one pass
@@ -774,15 +782,23 @@ __global__ void __launch_bounds__(OZR_BS) k_oz_repair(int64_t K, const q128 *__r
                                                       q128 *__restrict__ C, int64_t csr, int64_t csc,
                                                       uint32_t *__restrict__ hdr, const uint32_t *__restrict__ list,
                                                       uint32_t *__restrict__ wq) {
-  __shared__ uint32_t s_w[OZR_BS / 64][2 * WW + 1];
+  __shared__ ozr_lds lds;
   const uint32_t count = hdr[1];
   const bool useT = Bt != nullptr && count >= OZ_REPAIR_TRANSPOSE;
   const q128 *Br = useT ? Bt : B;
   const int64_t rbsr = useT ? 1 : bsr, rbsc = useT ? K : bsc;
-  for (uint32_t e = blockIdx.x; e < count; e += gridDim.x) {
-    const int64_t i = list[2 * (int64_t)e], j = list[2 * (int64_t)e + 1];
-    oz_repair_entry(K, A + i * asr, asc, Br + j * rbsc, rbsr, oz_anchor(eA[i], eB[j]), alpha, beta,
-                    C + i * csr + j * csc, hdr, s_w, e, wq);
+  for (uint64_t e0 = blockIdx.x; e0 < count; e0 += (uint64_t)OZR_SLOTS * gridDim.x) {
+    oz_clear_slots(lds);
+    int used = 0;
+    for (uint64_t e = e0; used < OZR_SLOTS && e < count; e += gridDim.x, ++used) {
+      const int64_t i = list[2 * (int64_t)e], j = list[2 * (int64_t)e + 1];
+      oz_block_dot(K, A + i * asr, asc, Br + j * rbsc, rbsr, oz_anchor(eA[i], eB[j]), used, lds);
+    }
+    if ((int)threadIdx.x < used) {
+      const uint64_t e = e0 + (uint64_t)threadIdx.x * gridDim.x;
+      const int64_t i = list[2 * (int64_t)e], j = list[2 * (int64_t)e + 1];
+      oz_repair_round(lds, threadIdx.x, oz_anchor(eA[i], eB[j]), alpha, beta, C + i * csr + j * csc, hdr, (uint32_t)e, wq);
+    }
   }
 }
 
@@ -825,7 +841,7 @@ __global__ void __launch_bounds__(OZR_BS) k_oz_probe(int64_t M, int64_t N, int64
                                                      int64_t asr, int64_t asc, const q128 *__restrict__ B,
                                                      int64_t bsr, int64_t bsc, const int32_t *__restrict__ eA,
                                                      const int32_t *__restrict__ eB, int P, int *__restrict__ out) {
-  __shared__ uint32_t s_w[OZR_BS / 64][2 * WW + 1];
+  __shared__ ozr_lds lds;
   for (int e = blockIdx.x; e < P; e += gridDim.x) {
     // splitmix64 of the sample number picks (i, j)
     uint64_t z = 0x5eed0000ull + (uint64_t)(e + 1) * 0x9e3779b97f4a7c15ull;
@@ -839,20 +855,19 @@ __global__ void __launch_bounds__(OZR_BS) k_oz_probe(int64_t M, int64_t N, int64
       continue;
     }
     const int An = oz_anchor(ei, ej);
-    uint32_t Wl[WW], Wh[WW], flags;
-    oz_block_dot(K, A + i * asr, asc, B + j * bsc, bsr, An, Wl, Wh, flags, s_w);
+    oz_clear_slots(lds);
+    oz_block_dot(K, A + i * asr, asc, B + j * bsc, bsr, An, 0, lds);
     if (threadIdx.x == 0) {
       int r = 0x7fffffff;
-      if (!(flags & (FL_LOST | FL_NAN | FL_PINF | FL_NINF))) {
-        uint32_t Mw[SW];
-        uint32_t sign;
+      if (!(lds.flags[0] & (FL_LOST | FL_NAN | FL_PINF | FL_NINF))) {
+        uint32_t Wl[WW], Wh[WW], Mw[SW], sign;
+        dig_to_windows(&lds.slot[0][0], Wl, Wh);
         s_from_windows(Mw, sign, Wl, Wh);
         const int msb = rmsb<SW>(Mw);
         if (msb >= 0) r = An + msb - (ei + 3) - (ej + 3);
       }
       out[e] = r;
     }
-    __syncthreads();
   }
 }
 
@@ -1401,16 +1416,28 @@ __global__ void __launch_bounds__(OZR_BS) k_bo_repair(const qblas_gemm_problem *
                                                       const int32_t *__restrict__ eA, const int32_t *__restrict__ eB,
                                                       uint32_t *__restrict__ hdr, const uint32_t *__restrict__ list,
                                                       uint32_t *__restrict__ wq) {
-  __shared__ uint32_t s_w[OZR_BS / 64][2 * WW + 1];
+  __shared__ ozr_lds lds;
   const uint32_t nq = hdr[1];
-  for (uint32_t e = blockIdx.x; e < nq; e += gridDim.x) {
-    const int64_t p = list[4 * (int64_t)e], i = list[4 * (int64_t)e + 1], j = list[4 * (int64_t)e + 2];
-    const qblas_gemm_problem &pr = P[p];
-    const bo_geom G = bo_geometry(pr, colmajor);
-    const int64_t *o = off + p * BO_F;
-    oz_repair_entry(G.k, (const q128 *)pr.A + i * G.asr, G.asc, (const q128 *)pr.B + j * G.bsc, G.bsr,
-                    oz_anchor(eA[o[BO_ROWS] + i], eB[o[BO_COLS] + j]), q_make(pr.alpha[0], pr.alpha[1]),
-                    q_make(pr.beta[0], pr.beta[1]), (q128 *)pr.C + i * G.csr + j * G.csc, hdr, s_w, e, wq);
+  for (uint64_t e0 = blockIdx.x; e0 < nq; e0 += (uint64_t)OZR_SLOTS * gridDim.x) {
+    oz_clear_slots(lds);
+    int used = 0;
+    for (uint64_t e = e0; used < OZR_SLOTS && e < nq; e += gridDim.x, ++used) {
+      const int64_t p = list[4 * (int64_t)e], i = list[4 * (int64_t)e + 1], j = list[4 * (int64_t)e + 2];
+      const qblas_gemm_problem &pr = P[p];
+      const bo_geom G = bo_geometry(pr, colmajor);
+      const int64_t *o = off + p * BO_F;
+      oz_block_dot(G.k, (const q128 *)pr.A + i * G.asr, G.asc, (const q128 *)pr.B + j * G.bsc, G.bsr,
+                   oz_anchor(eA[o[BO_ROWS] + i], eB[o[BO_COLS] + j]), used, lds);
+    }
+    if ((int)threadIdx.x < used) {
+      const uint64_t e = e0 + (uint64_t)threadIdx.x * gridDim.x;
+      const int64_t p = list[4 * (int64_t)e], i = list[4 * (int64_t)e + 1], j = list[4 * (int64_t)e + 2];
+      const qblas_gemm_problem &pr = P[p];
+      const bo_geom G = bo_geometry(pr, colmajor);
+      const int64_t *o = off + p * BO_F;
+      oz_repair_round(lds, threadIdx.x, oz_anchor(eA[o[BO_ROWS] + i], eB[o[BO_COLS] + j]), q_make(pr.alpha[0], pr.alpha[1]),
+                      q_make(pr.beta[0], pr.beta[1]), (q128 *)pr.C + i * G.csr + j * G.csc, hdr, (uint32_t)e, wq);
+    }
   }
 }
 
