@@ -104,7 +104,7 @@ __device__ __forceinline__ void put_parts(part_t *p, int A, uint32_t flags, cons
 // 64-bit digits at d[k * 64] (d = the wave's digit array + l), digit k weighing 2^(A + 29 k).  A
 // product with lsb offset o = e_p - A in [1, WIN_BAND + WIN_OMAX] (the band of the two register
 // windows, so the same products go to the full-range path) is formed at its offset within digit
-// w = o / 29: one significand shifted by r = o - 29 w is cut into five 29-bit limbs, the other
+// w = (o - 1) / 29: one significand shifted by r = o - 29 w is cut into five 29-bit limbs, the other
 // into four, and the column sums of the 20 limb products (each < 2^58, a column < 2^61 with its
 // carry in, one 64-bit multiply-add each) are cut into nine 29-bit digits that go to LDS digits
 // w .. w + 8 by 64-bit atomic adds -- no carries between LDS digits, no shifting network, no
@@ -126,48 +126,56 @@ __device__ __forceinline__ void dig_clear(unsigned long long *d) {
   for (int k = 0; k < DIG; ++k) d[k * 64] = 0;
 }
 
-// the product (-1)^s a.m b.m 2^(A + o) into the digits: b given as its four 29-bit limbs
+// the product (-1)^s a.m b.m 2^(A + o) into the digits: b given as its four 29-bit limbs.  All shifts are
+// 32-bit funnels, o / 29 a 24-bit product, and each column's carry the first addend of the next column's
+// multiply-adds (the empty asm keeps it there; reassociated, it costs an addition of its own): 8192^2
+// column-major gemv 235 us against 240 with 64-bit shifts and carries added afterwards.
 __device__ __forceinline__ void dig_core(unsigned long long *d, int o, uint64_t aml, uint64_t amh, uint32_t B0,
                                          uint32_t B1, uint32_t B2, uint32_t B3, uint32_t s) {
-  const uint32_t w = ((uint32_t)o * 565u) >> 14;  // o / 29 for 0 <= o < 300 (checked exhaustively)
-  const uint32_t r = (uint32_t)o - w * (uint32_t)DB;  // 0..28
-  // a.m << r (at most 141 bits) as five 29-bit limbs
-  const uint64_t lo = aml << r;
-  const uint64_t mid = (amh << r) | ((aml >> 1) >> (63u - r));
-  const uint64_t hi = (amh >> 1) >> (63u - r);
-  const uint32_t A0 = (uint32_t)lo & DMASK, A1 = (uint32_t)(lo >> 29) & DMASK,
-                 A2 = (uint32_t)((lo >> 58) | (mid << 6)) & DMASK, A3 = (uint32_t)(mid >> 23) & DMASK,
-                 A4 = (uint32_t)((mid >> 52) | (hi << 12)) & DMASK;
+  // (o - 1) / 29 for 1 <= o < 300 (checked exhaustively), so that r is 1..29 and no funnel shifts by 32
+  const uint32_t w = __umul24((uint32_t)o - 1u, 565u) >> 14;
+  const uint32_t r = (uint32_t)o - __umul24(w, (uint32_t)DB), f = 32u - r;
+  // a.m << r (at most 142 bits) as five 29-bit limbs: limb i holds bits 29 i - r .. of a.m, the funnel of the
+  // words of a.m that begin at bits 29 i and 29 i - 32
+  const uint32_t x0 = (uint32_t)aml, x1 = (uint32_t)(aml >> 32), x2 = (uint32_t)amh, x3 = (uint32_t)(amh >> 32);
+  const uint32_t A0 = (x0 << r) & DMASK, A1 = alignbit32(alignbit32(x1, x0, 29), x0 << 3, f) & DMASK,
+                 A2 = alignbit32(alignbit32(x2, x1, 26), alignbit32(x1, x0, 26), f) & DMASK,
+                 A3 = alignbit32(alignbit32(x3, x2, 23), alignbit32(x2, x1, 23), f) & DMASK,
+                 A4 = alignbit32(x3, x2, 20) >> f;
   uint32_t t[9];
   uint64_t acc = (uint64_t)A0 * B0;
   t[0] = (uint32_t)acc & DMASK;
-  acc = (acc >> 29) + (uint64_t)A1 * B0;
+#define QB_DIG_CARRY(x, y)           \
+  acc = (acc >> 29) + (uint64_t)x * y;  \
+  asm("" : "+v"(acc));
+  QB_DIG_CARRY(A1, B0)
   acc += (uint64_t)A0 * B1;
   t[1] = (uint32_t)acc & DMASK;
-  acc = (acc >> 29) + (uint64_t)A2 * B0;
+  QB_DIG_CARRY(A2, B0)
   acc += (uint64_t)A1 * B1;
   acc += (uint64_t)A0 * B2;
   t[2] = (uint32_t)acc & DMASK;
-  acc = (acc >> 29) + (uint64_t)A3 * B0;
+  QB_DIG_CARRY(A3, B0)
   acc += (uint64_t)A2 * B1;
   acc += (uint64_t)A1 * B2;
   acc += (uint64_t)A0 * B3;
   t[3] = (uint32_t)acc & DMASK;
-  acc = (acc >> 29) + (uint64_t)A4 * B0;
+  QB_DIG_CARRY(A4, B0)
   acc += (uint64_t)A3 * B1;
   acc += (uint64_t)A2 * B2;
   acc += (uint64_t)A1 * B3;
   t[4] = (uint32_t)acc & DMASK;
-  acc = (acc >> 29) + (uint64_t)A4 * B1;
+  QB_DIG_CARRY(A4, B1)
   acc += (uint64_t)A3 * B2;
   acc += (uint64_t)A2 * B3;
   t[5] = (uint32_t)acc & DMASK;
-  acc = (acc >> 29) + (uint64_t)A4 * B2;
+  QB_DIG_CARRY(A4, B2)
   acc += (uint64_t)A3 * B3;
   t[6] = (uint32_t)acc & DMASK;
-  acc = (acc >> 29) + (uint64_t)A4 * B3;
+  QB_DIG_CARRY(A4, B3)
   t[7] = (uint32_t)acc & DMASK;
-  t[8] = (uint32_t)(acc >> 29);  // < 2^22: the product is below 2^254
+  t[8] = (uint32_t)(acc >> 29);  // < 2^23: the product is below 2^255
+#undef QB_DIG_CARRY
   const uint32_t m = 0u - (s & 1u), m29 = m & DMASK;
   unsigned long long *q = d + w * 64;
   dig_add(q, (unsigned long long)((t[0] ^ m29) + (m & 1u)));
@@ -254,13 +262,14 @@ __device__ __forceinline__ void dig_accumulate(unsigned long long *d, int A, q12
 // This lane's digits as the two windows of anchor A: V = sum_k D_k 2^(29 k) with the carries
 // rippled once (two's complement over 32-bit words), split as V = Wl + Wh 2^WIN_BAND with
 // Wl = V mod 2^WIN_BAND.
+template <int STRIDE = 64>
 __device__ __forceinline__ void dig_to_windows(const unsigned long long *d, uint32_t (&Wl)[WW], uint32_t (&Wh)[WW]) {
   constexpr int VW = (DIG * DB + 31) / 32 + 1;  // 18 words
   uint32_t nd[DIG];
   int64_t carry = 0;
 #pragma unroll
   for (int k = 0; k < DIG; ++k) {
-    const int64_t s = (int64_t)d[k * 64] + carry;
+    const int64_t s = (int64_t)d[k * STRIDE] + carry;
     nd[k] = (uint32_t)s & DMASK;
     carry = s >> 29;  // arithmetic
   }

@@ -691,17 +691,17 @@ __global__ void __launch_bounds__(256) k_oz_finish(int64_t M, int64_t N, int S, 
 // alpha*S + beta*C rounded once.  An entry with a product below the range is recomputed on the
 // full-range path.  Bound by VALU issue, about 125 instructions a product; the rounding, 1400
 // instructions of one lane, waits until the workgroup has summed up to OZR_SLOTS entries and is
-// done for all of them at once, one a lane.  4096^3 log-uniform with 33817 queued entries: 0.51 ms
-// (1.2 ms with two register windows a lane, summed over the lanes and rounded entry by entry).
+// done for all of them at once, one a lane.  4096^3 log-uniform with 33817 queued entries: 0.65 ms
+// (1.2 ms with two register windows a lane, summed over the lanes and rounded entry by entry; 0.91 ms with two
+// pairs in flight and three workgroups a CU).
 constexpr int OZR_BS = 256;
 
-constexpr int OZR_SLOTS = 64;  // the lanes of the wave that rounds
+constexpr int OZR_SLOTS = 16;  // lanes that round; with more, LDS holds three workgroups a CU, not four
 struct ozr_lds {
   unsigned long long dig[OZR_BS / 64][DIG][64];
   unsigned long long slot[DIG][OZR_SLOTS];  // digit sums of the entries
   uint32_t flags[OZR_SLOTS];
 };
-static_assert(OZR_SLOTS == 64, "slots are digits of stride 64");
 
 // every thread, before the slots are used again
 __device__ __forceinline__ void oz_clear_slots(ozr_lds &lds) {
@@ -718,13 +718,30 @@ __device__ __forceinline__ void oz_block_dot(int64_t K, const q128 *__restrict__
   dig_clear(d);
   uint32_t flags = 0;
   int64_t l = threadIdx.x;
-  for (; l + OZR_BS < K; l += 2 * OZR_BS) {  // two pairs in flight
-    const q128 a0 = ldq_c(ar + l * asc), b0 = ldq_c(bc + l * bsr);
-    const q128 a1 = ldq_c(ar + (l + OZR_BS) * asc), b1 = ldq_c(bc + (l + OZR_BS) * bsr);
-    dig_accumulate(d, An, a0, b0, flags);
-    dig_accumulate(d, An, a1, b1, flags);
+  constexpr int U = 4;  // pairs in flight
+  q128 a[U], b[U];
+  for (; l + (U - 1) * OZR_BS < K; l += U * OZR_BS) {
+#pragma unroll
+    for (int v = 0; v < U; ++v) {
+      a[v] = ldq_c(ar + (l + v * OZR_BS) * asc);
+      b[v] = ldq_c(bc + (l + v * OZR_BS) * bsr);
+    }
+#pragma unroll
+    for (int v = 0; v < U; ++v) dig_accumulate(d, An, a[v], b[v], flags);
   }
-  if (l < K) dig_accumulate(d, An, ldq_c(ar + l * asc), ldq_c(bc + l * bsr), flags);
+#pragma unroll
+  for (int v = 0; v < U - 1; ++v) {
+    if (l + v * OZR_BS < K) {
+      a[v] = ldq_c(ar + (l + v * OZR_BS) * asc);
+      b[v] = ldq_c(bc + (l + v * OZR_BS) * bsr);
+    }
+  }
+#pragma unroll 1
+  for (int v = 0; v < U - 1 && l < K; ++v, l += OZR_BS) {
+    dig_accumulate(d, An, a[0], b[0], flags);
+    a[0] = a[1], b[0] = b[1];
+    a[1] = a[2], b[1] = b[2];
+  }
   if (__ballot(flags != 0)) {
     flags = wave_or(flags);
     if (lane == 0) atomicOr(&lds.flags[u], flags);
@@ -764,7 +781,7 @@ __device__ __forceinline__ void oz_repair_round(const ozr_lds &lds, int u, int A
     return;
   }
   uint32_t Wl[WW], Wh[WW], Mw[SW], sign;
-  dig_to_windows(&lds.slot[0][u], Wl, Wh);
+  dig_to_windows<OZR_SLOTS>(&lds.slot[0][u], Wl, Wh);
   s_from_windows(Mw, sign, Wl, Wh);
   stq_c(cp, finish_reg(Mw, An, sign, 0u, flags, true, alpha, beta, ldq_c(cp)));
 }
@@ -775,7 +792,7 @@ constexpr uint32_t OZ_REPAIR_TRANSPOSE = 2048;
 
 // Bt: null, or the transposed copy of B (N x K row-major) that k_oz_transpose writes when the queue
 // holds at least OZ_REPAIR_TRANSPOSE entries; the same count selects it here.
-__global__ void __launch_bounds__(OZR_BS) k_oz_repair(int64_t K, const q128 *__restrict__ A, int64_t asr, int64_t asc,
+__global__ void __launch_bounds__(OZR_BS, 4) k_oz_repair(int64_t K, const q128 *__restrict__ A, int64_t asr, int64_t asc,
                                                       const q128 *__restrict__ B, int64_t bsr, int64_t bsc,
                                                       const q128 *__restrict__ Bt, const int32_t *__restrict__ eA,
                                                       const int32_t *__restrict__ eB, q128 alpha, q128 beta,
@@ -861,7 +878,7 @@ __global__ void __launch_bounds__(OZR_BS) k_oz_probe(int64_t M, int64_t N, int64
       int r = 0x7fffffff;
       if (!(lds.flags[0] & (FL_LOST | FL_NAN | FL_PINF | FL_NINF))) {
         uint32_t Wl[WW], Wh[WW], Mw[SW], sign;
-        dig_to_windows(&lds.slot[0][0], Wl, Wh);
+        dig_to_windows<OZR_SLOTS>(&lds.slot[0][0], Wl, Wh);
         s_from_windows(Mw, sign, Wl, Wh);
         const int msb = rmsb<SW>(Mw);
         if (msb >= 0) r = An + msb - (ei + 3) - (ej + 3);
@@ -1411,7 +1428,7 @@ __global__ void __launch_bounds__(256) k_bo_finish(const qblas_gemm_problem *__r
 }
 
 // exact recomputation of the queued entries, one workgroup per entry (grid-stride)
-__global__ void __launch_bounds__(OZR_BS) k_bo_repair(const qblas_gemm_problem *__restrict__ P, int64_t count,
+__global__ void __launch_bounds__(OZR_BS, 4) k_bo_repair(const qblas_gemm_problem *__restrict__ P, int64_t count,
                                                       const int64_t *__restrict__ off, int colmajor,
                                                       const int32_t *__restrict__ eA, const int32_t *__restrict__ eB,
                                                       uint32_t *__restrict__ hdr, const uint32_t *__restrict__ list,
