@@ -125,10 +125,10 @@ __global__ void __launch_bounds__(XD_BS) k_dot_exact_partial(const q128 *__restr
   }
 }
 
-// A short dot in one launch of one workgroup, which rounds its digits itself: n = 1001 takes 6.9 us a call,
-// 12.8 with the partial and combine kernels, whose time is two launches' latency.
+// A short dot in one launch of one workgroup, which rounds its digits itself: n = 1001 takes 6.8 us a call, 4096 9.1;
+// 12.8 and 14.6 with the partial and combine kernels, whose time is two launches' latency.
 constexpr int XS_BS = 512;
-constexpr int64_t XS_MAX = 2048;  // 4 products a lane; above it the partial kernel has more than one block
+constexpr int64_t XS_MAX = 8192;  // 16 products a lane: 13.4 us, the two kernels 14.7
 __global__ void __launch_bounds__(XS_BS) k_dot_exact_small(const q128 *__restrict__ x, int64_t incx,
                                                            const q128 *__restrict__ y, int64_t incy, int64_t n,
                                                            q128 *__restrict__ out, uint32_t *__restrict__ hdr) {

@@ -1,5 +1,5 @@
-"""GPU: the EXACT dot that one workgroup finishes by itself (n <= 2048), and the first size above it, against
-the oracle's correctly rounded sum: fewer elements than the workgroup has lanes, one to four a lane, strides,
+"""GPU: the EXACT dot that one workgroup finishes by itself (n <= 8192), and the first size above it, against
+the oracle's correctly rounded sum: fewer elements than the workgroup has lanes, one to sixteen a lane, strides,
 exact cancellation, and products far apart (the full-range path)."""
 import numpy as np
 import pytest
@@ -26,7 +26,7 @@ def values(O, kind, seed, n):
 
 @pytest.mark.parametrize("kind", ("uniform", "log", "cancel", "zero", "far"))
 @pytest.mark.parametrize("n,incx,incy", [(1, 1, 1), (65, 1, 1), (511, 1, 1), (512, 1, 1), (513, 2, 1), (1001, 1, 1), (1025, 1, 3),
-                                         (1537, 1, 1), (2048, 1, 1), (2049, 1, 1)])
+                                         (1537, 1, 1), (2048, 1, 1), (2049, 2, 1), (8191, 1, 1), (8192, 1, 2), (8193, 1, 1)])
 def test_dot_exact_small(O, Q, cuda, n, incx, incy, kind):
     print(f"dot exact {kind} n={n} incx={incx} incy={incy}", flush=True)
     u, v = values(O, kind, 71 + n, n)
@@ -40,7 +40,7 @@ def test_dot_exact_small(O, Q, cuda, n, incx, incy, kind):
         assert pair(from_dev(out)[0]) == O.exact_dot(u, v)[0]
 
 
-@pytest.mark.parametrize("n", (3, 600, 2048))
+@pytest.mark.parametrize("n", (3, 600, 8192))
 def test_dot_exact_small_specials(O, Q, cuda, n):
     print(f"dot exact specials n={n}", flush=True)
     inf = (0, 0x7FFF << 48)
