@@ -223,15 +223,19 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
 // part == null: the workgroup takes all blocks of k.  Else it takes block kb0 + blockIdx.z and writes its t to
 // part[(blockIdx.z n + j) m + i], for k_gemm_ref_fold: the blocks' chains do not depend on each other,
 // so a C of few tiles still fills the chip: 500 x 333 x 700 427 us against 561, 64 x 64 x 2000 68 us
-// against 874 (both with the step of 105 instructions; now 340 us and 72 us).
-constexpr int GR_KT = 32;
+// against 874 (both with the step of 105 instructions; now 329 us and 72 us).
+// KT: values of k staged at a time, 1 KB of LDS each.  32 let five workgroups share a CU, 16 eight: with more
+// workgroups than five a CU 16 is faster (1000^3 2734 us against 2850, 500 x 333 x 700 363 against 377), with
+// fewer the barriers cost more than there is to overlap them with (100 x 100 x 900 78 us against 75).
+constexpr int64_t GR_FIVE = 5 * 256;
+template <int KT>
 __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_t kc,
                                                   q128 alpha, const q128 *__restrict__ A, int64_t lda,
                                                   const q128 *__restrict__ B, int64_t ldb, q128 beta,
                                                   q128 *__restrict__ C, int64_t ldc, int64_t kb0,
                                                   q128 *__restrict__ part) {
-  __shared__ __attribute__((aligned(16))) cop sA[GR_KT * 16];
-  __shared__ __attribute__((aligned(16))) cop sB[GR_KT * 16];
+  __shared__ __attribute__((aligned(16))) cop sA[KT * 16];
+  __shared__ __attribute__((aligned(16))) cop sB[KT * 16];
   const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
   const int64_t i0 = (int64_t)blockIdx.y * 16, j0 = (int64_t)blockIdx.x * 16;
   const int64_t i = i0 + ti, j = j0 + tj;
@@ -242,7 +246,7 @@ __global__ void __launch_bounds__(256) k_gemm_ref(int colmajor, int64_t m, int64
   if (!part) cacc_set(c, live ? chain_mul(beta, ld(ci)) : q_zero(0));
   for (int64_t kk = k0; kk < k1; kk += kc) {
     const int64_t ke = (kk + kc < k1) ? kk + kc : k1;
-    const q128 t = tile_chain<16, 16, GR_KT>(colmajor, m, n, A, lda, B, ldb, i0, j0, kk, ke, sA, sB);
+    const q128 t = tile_chain<16, 16, KT>(colmajor, m, n, A, lda, B, ldb, i0, j0, kk, ke, sA, sB);
     if (live) {
       if (!part) chain_fma(c, alpha, t);
       else st(part + ((int64_t)blockIdx.z * n + j) * m + i, t);
@@ -395,7 +399,7 @@ hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const
 }
 
 // Workspace for splitting the blocks of k over workgroups (0: not split): a workgroup of four waves is
-// a tile, and the chip takes 5 of them per CU at a time (LDS), so below about 2048 tiles it is idle in
+// a tile, and the chip takes 5 or 8 of them per CU at a time (LDS), so below about 2048 tiles it is idle in
 // part or for the last wave.  Rounds of at most 64 MB of t.
 size_t gemm_ref_ws(int64_t m, int64_t n, int64_t k, int64_t kc) {
   const int64_t nb = (k + kc - 1) / kc, tm = (m + 15) / 16, tn = (n + 15) / 16;
@@ -409,15 +413,18 @@ hipError_t launch_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_
                            hipStream_t st) {
   if (!grid_fits((n + 15) / 16, 256)) return hipErrorInvalidValue;
   const unsigned tn = (unsigned)((n + 15) / 16), tm = (unsigned)((m + 15) / 16);
+  const int64_t tiles = (int64_t)tn * tm;
   if (!part) {
-    hipLaunchKernelGGL(k_gemm_ref, dim3(tn, tm), dim3(256), 0, st, colmajor, m, n, k, kc, alpha, A, lda, B, ldb, beta,
+    const auto f = tiles > GR_FIVE ? k_gemm_ref<16> : k_gemm_ref<32>;
+    hipLaunchKernelGGL(f, dim3(tn, tm), dim3(256), 0, st, colmajor, m, n, k, kc, alpha, A, lda, B, ldb, beta,
                        C, ldc, (int64_t)0, part);
     return hipGetLastError();
   }
   const int64_t nb = (k + kc - 1) / kc, zb = (int64_t)(gemm_ref_ws(m, n, k, kc) / (size_t)(16 * m * n));
   for (int64_t z = 0; z < nb; z += zb) {
     const int64_t c = nb - z < zb ? nb - z : zb;
-    hipLaunchKernelGGL(k_gemm_ref, dim3(tn, tm, (unsigned)c), dim3(256), 0, st, colmajor, m, n, k, kc, alpha, A, lda, B,
+    const auto f = tiles * c > GR_FIVE ? k_gemm_ref<16> : k_gemm_ref<32>;
+    hipLaunchKernelGGL(f, dim3(tn, tm, (unsigned)c), dim3(256), 0, st, colmajor, m, n, k, kc, alpha, A, lda, B,
                        ldb, beta, C, ldc, z, part);
     hipLaunchKernelGGL(k_gemm_ref_fold, dim3((unsigned)((m * n + 255) / 256)), dim3(256), 0, st, colmajor, m, n, z, c,
                        alpha, beta, part, C, ldc);

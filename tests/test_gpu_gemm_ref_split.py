@@ -29,6 +29,13 @@ def test_gemm_blocks_of_k(O, Q, cuda, layout, m, n, k, alpha, beta, kind):
     assert np.array_equal(from_dev(dC), want)
 
 
+# 35 x 36 = 1260 tiles stage 32 values of k at a time, 36 x 36 = 1296 sixteen; 127 is two blocks of k
+@pytest.mark.parametrize("kind", (0, 1))
+@pytest.mark.parametrize("layout,m,n,k", [(0, 560, 561, 33), (0, 561, 576, 15), (1, 576, 561, 16), (0, 562, 563, 33), (1, 561, 575, 127), (1, 560, 575, 127)])
+def test_gemm_either_side_of_the_staging_rule(O, Q, cuda, layout, m, n, k, kind):
+    test_gemm_blocks_of_k(O, Q, cuda, layout, m, n, k, 1.5, -0.5, kind)
+
+
 def test_gemm_captured_without_a_workspace(O, Q, cuda):
     m, n, k = 40, 50, 400
     A, B, C = O.fill(0, 61, m * k), O.fill(0, 62, k * n), O.fill(0, 63, m * n)
