@@ -837,9 +837,10 @@ int dev_gemm(int mode, int layout, int64_t m, int64_t n, int64_t k, q128 alpha, 
   // gemm_simple for m,n,k <= 64 is one chain over all of k; otherwise blocks of kc
   // (level3.hpp:224-229, :244-246).  For k <= kc both are one block.
   const int64_t kc = (m <= 64 && n <= 64 && k <= 64) ? k : (int64_t)g_kc.load();
-  // without the workspace (a capture that has none, memory exhausted) the same result, slower
+  // without the workspace (memory exhausted) the same result, slower.  None under capture: a graph's branches, two
+  // graphs captured on one stream, and a replay beside the stream's later calls run at the same time, and would share it
   void *part = nullptr;
-  const size_t need = qbk::gemm_ref_ws(m, n, k, kc);
+  const size_t need = stream_capturing(s) ? 0 : qbk::gemm_ref_ws(m, n, k, kc);
   if (need) {
     const std::string err = t_err;
     // an allocation here must not end a capture that another thread has under way
