@@ -196,6 +196,12 @@ bool stream_capturing(hipStream_t s) {
   }
   return cs == hipStreamCaptureStatusActive;
 }
+// Within its scope, the thread's allocations and frees do not end a capture that another thread has under way.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
 // Where a call's status words live: valid while the workspace entry has not been handed out again
 // (its stamp unchanged) -- a later call on that stream reuses, regrows or drops the buffer.
 struct StatusRef {
@@ -278,8 +284,54 @@ int ws_acquire(StreamWorkspaces &W, size_t bytes, hipStream_t s, void **out,
 }
 int ws_release(StreamWorkspaces &, hipStream_t) { return QBLAS_OK; }
 
+// Scratch of the REFERENCE gemm's blocks of k, which only makes the call faster: a buffer of each of the first
+// WS_STREAMS (device, stream) that the thread calls on, and none for others or under capture (a graph's branches, two
+// graphs of one stream, and a replay beside the stream's later calls run at the same time, and would share it).  No
+// call waits: a buffer that a larger call outgrows stays, for the stream's earlier calls, until the thread ends; sizes
+// double, so these are no more than the buffers in use.  hipFree waits for the device.
+struct RefScratch {
+  struct Slot {
+    int dev = -1;
+    hipStream_t s = nullptr;
+    void *p = nullptr;
+    size_t cap = 0;
+  } e[WS_STREAMS];
+  std::vector<void *> outgrown;
+
+  // null: the call does without
+  void *get(size_t bytes, hipStream_t s) {
+    int dev = 0;
+    if (stream_capturing(s) || hipGetDevice(&dev) != hipSuccess) return nullptr;
+    Slot *x = nullptr;
+    for (auto &i : e)
+      if ((i.dev == dev && i.s == s) || (!x && i.dev < 0)) x = &i;
+    if (!x) return nullptr;
+    if (x->cap < bytes) {
+      const size_t want = std::max(bytes, std::min(2 * x->cap, (size_t)(64 << 20)));
+      const RelaxedCapture relaxed;
+      void *p = nullptr;
+      if (hipMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
+      if (x->p) outgrown.push_back(x->p);
+      x->dev = dev;
+      x->s = s;
+      x->p = p;
+      x->cap = want;
+    }
+    return x->p;
+  }
+  ~RefScratch() {
+    const RelaxedCapture relaxed;
+    for (auto &i : e)
+      if (i.p) (void)hipFree(i.p);
+    for (void *p : outgrown) (void)hipFree(p);
+  }
+};
+
 thread_local StreamWorkspaces t_ws;
-thread_local StreamWorkspaces t_rws;                    // the REFERENCE gemm's blocks of k
+thread_local RefScratch t_ref;
 thread_local StreamWorkspaces t_bws;                    // batched calls: prefix sums, OZAKI batch arrays
 thread_local StatusRef t_exact_status;                  // status words of the last EXACT/OZAKI-form call
 thread_local StatusRef t_oz_hdr;                        // header of the last OZAKI-form call
@@ -837,22 +889,8 @@ int dev_gemm(int mode, int layout, int64_t m, int64_t n, int64_t k, q128 alpha, 
   // gemm_simple for m,n,k <= 64 is one chain over all of k; otherwise blocks of kc
   // (level3.hpp:224-229, :244-246).  For k <= kc both are one block.
   const int64_t kc = (m <= 64 && n <= 64 && k <= 64) ? k : (int64_t)g_kc.load();
-  // without the workspace (memory exhausted) the same result, slower.  None under capture: a graph's branches, two
-  // graphs captured on one stream, and a replay beside the stream's later calls run at the same time, and would share it
-  void *part = nullptr;
-  const size_t need = stream_capturing(s) ? 0 : qbk::gemm_ref_ws(m, n, k, kc);
-  if (need) {
-    const std::string err = t_err;
-    // an allocation here must not end a capture that another thread has under way
-    hipStreamCaptureMode cm = hipStreamCaptureModeRelaxed;
-    (void)hipThreadExchangeStreamCaptureMode(&cm);
-    if (ws_acquire(t_rws, need, s, &part) != QBLAS_OK) {
-      part = nullptr;
-      t_err = err;
-      (void)hipGetLastError();
-    }
-    (void)hipThreadExchangeStreamCaptureMode(&cm);
-  }
+  const size_t need = qbk::gemm_ref_ws(m, n, k, kc);
+  void *part = need ? t_ref.get(need, s) : nullptr;  // without it the same result, slower
   QB_CHECK(qbk::launch_gemm_ref(colmajor, m, n, k, kc, alpha, (const q128 *)A, lda, (const q128 *)B, ldb, beta,
                                 (q128 *)C, ldc, (q128 *)part, s));
   return QBLAS_OK;
