@@ -128,7 +128,13 @@ __global__ void __launch_bounds__(XD_BS) k_dot_exact_partial(const q128 *__restr
 // A short dot in one launch of one workgroup, which rounds its digits itself: n = 1001 takes 6.8 us a call, 4096 9.1;
 // 12.8 and 14.6 with the partial and combine kernels, whose time is two launches' latency.
 constexpr int XS_BS = 512;
-constexpr int64_t XS_MAX = 8192;  // 16 products a lane: 13.4 us, the two kernels 14.7
+// One workgroup's loads wait longer the more 128-byte lines they touch.  Measured, us (one launch, two): contiguous 8192
+// 13.4, 14.7; stride 2, 5000 10.6, 14.8, 6500 14.5, 14.6, 8192 18.7, 15.4; stride 4, 5000 13.7, 16.1, 6500 16.2, 15.9;
+// stride 64, 3000 15.2, 17.2, 4096 20.3, 19.7, 8192 36.3, 20.6.
+static bool dot_exact_one_launch(int64_t n, int64_t incx, int64_t incy) {
+  if (incx == 1 && incy == 1) return n <= 8192;
+  return n <= 6144 && n * ((incx < 8 ? incx : 8) + (incy < 8 ? incy : 8)) <= 49152;
+}
 __global__ void __launch_bounds__(XS_BS) k_dot_exact_small(const q128 *__restrict__ x, int64_t incx,
                                                            const q128 *__restrict__ y, int64_t incy, int64_t n,
                                                            q128 *__restrict__ out, uint32_t *__restrict__ hdr) {
@@ -732,7 +738,7 @@ size_t gemv_exact_ws(int colmajor, int64_t m, int64_t n) {
 hipError_t launch_dot_exact(const q128 *x, int64_t incx, const q128 *y, int64_t incy, int64_t n, void *ws,
                             q128 *out, hipStream_t st) {
   uint32_t *hdr = (uint32_t *)ws;
-  if (n <= XS_MAX) {
+  if (dot_exact_one_launch(n, incx, incy)) {
     hipLaunchKernelGGL(k_dot_exact_small, dim3(1), dim3(XS_BS), 0, st, x, incx, y, incy, n, out, hdr);
     return hipGetLastError();
   }
