@@ -284,11 +284,11 @@ int ws_acquire(StreamWorkspaces &W, size_t bytes, hipStream_t s, void **out,
 }
 int ws_release(StreamWorkspaces &, hipStream_t) { return QBLAS_OK; }
 
-// Scratch of the REFERENCE gemm's blocks of k, which only makes the call faster: a buffer of each of the first
-// WS_STREAMS (device, stream) that the thread calls on, and none for others or under capture (a graph's branches, two
-// graphs of one stream, and a replay beside the stream's later calls run at the same time, and would share it).  No
-// call waits: a buffer that a larger call outgrows stays, for the stream's earlier calls, until the thread ends; sizes
-// double, so these are no more than the buffers in use.  hipFree waits for the device.
+// Scratch of the REFERENCE gemm's blocks of k and the gemv's rows left over, which only make the calls faster: a buffer
+// of each of the first WS_STREAMS (device, stream) that the thread calls on, and none for others or under capture (a
+// graph's branches, two graphs of one stream, and a replay beside the stream's later calls run at the same time, and
+// would share it).  No call waits: a buffer that a larger call outgrows stays, for the stream's earlier calls, until the
+// thread ends; sizes double, so these are no more than the buffers in use.  hipFree waits for the device.
 struct RefScratch {
   struct Slot {
     int dev = -1;
@@ -714,8 +714,10 @@ int dev_gemv(int mode, int layout, int64_t m, int64_t n, q128 alpha, const void 
     int rc = ws_acquire(t_ws, (size_t)n * 16, s, &ax);
     if (rc) return rc;
   }
+  const size_t need = qbk::gemv_ref_left(colmajor, m, n, incx);
+  int *left = need ? (int *)t_ref.get(need, s) : nullptr;
   QB_CHECK(qbk::launch_gemv_ref(colmajor, m, n, alpha, (const q128 *)A, lda, (const q128 *)x, incx, beta,
-                                (q128 *)y, incy, (q128 *)ax, s));
+                                (q128 *)y, incy, (q128 *)ax, left, s));
   if (colmajor) return ws_release(t_ws, s);
   return QBLAS_OK;
 }

@@ -15,6 +15,14 @@
 //   5. a check that every S_i lies strictly inside its predicted binade.  The sums before the first
 //      lane that fails are final; that lane's step is done by itself and the lanes after it are taken
 //      again from there.
+// Sums of small integers, of +-1, of terms that cancel pass zero and powers of two all the time, and fail: a pass a
+// step, and a single step besides.  After SC_POOR short passes in a row a chain goes on with blocks that also take
+// the steps that round nothing (LOSSLESS): with S_{i-1} and the product multiples of u_i their sum is a binary128 value
+// wherever it lies below 2^(b_i + 1).  Entries +-1, 8192 x 2048 row-major gemv: 0.33 ms, 3.9 ms without; dot of 2^20: 0.24
+// and 17 ms.  A copy of the code, as the few instructions more cost other chains 3 to 6%.
+// Where those blocks fail too (sums that fall by more binades than a block has, subnormal numbers), steps go one at a
+// time: by all lanes (lane_steps), 2 us each, or, in a launch of many chains, a chain a lane in a kernel of its
+// own (wave_chain_or_not): subnormal entries, 8192 x 2048, 2.5 ms, 14 ms a wave a chain.
 // Integers are in units of 2^(bmin - 112) with bmin = b - 7 for the b of the block's first sum, so
 // binades bmin .. bmin + 13 fit 128 bits.  A product of zero leaves S as it is; steps that are done
 // count as such products.
@@ -27,6 +35,11 @@ namespace qb {
 
 constexpr int SC_WIN = 14;      // binades of a block
 constexpr int SC_LOW = 7;       // of them below the first sum's
+// Passes in a row that end within 16 steps before a chain goes on with lossless blocks, and of those before it is left to a
+// lane (wave_chain_or_not).  The first sums of a chain climb and fall through many binades: of 10000 chains of log-uniform
+// terms 78% have two such passes in a row, 11% four, 2.6% five, one eight.  Few chains that turn hold a launch up: with
+// five, column-major 8192^2 takes 0.86 ms, not 0.77, as the rows of a cache line part.
+constexpr int SC_POOR = 8;
 constexpr int32_t SC_BIG = 1 << 20;
 constexpr int32_t SC_EMAX = 16200;
 
@@ -63,8 +76,9 @@ QB_HD q128 sstate_get(const sstate &s) {
   return q_make((lo >> SC_LOW) | (hi << (64 - SC_LOW)),
                 ((uint64_t)(s.neg & 1u) << 63) | ((uint64_t)(s.b + QBIAS) << 48) | ((hi >> SC_LOW) & FRAC_HI_MASK));
 }
-// S (two's complement, units of 2^(bmin - 112)) as the state; S is a binary128 value or zero
-QB_HD void sstate_from_sum(sstate &s, const uint32_t (&S)[4], int32_t bmin) {
+// S (two's complement, units of 2^(bmin - 112)) as the state; S is a binary128 value or zero, its leading bit in
+// 112..125, or, any: anywhere below
+QB_HD void sstate_from_sum(sstate &s, const uint32_t (&S)[4], int32_t bmin, bool any = false) {
   const uint32_t x = (uint32_t)((int32_t)S[3] >> 31);
   uint64_t lo = (((uint64_t)S[1] << 32) | S[0]) ^ (((uint64_t)x << 32) | x);
   uint64_t hi = (((uint64_t)S[3] << 32) | S[2]) ^ (((uint64_t)x << 32) | x);
@@ -76,7 +90,12 @@ QB_HD void sstate_from_sum(sstate &s, const uint32_t (&S)[4], int32_t bmin) {
     s.w[0] = s.w[1] = s.w[2] = s.w[3] = 0;
     return;
   }
-  // the leading bit lies in 112..125, at bit 48..61 of hi: to bit 48 + SC_LOW
+  if (any && hi == 0) {
+    hi = lo;
+    lo = 0;
+    bmin -= 64;
+  }
+  // the leading bit to bit 48 + SC_LOW of hi
   const int lz = clz64(hi), L = lz - (15 - SC_LOW);
   s.b = bmin + 15 - lz;
   if (L >= 0) {
@@ -147,9 +166,10 @@ QB_HD sprod sc_product(q128 qa, q128 qb) {
   r.F[4] = ch_alignbit((uint32_t)(c[6] >> 32), (uint32_t)c[6], 21);
   r.neg = a.neg ^ b.neg;
   r.tz = a.tz + b.tz + 72;
-  r.Ep = a.e + b.e;
-  r.bad = r.Ep < -SC_EMAX || r.Ep > SC_EMAX;  // CH_ESPECIAL operands among them
-  if (a.e == CH_ESPECIAL || b.e == CH_ESPECIAL) {
+  const uint32_t ea = q_bexp(qa), eb = q_bexp(qb);
+  r.Ep = (int32_t)(ea + eb) - 2 * QBIAS;
+  r.bad = r.Ep < -SC_EMAX || r.Ep > SC_EMAX;
+  if (ea - 1u > 0x7ffdu || eb - 1u > 0x7ffdu) {
     const bool fin = q_bexp(qa) != 0x7fffu && q_bexp(qb) != 0x7fffu;
     const bool zero = fin && (q_iszero(qa) || q_iszero(qb));
     sc_clear(r);
@@ -173,15 +193,15 @@ QB_HD double sc_first(const sstate &s) {  // S over 2^b
   const double m = ((double)s.w[3] * 0x1p32 + (double)s.w[2]) * (1.0 / (double)(1ull << (48 + SC_LOW)));
   return s.kind == 1 ? 0.0 : (s.neg ? -m : m);
 }
-// exponent of the leading bit of s 2^eref, SC_BIG for zero
-QB_HD int32_t sc_binade(double s, int32_t eref) {
+// exponent of the leading bit of s 2^eref, `zero` for zero
+QB_HD int32_t sc_binade(double s, int32_t eref, int32_t zero = SC_BIG) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const int e = __builtin_amdgcn_frexp_exp(s);
 #else
   int e;
   (void)__builtin_frexp(s, &e);
 #endif
-  return s == 0.0 ? SC_BIG : e - 1 + eref;
+  return s == 0.0 ? zero : e - 1 + eref;
 }
 
 // one lane's step on the grid of its predicted binade
@@ -190,9 +210,11 @@ struct slane {
   uint32_t x0, x1;  // the signed product's floor: 32 bits below the unit, and the lowest word
   int32_t k;      // b - bmin
   bool lost;      // product bits below x0
-  bool live;      // a nonzero product whose grid is in the window
+  bool live;      // a nonzero product on a grid of the window
   bool fix;       // climbs into a higher binade, or a tie
 };
+// LOSSLESS: a product that is a multiple of the lowest grid is live also where the sum is predicted below it
+template <bool LOSSLESS = false>
 QB_HD slane sc_round(const sprod &p, int32_t b, int32_t bprev, int32_t bmin) {
   slane r;
   const int32_t k = b - bmin;
@@ -226,6 +248,7 @@ QB_HD slane sc_round(const sprod &p, int32_t b, int32_t bprev, int32_t bmin) {
   const uint32_t y2 = ch_addc(X[2], 0u, c, c), y3 = ch_addc(X[3], 0u, c, c), y4 = ch_addc(X[4], 0u, c, c);
   const uint32_t below = (1u << r.k) - 1u;
   const bool tie = (y0 | (y1 & below)) == 0 && !r.lost;  // exactly half a unit
+  if (LOSSLESS) r.live = r.live || (k < 0 && !p.bad && p.Ep != -SC_BIG && p.Ep <= bmin + SC_WIN - 1 && X[0] == 0 && !r.lost);
   const uint32_t on = r.live ? ~0u : 0u;
   const uint32_t neg = p.neg & on;
   c = neg & 1u;
@@ -253,6 +276,45 @@ QB_HD bool sc_inside(uint32_t S3, int32_t k) {
   const uint32_t h = S3 ^ (uint32_t)((int32_t)S3 >> 31);
   const uint32_t f = (h + 1u) & ((1u << (16 + k)) - 1u);
   return (h >> (16 + k)) == 1u && f > 1u;
+}
+// LOSSLESS: S lies inside the binade bmin + k, with its lower words looked at (a chain may stay next to the end of a binade
+// for hundreds of steps), or the step is exact: the product and the sum before (its lowest word) are multiples of
+// the unit, and |S| is below the end of the binade.
+QB_HD bool sc_final(const slane &l, const uint32_t (&S)[4], uint32_t before) {
+  const uint32_t h = S[3] ^ (uint32_t)((int32_t)S[3] >> 31), t = h >> (16 + l.k), unit = (1u << l.k) - 1u;
+  const bool inside = t == 1u && ((h & ((1u << (16 + l.k)) - 1u)) | S[0] | S[1] | S[2]) != 0;
+  const bool exact = t <= 1u && !l.lost && (l.x0 | ((l.x1 | before) & unit)) == 0;
+  return l.live && (inside || exact);
+}
+
+// How many steps a chain takes one at a time after a block that ended early: one, or ever more, up to 512, where blocks
+// go on ending within 16 steps (short: their number in a row)
+QB_HD int sc_pace(int &short_blocks, int64_t done) {
+  short_blocks = done >= 16 ? 0 : short_blocks < 13 ? short_blocks + 1 : 13;
+  return short_blocks <= 4 ? 1 : 1 << (short_blocks - 4);
+}
+
+// a chain by a workgroup (group_chain)
+constexpr int SG_WAVES = 8;  // at most 16: a row of lanes holds a value of each
+constexpr int SG_PER = 4;    // two prefix sums for 256 steps of a wave
+constexpr int SG_SPAN = 64 * SG_PER;
+constexpr int SG_STEPS = SG_SPAN * SG_WAVES;
+// sc_fix as a step E -> ((A + E + add + ((A + E) & odd ? 1 : 0)) & grid) - after on the corrections so far, E, in
+// halves of 2^(bmin - 112): A is the exact sum before the step plus the product's floor; what lies below A
+// takes the tie's place of the odd bit
+struct sg_fix {
+  uint32_t A, odd, after;
+  int32_t k;
+};
+QB_HD sg_fix sg_make_fix(const slane &l, uint32_t S0) {
+  const uint64_t z = ((uint64_t)(S0 - l.v[0]) << 32) + (((uint64_t)l.x1 << 32) | l.x0);
+  const bool low = l.lost || ((uint32_t)z & 0x7fffffffu) != 0;
+  sg_fix r;
+  r.A = (uint32_t)(z >> 31);
+  r.k = l.k + 1;
+  r.odd = low ? 0u : 1u << r.k;
+  r.after = S0 << 1;
+  return r;
 }
 
 #if defined(__HIPCC__)
@@ -319,9 +381,11 @@ struct sc_const {
 };
 
 // S = RN(S + a(i) b(i)) for i = pos..n-1 by one whole wave.  s (in scalar registers), a, b, pos and n are
-// the same in all lanes.
-template <typename LA, typename LB>
-__device__ __forceinline__ void wave_steps(sstate &s, const LA a, const LB b, int64_t pos, int64_t n) {
+// the same in all lanes.  Returns the first step not done: n, or, where SC_POOR passes in a row were short, or, LOSSLESS,
+// where a pass fails.
+template <bool LOSSLESS, typename LA, typename LB>
+__device__ __forceinline__ int64_t wave_steps(sstate &s, const LA a, const LB b, int64_t pos, int64_t n) {
+  int poor = 0;  // passes in a row
   const int lane = (int)(threadIdx.x & 63);
   q128 qa = q_zero(0), qb_ = q_zero(0);
   if (pos + lane < n) {
@@ -346,7 +410,7 @@ __device__ __forceinline__ void wave_steps(sstate &s, const LA a, const LB b, in
         if (q_isnan(sstate_get(s))) {
           sstate_set(s, q_nan());
           sstate_uniform(s);
-          return;
+          return n;
         }
         // an infinity stays until an operand is not finite
         const int64_t at = pos + lane;
@@ -360,13 +424,13 @@ __device__ __forceinline__ void wave_steps(sstate &s, const LA a, const LB b, in
         double d = sc_value(p, b0);
         sc_scan(d);
         d += sc_first(s);
-        const int32_t bi = sc_binade(d, b0);
+        const int32_t bi = sc_binade(d, b0, LOSSLESS ? p.Ep : SC_BIG);
         // the binade before: of the last lane below with a product (whose own check covers it), S's for
         // the first one (a zero S is a multiple of every unit)
         const uint64_t below = __ballot(p.Ep != -SC_BIG) & ((1ull << lane) - 1);
         int32_t bp = __builtin_amdgcn_ds_bpermute(4 * (63 - clz64(below)), bi);
         if (below == 0) bp = s.kind == 0 ? s.b : SC_BIG;
-        const slane l = sc_round(p, bi, bp, bmin);
+        const slane l = sc_round<LOSSLESS>(p, bi, bp, bmin);
         uint32_t S[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[i] = l.v[i];
@@ -390,26 +454,39 @@ __device__ __forceinline__ void wave_steps(sstate &s, const LA a, const LB b, in
 #pragma unroll
           for (int i = 1; i < 4; ++i) S[i] = ch_addc(S[i], x, c, c);
         }
-        const bool ok = !p.bad && (p.Ep == -SC_BIG || (l.live && sc_inside(S[3], l.k)));
+        bool ok;
+        if constexpr (LOSSLESS) {
+          const uint32_t first = s.kind == 0 ? (s.w[0] ^ s.neg) - s.neg : 0u;  // of the sum before the block
+          const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)S[0], 0x138, 0xf, 0xf, false);  // wave_shr:1
+          ok = !p.bad && (p.Ep == -SC_BIG || sc_final(l, S, before));
+        } else {
+          ok = !p.bad && (p.Ep == -SC_BIG || (l.live && sc_inside(S[3], l.k)));
+        }
         const uint64_t badm = ~__ballot(ok);
         cut = badm ? __ffsll((unsigned long long)badm) - 1 : 64;
         if (cut > lo) {
           uint32_t T[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) T[i] = sc_lane(S[i], cut - 1);
-          sstate_from_sum(s, T, bmin);
+          sstate_from_sum(s, T, bmin, LOSSLESS);
         }
       }
+      const int from = lo;
       lo = cut;
-      if (cut < cnt) {
+      if constexpr (LOSSLESS) {
+        if (cut < cnt) return pos + cut;
+      } else if (cut < cnt) {
         sstate_step(s, a(pos + cut), b(pos + cut));  // loaded again: seldom
         sstate_uniform(s);
         if (lane <= cut) sc_clear(p);
         lo = cut + 1;
+        poor = cut - from < 16 ? poor + 1 : 0;
+        if (poor == SC_POOR) return pos + lo;
         if (lo > 32) break;  // few lanes left: the next block begins here
       }
     }
     if (lo >= cnt) {
+      poor = 0;
       pos += 64;
       qa = na;
       qb_ = nb;
@@ -422,15 +499,100 @@ __device__ __forceinline__ void wave_steps(sstate &s, const LA a, const LB b, in
       }
     }
   }
+  return n;
+}
+// S = RN(S + a(i) b(i)) for i = pos..to-1, a step at a time by all lanes: where blocks fail.  Lanes load and unpack
+// LANE_SPAN operands at once, the next ones on their way meanwhile.  Vector instructions, as the operands come from
+// LDS: as scalar ones a step takes several times as long.
+constexpr int LANE_SPAN = 16;
+struct alignas(16) lane_lds {
+  cop a[LANE_SPAN], b[LANE_SPAN];
+  q128 pa[LANE_SPAN], pb[LANE_SPAN];
+};
+template <typename LA, typename LB>
+__device__ __forceinline__ q128 lane_steps(q128 v, const LA a, const LB b, int64_t pos, int64_t to, lane_lds &lds) {
+  const int lane = (int)(threadIdx.x & 63);
+  const bool mine = lane < LANE_SPAN;
+  cacc acc;
+  cacc_set(acc, v);
+  q128 x = q_zero(0), y = q_zero(0);
+  if (mine && pos + lane < to) {
+    x = a(pos + lane);
+    y = b(pos + lane);
+  }
+  for (; pos < to; pos += LANE_SPAN) {
+    __builtin_amdgcn_wave_barrier();  // the reads of the operands before are done
+    if (mine) {
+      lds.a[lane] = cop_unpack(x);
+      lds.b[lane] = cop_unpack(y);
+      lds.pa[lane] = x;
+      lds.pb[lane] = y;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int cnt = (int)(to - pos < LANE_SPAN ? to - pos : LANE_SPAN);
+    if (mine && pos + LANE_SPAN + lane < to) {
+      x = a(pos + LANE_SPAN + lane);
+      y = b(pos + LANE_SPAN + lane);
+    }
+    cop A = lds.a[0], B = lds.b[0];
+    for (int q = 0; q < cnt; ++q) {
+      const int nq = (q + 1) % LANE_SPAN;
+      const cop nA = lds.a[nq], nB = lds.b[nq];
+      if (!cacc_step(acc, A, B)) chain_slow(acc, lds.pa[q], lds.pb[q]);
+      A = nA;
+      B = nB;
+    }
+  }
+  return cacc_get(acc);
+}
+// a chain's steps pos..n-1 with lossless blocks
+template <typename LA, typename LB>
+__device__ __forceinline__ void wave_lossless_steps(sstate &s, int &short_blocks, const LA a, const LB b, int64_t pos, int64_t n,
+                                                 lane_lds &lds) {
+  while (pos < n) {
+    const int64_t at = wave_steps<true>(s, a, b, pos, n);
+    if (at >= n) return;
+    const int by = sc_pace(short_blocks, at - pos);
+    pos = n - at < by ? n : at + by;
+    sstate_set(s, lane_steps(sstate_get(s), a, b, at, pos, lds));
+    sstate_uniform(s);
+  }
 }
 // a whole chain of n steps from init; every lane returns the result
 template <typename LA, typename LB>
-__device__ __forceinline__ q128 wave_chain(q128 init, const LA a, const LB b, int64_t n) {
+__device__ __forceinline__ q128 wave_chain(q128 init, const LA a, const LB b, int64_t n, lane_lds &lds) {
   sstate s;
   sstate_set(s, init);
   sstate_uniform(s);
-  wave_steps(s, a, b, 0, n);
+  const int64_t pos = wave_steps<false>(s, a, b, 0, n);
+  if (pos < n) {
+    int short_blocks = 0;
+    wave_lossless_steps(s, short_blocks, a, b, pos, n, lds);
+  }
   return sstate_get(s);
+}
+
+// The same in a launch of many chains; false where the result is not there as blocks go on failing.  A step alone takes a
+// wave as many instructions as 64 chains of a wave: 16 waves a SIMD of them took 7 to 15 times as long as those.
+template <typename LA, typename LB>
+__device__ __forceinline__ bool wave_chain_or_not(q128 &v, const LA a, const LB b, int64_t n) {
+  sstate s;
+  sstate_set(s, v);
+  sstate_uniform(s);
+  int64_t pos = wave_steps<false>(s, a, b, 0, n);
+  for (int poor = 0; pos < n;) {
+    const int64_t at = wave_steps<true>(s, a, b, pos, n);
+    if (at < n) {
+      poor = at - pos < 16 ? poor + 1 : 0;
+      if (poor == SC_POOR) return false;
+      sstate_step(s, a(at), b(at));
+      sstate_uniform(s);
+    }
+    pos = at + 1;
+  }
+  v = sstate_get(s);
+  return true;
 }
 
 // The same by a workgroup of SG_WAVES waves, SG_PER consecutive steps a lane and SG_STEPS at a time, for a
@@ -442,36 +604,18 @@ __device__ __forceinline__ q128 wave_chain(q128 init, const LA a, const LB b, in
 // state itself).  Where a sum leaves the window, or the state is not of kind 0, the next 64 steps are one
 // wave's work, which every wave does for itself.  Every barrier is met by all waves: what decides is the same
 // in all of them.
-constexpr int SG_WAVES = 8;  // at most 16: a row of lanes holds a value of each
-constexpr int SG_PER = 4;    // two prefix sums for 256 steps of a wave
-constexpr int SG_SPAN = 64 * SG_PER;
-constexpr int SG_STEPS = SG_SPAN * SG_WAVES;
 struct sg_lds {
   double dsum[16];         // the waves' sums of products, in double precision
   uint4 total[16];         // of rounded products
   uint32_t fixes[16];      // roundings to be done again
-  uint4 list[SG_STEPS];    // of each: sum + product below the grid, doubled (sg_fix)
+  union {
+    uint4 list[SG_STEPS];        // of each: sum + product below the grid, doubled (sg_fix)
+    lane_lds lanes[SG_WAVES];    // the waves' single steps, between passes
+  };
   uint32_t corr[SG_STEPS]; // the correction of the sums from there on
   uint4 end[16];           // the sum after the wave's last good step
   int cut[16];             // good steps
 };
-// sc_fix as a step E -> ((A + E + add + ((A + E) & odd ? 1 : 0)) & grid) - after on the corrections so far, E, in
-// halves of 2^(bmin - 112): A is the exact sum before the step plus the product's floor; what lies below A
-// takes the tie's place of the odd bit
-struct sg_fix {
-  uint32_t A, odd, after;
-  int32_t k;
-};
-__device__ __forceinline__ sg_fix sg_make_fix(const slane &l, uint32_t S0) {
-  const uint64_t z = ((uint64_t)(S0 - l.v[0]) << 32) + (((uint64_t)l.x1 << 32) | l.x0);
-  const bool low = l.lost || ((uint32_t)z & 0x7fffffffu) != 0;
-  sg_fix r;
-  r.A = (uint32_t)(z >> 31);
-  r.k = l.k + 1;
-  r.odd = low ? 0u : 1u << r.k;
-  r.after = S0 << 1;
-  return r;
-}
 // The fixes of lanes F0 .. F0 + 7, z = A + E of the first one in, (E + after) of the last one out; the next
 // one's z is (E + after) + C.  Inline assembly: the condition of the AND is the addition's carry, which the
 // compiler makes with two compares and a select, and a lane is written by its number.
@@ -497,21 +641,12 @@ __device__ __forceinline__ void sg_fix_lanes(uint32_t &z, uint32_t &kept, uint32
           (sg_fix_eight<8 * G>(z, kept, C, odd, add, grid, std::make_integer_sequence<int, 8>{}), true)) &&
          ...);
 }
-template <typename LA, typename LB>
-__device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, int64_t n, sg_lds &lds) {
+// Steps pos..n-1; returns the first one not done: n, or, not LOSSLESS, where the chain
+// gets on poorly: three passes in a row end within 128 steps, or wave_steps gives up.
+template <bool LOSSLESS, typename LA, typename LB>
+__device__ __forceinline__ int64_t group_steps(sstate &s, const LA a, const LB b, int64_t pos, int64_t n, sg_lds &lds) {
   const int lane = (int)(threadIdx.x & 63), wl = lane & 15;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  if (threadIdx.x < 16) {  // waves that the workgroup does not have
-    lds.dsum[wl] = 0.0;
-    lds.total[wl] = make_uint4(0, 0, 0, 0);
-    lds.fixes[wl] = 0;
-    lds.cut[wl] = SG_SPAN;
-  }
-  __syncthreads();
-  sstate s;
-  sstate_set(s, init);
-  sstate_uniform(s);
-  int64_t pos = 0;
   q128 qa[SG_PER], qb_[SG_PER];
   auto fetch = [&](int64_t at) {
     const int64_t i = at + SG_PER * (int)threadIdx.x;
@@ -524,13 +659,21 @@ __device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, i
       }
     }
   };
-  fetch(0);
+  fetch(pos);
+  int poor = 0;  // passes in a row
+  int64_t alone = 64;
+  int short_blocks = 0;
   for (bool single = true; pos < n;) {  // the first sums climb and fall through many binades
     if (single || s.kind != 0) {
-      const int64_t to = n - pos < 64 ? n : pos + 64;
-      wave_steps(s, a, b, pos, to);
-      if (s.kind == 2 && q_isnan(sstate_get(s))) return q_nan();
-      pos = to;
+      const int64_t by = LOSSLESS ? alone : 64, to = n - pos < by ? n : pos + by;
+      if constexpr (LOSSLESS) {
+        wave_lossless_steps(s, short_blocks, a, b, pos, to, lds.lanes[wv]);
+        pos = to;
+      } else {
+        pos = wave_steps<false>(s, a, b, pos, to);
+        if (pos < to) return pos;
+      }
+      if (s.kind == 2 && q_isnan(sstate_get(s))) return n;
       fetch(pos);
       single = false;
       continue;
@@ -555,8 +698,7 @@ __device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, i
     double before = lds.dsum[wl];
     sc_scan_row(before);
     before += sc_first(s);
-    int32_t top = sc_binade(before, s.b);
-    if (top == SC_BIG) top = s.b;
+    int32_t top = sc_binade(before, s.b, s.b);
 #pragma unroll
     for (int i = 1; i < 16; i <<= 1) top = max(top, __shfl_xor(top, i));
     top = max(__builtin_amdgcn_readfirstlane(top), s.b);
@@ -571,7 +713,7 @@ __device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, i
     int32_t bi[SG_PER], last = 0;
 #pragma unroll
     for (int r = 0; r < SG_PER; ++r) {
-      bi[r] = sc_binade(dl + d[r], s.b);
+      bi[r] = sc_binade(dl + d[r], s.b, LOSSLESS ? p[r].Ep : SC_BIG);
       last = p[r].Ep != -SC_BIG ? bi[r] : last;
     }
     const uint64_t lanes_below = (1ull << lane) - 1;
@@ -583,7 +725,7 @@ __device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, i
     int at = 0, mine = 0, all = 0;  // fixes before the lane, of the lane, of the wave
 #pragma unroll
     for (int r = 0; r < SG_PER; ++r) {
-      l[r] = sc_round(p[r], bi[r], bp, bmin);
+      l[r] = sc_round<LOSSLESS>(p[r], bi[r], bp, bmin);
       bp = p[r].Ep != -SC_BIG ? bi[r] : bp;
       uint32_t c = 0;
 #pragma unroll
@@ -652,7 +794,7 @@ __device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, i
     }
     __syncthreads();
     // the sums of the lane's steps, checked: `good` of them are final, the last of those in S
-    uint32_t corr = at ? lds.corr[at - 1] : 0u;
+    uint32_t corr = at ? lds.corr[at - 1] : 0u, prev = S[0] + corr;
     uint32_t G[4];
     int good = 0;
     bool still = true;
@@ -668,7 +810,8 @@ __device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, i
         X[i] = ch_addc(S[i], V[r][i], c, c);
         X[i] = ch_addc(X[i], i ? x : corr, c2, c2);
       }
-      still = still && !p[r].bad && (p[r].Ep == -SC_BIG || (l[r].live && sc_inside(X[3], l[r].k)));
+      still = still && !p[r].bad && (p[r].Ep == -SC_BIG || (LOSSLESS ? sc_final(l[r], X, prev) : l[r].live && sc_inside(X[3], l[r].k)));
+      prev = X[0];
       good += still ? 1 : 0;
 #pragma unroll
       for (int i = 0; i < 4; ++i) G[i] = still ? X[i] : G[i];
@@ -689,12 +832,32 @@ __device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, i
     if (done) {
       const uint4 t = lds.end[cut ? w : w - 1];
       const uint32_t T[4] = {t.x, t.y, t.z, t.w};
-      sstate_from_sum(s, T, bmin);
+      sstate_from_sum(s, T, bmin, LOSSLESS);
       sstate_uniform(s);
     }
     pos += done;
     single = done < SG_STEPS;
+    poor = done < 128 ? poor + 1 : 0;
+    if constexpr (LOSSLESS) alone = poor < 2 ? 64 : alone < 8192 ? 2 * alone : 8192;
+    else if (poor == 3) return pos;
   }
+  return n;
+}
+// a whole chain of n steps from init; every lane returns the result
+template <typename LA, typename LB>
+__device__ __forceinline__ q128 group_chain(q128 init, const LA a, const LB b, int64_t n, sg_lds &lds) {
+  if (threadIdx.x < 16) {  // waves that the workgroup does not have
+    lds.dsum[threadIdx.x] = 0.0;
+    lds.total[threadIdx.x] = make_uint4(0, 0, 0, 0);
+    lds.fixes[threadIdx.x] = 0;
+    lds.cut[threadIdx.x] = SG_SPAN;
+  }
+  __syncthreads();
+  sstate s;
+  sstate_set(s, init);
+  sstate_uniform(s);
+  const int64_t pos = group_steps<false>(s, a, b, 0, n, lds);
+  if (pos < n) group_steps<true>(s, a, b, pos, n, lds);
   return sstate_get(s);
 }
 #endif  // __HIPCC__

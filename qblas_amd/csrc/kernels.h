@@ -28,7 +28,9 @@ hipError_t launch_dot_ref(const q128 *x, int64_t incx, const q128 *y, int64_t in
                           q128 *part /* 2*T */, q128 *out, hipStream_t st);
 hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const q128 *A, int64_t lda,
                            const q128 *x, int64_t incx, q128 beta, q128 *y, int64_t incy,
-                           q128 *ax /* n, colmajor only */, hipStream_t st);
+                           q128 *ax /* n, colmajor only */,
+                           int *left /* gemv_ref_left bytes, or null */, hipStream_t st);
+size_t gemv_ref_left(int colmajor, int64_t m, int64_t n, int64_t incx);  // 0: launch_gemv_ref takes null
 hipError_t launch_gemm_ref(int colmajor, int64_t m, int64_t n, int64_t k, int64_t kc, q128 alpha, const q128 *A,
                            int64_t lda, const q128 *B, int64_t ldb, q128 beta, q128 *C, int64_t ldc,
                            q128 *part /* gemm_ref_ws bytes, or null */, hipStream_t st);

@@ -72,13 +72,14 @@ __global__ void __launch_bounds__(128) k_dot_ref_chunks(const q128 *__restrict__
                                                         const q128 *__restrict__ y, int64_t incy, int64_t n, int T,
                                                         int direct, q128 *__restrict__ part, q128 *__restrict__ out) {
   __shared__ q128 second;
+  __shared__ lane_lds lds[2];
   const int t = (int)blockIdx.x, pair = blockDim.x > 64;  // two waves: contiguous
   const int p = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int64_t s, e;
   chunk_range(n, T, t, s, e);
   const int64_t len = e > s ? e - s : 0, step = 1 + pair;
   const q128 *xc = x + (s + p) * incx, *yc = y + (s + p) * incy;
-  q128 r = wave_chain(q_zero(0), sc_strided{xc, step * incx}, sc_strided{yc, step * incy}, len / step);
+  q128 r = wave_chain(q_zero(0), sc_strided{xc, step * incx}, sc_strided{yc, step * incy}, len / step, lds[p]);
   if (pair) {
     if (threadIdx.x == 64) second = r;
     __syncthreads();
@@ -108,18 +109,20 @@ __global__ void __launch_bounds__(64 * SG_WAVES) k_dot_ref_group(const q128 *__r
 __global__ void __launch_bounds__(64) k_dot_ref_group_sum(const q128 *__restrict__ x, const q128 *__restrict__ y,
                                                           int64_t n, int T, int pair, q128 *__restrict__ part,
                                                           q128 *__restrict__ out) {
+  __shared__ lane_lds lds;
   for (int t = threadIdx.x; pair && t < T; t += 64) {
     int64_t s, e;
     chunk_range(n, T, t, s, e);
     st(part + 2 * t, dot_pair_end(ld(part + 2 * t), ld(part + 2 * t + 1), x, y, e, (int)((e - s) & 1)));
   }
   __syncthreads();
-  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1 + pair}, sc_const{q_one()}, T);
+  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1 + pair}, sc_const{q_one()}, T, lds);
   if (threadIdx.x == 0) st(out, r);
 }
 // the chunks' values summed from +0 in chunk order (level1.hpp:67-71, :117-120): one more chain
 __global__ void __launch_bounds__(64) k_dot_ref_sum(int T, const q128 *__restrict__ part, q128 *__restrict__ out) {
-  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1}, sc_const{q_one()}, T);
+  __shared__ lane_lds lds;
+  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1}, sc_const{q_one()}, T, lds);
   if (threadIdx.x == 0) st(out, r);
 }
 
@@ -133,11 +136,12 @@ __global__ void __launch_bounds__(64) k_dot_ref_sum(int T, const q128 *__restric
 // RowMajor, incx != 1: one chain per row (level2.hpp:41-44).
 __global__ void __launch_bounds__(64) k_gemv_row_ref(int64_t m, int64_t n, q128 alpha, const q128 *__restrict__ A,
                                                      int64_t lda, const q128 *__restrict__ x, int64_t incx, q128 beta,
-                                                     q128 *__restrict__ y, int64_t incy) {
+                                                     q128 *__restrict__ y, int64_t incy, const int *__restrict__ only) {
   __shared__ __attribute__((aligned(16))) chain_lds lds;
   const int pair = incx == 1, lane = (int)threadIdx.x, p = lane & pair;
   const int64_t i = (int64_t)blockIdx.x * (64 >> pair) + (lane >> pair);
-  const bool live = i < m;
+  const bool live = i < m && (!only || only[i]);  // all rows, or those that the kernel below left
+  if (!__ballot(live)) return;
   const q128 *row = A + i * lda;
   cacc ch;
   cacc_init(ch);
@@ -152,23 +156,42 @@ __global__ void __launch_bounds__(64) k_gemv_row_ref(int64_t m, int64_t n, q128 
                       odd ? ld(x + n - 1) : q_zero(0), alpha, beta, ld(yi)));
 }
 // Few rows: one wave per chain, 64 columns at a time (chain_scan.hpp); rows of a workgroup share x.
-// A pair's chains are neighbouring waves, the first of which ends the row.
+// A pair's chains are neighbouring waves, the first of which ends the row.  LEAVE: a row that blocks of 64 fail on is
+// left, marked in left[], for the kernel above.
+template <bool LEAVE>
 __global__ void __launch_bounds__(256) k_gemv_row_ref_scan(int64_t m, int64_t n, q128 alpha, const q128 *__restrict__ A,
                                                            int64_t lda, const q128 *__restrict__ x, int64_t incx,
-                                                           q128 beta, q128 *__restrict__ y, int64_t incy) {
+                                                           q128 beta, q128 *__restrict__ y, int64_t incy,
+                                                           int *__restrict__ left) {
   __shared__ q128 other[4];
+  __shared__ int s_left[4];
   const int pair = incx == 1;
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t c = (int64_t)blockIdx.x * 4 + w;
   const int64_t i = pair ? c >> 1 : c;
   const int p = pair ? (int)(c & 1) : 0;
   q128 r = q_zero(0);
-  if (i < m)
-    r = wave_chain(q_zero(0), sc_strided{A + i * lda + p, 1 + pair}, sc_strided{x + p, pair ? 2 : incx},
-                   pair ? n / 2 : n);
-  if ((threadIdx.x & 63) == 0) other[w] = r;
+  bool leave = false;
+  if (i < m) {
+    const sc_strided a{A + i * lda + p, 1 + pair}, b{x + p, pair ? 2 : incx};
+    if constexpr (LEAVE) {
+      leave = !wave_chain_or_not(r, a, b, n >> pair);
+    } else {
+      __shared__ lane_lds lds[4];
+      r = wave_chain(r, a, b, n >> pair, lds[w]);
+    }
+  }
+  if ((threadIdx.x & 63) == 0) {
+    other[w] = r;
+    s_left[w] = leave;
+  }
   __syncthreads();
   if (i < m && p == 0 && (threadIdx.x & 63) == 0) {
+    if constexpr (LEAVE) {
+      leave = s_left[w] || s_left[w ^ pair];
+      left[i] = leave;
+      if (leave) return;
+    }
     const int odd = pair && (n & 1);
     q128 *yi = y + i * incy;
     st(yi, gemv_row_end(r, other[w ^ pair], pair, odd, odd ? ld(A + i * lda + n - 1) : q_zero(0),
@@ -187,26 +210,39 @@ __global__ void k_scale_vec(int64_t n, q128 alpha, const q128 *__restrict__ x, i
 // j = 0..n-1 (level2.hpp:69-80); lane i owns row i, so loads of A columns coalesce.
 __global__ void __launch_bounds__(64) k_gemv_col_ref(int64_t m, int64_t n, const q128 *__restrict__ A, int64_t lda,
                                                      const q128 *__restrict__ ax, q128 beta, q128 *__restrict__ y,
-                                                     int64_t incy) {
+                                                     int64_t incy, const int *__restrict__ only) {
   __shared__ __attribute__((aligned(16))) chain_lds lds;
   for (int64_t i0 = (int64_t)blockIdx.x * 64; i0 < m; i0 += (int64_t)gridDim.x * 64) {
     const int64_t i = i0 + threadIdx.x;
+    const bool live = i < m && (!only || only[i]);  // all rows, or those that the kernel below left
+    if (!__ballot(live)) continue;
     q128 *yi = y + i * incy;
     cacc ch;
-    cacc_set(ch, i < m ? chain_mul(beta, ld(yi)) : q_zero(0));
-    lane_chain(ch, i < m, A + i, lda, n, 1, 0, [=](int64_t j) { return ld(ax + j); }, lds);
-    if (i < m) st(yi, cacc_get(ch));
+    cacc_set(ch, live ? chain_mul(beta, ld(yi)) : q_zero(0));
+    lane_chain(ch, live, A + i, lda, n, 1, 0, [=](int64_t j) { return ld(ax + j); }, lds);
+    if (live) st(yi, cacc_get(ch));
   }
 }
-// Few rows: one wave per row; the eight rows of a workgroup share the 128-byte lines of A's columns.
+// Few rows: one wave per row; the eight rows of a workgroup share the 128-byte lines of A's columns.  LEAVE: as above.
+template <bool LEAVE>
 __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n, const q128 *__restrict__ A,
                                                            int64_t lda, const q128 *__restrict__ ax, q128 beta,
-                                                           q128 *__restrict__ y, int64_t incy) {
-  const int64_t i = (int64_t)blockIdx.x * 8 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+                                                           q128 *__restrict__ y, int64_t incy, int *__restrict__ left) {
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t i = (int64_t)blockIdx.x * 8 + w;
   if (i >= m) return;
   q128 *yi = y + i * incy;
-  const q128 r = wave_chain(chain_mul(beta, ld(yi)), sc_strided{A + i, lda}, sc_strided{ax, 1}, n);
-  if ((threadIdx.x & 63) == 0) st(yi, r);
+  q128 r = chain_mul(beta, ld(yi));
+  const sc_strided a{A + i, lda}, b{ax, 1};
+  bool leave = false;
+  if constexpr (LEAVE) {
+    leave = !wave_chain_or_not(r, a, b, n);
+    if ((threadIdx.x & 63) == 0) left[i] = leave;
+  } else {
+    __shared__ lane_lds lds[8];
+    r = wave_chain(r, a, b, n, lds[w]);
+  }
+  if (!leave && (threadIdx.x & 63) == 0) st(yi, r);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -370,30 +406,42 @@ static bool few_chains(int64_t chains, int64_t len) {
   return chains <= 32768 && chains * ((len + 63) / 64 * 64 + 128) <= 36864 * len;
 }
 
+// Whether chains that get a wave each may be left to a lane each.  With more than four waves a SIMD, steps one at a time
+// wait for each other: subnormal entries, 8192 x 2048 row-major, 2.5 ms left, 14 ms not; with fewer they do not (1500^2
+// 1.7 ms left, 2.3 ms not), and the second launch costs other calls 2.5 us of 66.
+static bool leaves_chains(int64_t chains) { return chains > 4096; }
+size_t gemv_ref_left(int colmajor, int64_t m, int64_t n, int64_t incx) {
+  const int pair = !colmajor && incx == 1;
+  return few_chains(m << pair, n >> pair) && leaves_chains(m << pair) ? (size_t)m * sizeof(int) : 0;
+}
+
 hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const q128 *A, int64_t lda,
-                           const q128 *x, int64_t incx, q128 beta, q128 *y, int64_t incy, q128 *ax,
+                           const q128 *x, int64_t incx, q128 beta, q128 *y, int64_t incy, q128 *ax, int *left,
                            hipStream_t st) {
   const int threads = 64;
+  const int pair = !colmajor && incx == 1;
+  const bool scan = few_chains(m << pair, n >> pair);
   if (!colmajor) {
-    const int64_t lanes = (incx == 1) ? 2 * m : m;
-    if (few_chains(lanes, (incx == 1) ? n / 2 : n)) {
-      hipLaunchKernelGGL(k_gemv_row_ref_scan, dim3((unsigned)((lanes + 3) / 4)), dim3(256), 0, st, m, n, alpha, A, lda,
-                         x, incx, beta, y, incy);
-      return hipGetLastError();
+    const int64_t lanes = m << pair;
+    if (scan) {
+      const auto f = left ? k_gemv_row_ref_scan<true> : k_gemv_row_ref_scan<false>;
+      hipLaunchKernelGGL(f, dim3((unsigned)((lanes + 3) / 4)), dim3(256), 0, st, m, n, alpha, A, lda, x, incx, beta, y,
+                         incy, left);
+      if (!left) return hipGetLastError();
     }
     const int64_t blocks = (lanes + threads - 1) / threads;
     if (!grid_fits(blocks, threads)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_gemv_row_ref, dim3((unsigned)blocks), dim3(threads), 0, st, m, n, alpha, A, lda, x,
-                       incx, beta, y, incy);
+                       incx, beta, y, incy, left);
   } else {
     hipLaunchKernelGGL(k_scale_vec, dim3(stride_blocks(n, 256)), dim3(256), 0, st, n, alpha, x, incx, ax);
-    if (few_chains(m, n)) {
-      hipLaunchKernelGGL(k_gemv_col_ref_scan, dim3((unsigned)((m + 7) / 8)), dim3(512), 0, st, m, n, A, lda, ax, beta, y,
-                         incy);
-      return hipGetLastError();
+    if (scan) {
+      const auto f = left ? k_gemv_col_ref_scan<true> : k_gemv_col_ref_scan<false>;
+      hipLaunchKernelGGL(f, dim3((unsigned)((m + 7) / 8)), dim3(512), 0, st, m, n, A, lda, ax, beta, y, incy, left);
+      if (!left) return hipGetLastError();
     }
     hipLaunchKernelGGL(k_gemv_col_ref, dim3(stride_blocks(m, threads)), dim3(threads), 0, st, m, n,
-                       A, lda, ax, beta, y, incy);
+                       A, lda, ax, beta, y, incy, left);
   }
   return hipGetLastError();
 }
