@@ -539,7 +539,7 @@ __device__ __forceinline__ q128 lane_steps(q128 v, const LA a, const LB b, int64
     for (int q = 0; q < cnt; ++q) {
       const int nq = (q + 1) % LANE_SPAN;
       const cop nA = lds.a[nq], nB = lds.b[nq];
-      if (!cacc_step(acc, A, B)) chain_slow(acc, lds.pa[q], lds.pb[q]);
+      if (!cacc_step(acc, A, B)) chain_rest(acc, lds.pa[q], lds.pb[q]);
       A = nA;
       B = nB;
     }
