@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(128) k_dot_ref_chunks(const q128 *__restrict__
   else
     st(part + t, r);
 }
-// Long chunks: a workgroup per chain (group_chain), whose values k_dot_ref_group_sum puts together.  2048 steps
+// Long chunks: a workgroup per chain (group_chain), whose values k_dot_ref_sum puts together.  2048 steps
 // take 5 us of VALU issue and barriers and about 60 cycles more for each climb or tie.  2^20 elements, T = 16:
 // 0.29 ms (0.94 ms with a wave per chain; log-uniform 0.16 ms, 0.78 ms).
 __global__ void __launch_bounds__(64 * SG_WAVES) k_dot_ref_group(const q128 *__restrict__ x, int64_t incx,
@@ -106,23 +106,21 @@ __global__ void __launch_bounds__(64 * SG_WAVES) k_dot_ref_group(const q128 *__r
                              sc_strided{y + (s + p) * incy, step * incy}, (e - s) / step, lds);
   if (threadIdx.x == 0) st(part + blockIdx.x, r);
 }
-__global__ void __launch_bounds__(64) k_dot_ref_group_sum(const q128 *__restrict__ x, const q128 *__restrict__ y,
-                                                          int64_t n, int T, int pair, q128 *__restrict__ part,
-                                                          q128 *__restrict__ out) {
+// the chunks' values summed from +0 in chunk order (level1.hpp:67-71, :117-120): one more chain.  PAIR: part holds the
+// values of a chunk's two chains (dot_pair_end)
+template <bool PAIR>
+__global__ void __launch_bounds__(64) k_dot_ref_sum(const q128 *__restrict__ x, const q128 *__restrict__ y, int64_t n, int T,
+                                                    q128 *__restrict__ part, q128 *__restrict__ out) {
   __shared__ lane_lds lds;
-  for (int t = threadIdx.x; pair && t < T; t += 64) {
-    int64_t s, e;
-    chunk_range(n, T, t, s, e);
-    st(part + 2 * t, dot_pair_end(ld(part + 2 * t), ld(part + 2 * t + 1), x, y, e, (int)((e - s) & 1)));
+  if constexpr (PAIR) {
+    for (int t = threadIdx.x; t < T; t += 64) {
+      int64_t s, e;
+      chunk_range(n, T, t, s, e);
+      st(part + 2 * t, dot_pair_end(ld(part + 2 * t), ld(part + 2 * t + 1), x, y, e, (int)((e - s) & 1)));
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1 + pair}, sc_const{q_one()}, T, lds);
-  if (threadIdx.x == 0) st(out, r);
-}
-// the chunks' values summed from +0 in chunk order (level1.hpp:67-71, :117-120): one more chain
-__global__ void __launch_bounds__(64) k_dot_ref_sum(int T, const q128 *__restrict__ part, q128 *__restrict__ out) {
-  __shared__ lane_lds lds;
-  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1}, sc_const{q_one()}, T, lds);
+  const q128 r = wave_chain(q_zero(0), sc_strided{part, 1 + PAIR}, sc_const{q_one()}, T, lds);
   if (threadIdx.x == 0) st(out, r);
 }
 
@@ -388,12 +386,12 @@ hipError_t launch_dot_ref(const q128 *x, int64_t incx, const q128 *y, int64_t in
   if (group_chains(Teff << contiguous, (n / Teff) >> contiguous)) {
     hipLaunchKernelGGL(k_dot_ref_group, dim3((unsigned)(Teff << contiguous)), dim3(64 * SG_WAVES), 0, st, x, incx, y,
                        incy, n, Teff, contiguous, part);
-    hipLaunchKernelGGL(k_dot_ref_group_sum, dim3(1), dim3(64), 0, st, x, y, n, Teff, contiguous, part, out);
+    hipLaunchKernelGGL(contiguous ? k_dot_ref_sum<true> : k_dot_ref_sum<false>, dim3(1), dim3(64), 0, st, x, y, n, Teff, part, out);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_dot_ref_chunks, dim3(Teff), dim3(contiguous ? 128 : 64), 0, st, x, incx, y, incy, n, Teff, direct,
                      part, out);
-  if (Teff > 1) hipLaunchKernelGGL(k_dot_ref_sum, dim3(1), dim3(64), 0, st, Teff, part, out);
+  if (Teff > 1) hipLaunchKernelGGL(k_dot_ref_sum<false>, dim3(1), dim3(64), 0, st, x, y, n, Teff, part, out);
   return hipGetLastError();
 }
 
