@@ -122,7 +122,7 @@ hipError_t launch_gemv_batched(int form, int colmajor, int64_t count, const qbla
                                hipStream_t st);
 // batched OZAKI form (kernels_ozaki.hip, slice method, one slice count for the batch): the scan
 // writes per-problem prefix sums into ws (gemm_ozaki_batched_scan_ws bytes); the caller reads the
-// 9 totals at ws + gemm_ozaki_batched_totals_offset, grows ws to gemm_ozaki_batched_ws (running the
+// OZ_BATCHED_TOTALS totals at ws + gemm_ozaki_batched_totals_offset, grows ws to gemm_ozaki_batched_ws (running the
 // scan again when ws moved) and launches the rest.  ws word 0 is the status word.
 constexpr int OZ_BATCHED_TOTALS = 10;
 constexpr int OZ_HDR_STALE = 8;  // header word: planned totals did not match (nothing computed)

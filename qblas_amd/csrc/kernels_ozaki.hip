@@ -689,7 +689,7 @@ __global__ void __launch_bounds__(256) k_oz_finish(int64_t M, int64_t N, int S, 
 // sum_l A_il B_lj in each lane's LDS digits (exact_dev.hpp) with an anchor placing the largest
 // possible product (from the row and column maxima) at the top of their range, then the exact
 // alpha*S + beta*C rounded once.  An entry with a product below the range is recomputed on the
-// full-range path.  Bound by VALU issue, about 125 instructions a product; the rounding, 1400
+// full-range path.  Bound by VALU issue, about 110 instructions a product; the rounding, 1400
 // instructions of one lane, waits until the workgroup has summed up to OZR_SLOTS entries and is
 // done for all of them at once, one a lane.  4096^3 log-uniform with 33817 queued entries: 0.65 ms
 // (1.2 ms with two register windows a lane, summed over the lanes and rounded entry by entry; 0.91 ms with two

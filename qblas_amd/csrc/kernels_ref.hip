@@ -91,9 +91,11 @@ __global__ void __launch_bounds__(128) k_dot_ref_chunks(const q128 *__restrict__
   else
     st(part + t, r);
 }
-// Long chunks: a workgroup per chain (group_chain), whose values k_dot_ref_sum puts together.  2048 steps
-// take 5 us of VALU issue and barriers and about 60 cycles more for each climb or tie.  2^20 elements, T = 16:
-// 0.29 ms (0.94 ms with a wave per chain; log-uniform 0.16 ms, 0.78 ms).
+// Long chunks: a workgroup per chain (group_chain), whose values k_dot_ref_sum puts together.  2048 steps take
+// 6.3 us with the operands in L2, 9 us in the dot of 2^20, of VALU issue, barriers and waits for operands, and a climb or
+// tie 0.05 us more (120 cycles).  A chain of 32768 uniform terms takes 17.4 such passes, 1.4 of them ended early by a sum
+// near zero and followed by 64 steps of a wave, and has 570 climbs; of log-uniform ones 16.3 and 150.  2^20 elements,
+// T = 16: 0.25 ms (0.94 ms with a wave per chain; log-uniform 0.165 ms, 0.78 ms).
 __global__ void __launch_bounds__(64 * SG_WAVES) k_dot_ref_group(const q128 *__restrict__ x, int64_t incx,
                                                                  const q128 *__restrict__ y, int64_t incy, int64_t n,
                                                                  int T, int pair, q128 *__restrict__ part) {
@@ -253,11 +255,12 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
 // nothing, so C = fma(alpha, t, C) over the blocks is one more chain, from beta * C.  Layout-aware indexing for
 // both layouts.  A workgroup computes a 16 x 16 tile of C (tile_chain).
 // Bound by VALU issue: 85 to 105 instructions per wave and multiply-add (chain.hpp).  4096^3
-// log-uniform: 222 ms = 619 quad GFLOP/s (577 ms with a 401-instruction step); 2048^3 uniform 21.9 ms.
+// log-uniform: 214 ms = 643 quad GFLOP/s (577 ms with a 401-instruction step); 2048^3 uniform 21.9 ms.
 // part == null: the workgroup takes all blocks of k.  Else it takes block kb0 + blockIdx.z and writes its t to
 // part[(blockIdx.z n + j) m + i], for k_gemm_ref_fold: the blocks' chains do not depend on each other,
-// so a C of few tiles still fills the chip: 500 x 333 x 700 427 us against 561, 64 x 64 x 2000 68 us
-// against 874 (both with the step of 105 instructions; now 329 us and 72 us).
+// so a C of few tiles still fills the chip: 500 x 333 x 700 326 us against 454, 64 x 64 x 2000 70 us against 823.
+// The latter's 256 workgroups are one wave a SIMD: bound by a step's latency of 0.46 us, which 85 instructions in place of
+// 105 did not shorten (68 us then), as the chain of dependent additions stayed as long.
 // KT: values of k staged at a time, 1 KB of LDS each.  32 let five workgroups share a CU, 16 eight: with more
 // workgroups than five a CU 16 is faster (1000^3 2734 us against 2850, 500 x 333 x 700 363 against 377), with
 // fewer the barriers cost more than there is to overlap them with (100 x 100 x 900 78 us against 75).
