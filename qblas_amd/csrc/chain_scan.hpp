@@ -573,23 +573,26 @@ __device__ __forceinline__ q128 wave_chain(q128 init, const LA a, const LB b, in
   return sstate_get(s);
 }
 
-// The same in a launch of many chains; false where the result is not there as blocks go on failing.  A step alone takes a
-// wave as many instructions as 64 chains of a wave: 16 waves a SIMD of them took 7 to 15 times as long as those.
+// The same in a launch of many chains, with fewer registers: steps alone are scalar ones.  False where the result is not there,
+// as blocks go on failing and the chain may be left (leave): a step alone takes a wave as many instructions as 64
+// chains of a wave, and 16 waves a SIMD of them took 7 to 15 times as long as those.
 template <typename LA, typename LB>
-__device__ __forceinline__ bool wave_chain_or_not(q128 &v, const LA a, const LB b, int64_t n) {
+__device__ __forceinline__ bool wave_chain_or_not(q128 &v, const LA a, const LB b, int64_t n, bool leave) {
   sstate s;
   sstate_set(s, v);
   sstate_uniform(s);
   int64_t pos = wave_steps<false>(s, a, b, 0, n);
-  for (int poor = 0; pos < n;) {
+  int short_blocks = 0;
+  while (pos < n) {
     const int64_t at = wave_steps<true>(s, a, b, pos, n);
-    if (at < n) {
-      poor = at - pos < 16 ? poor + 1 : 0;
-      if (poor == SC_POOR) return false;
-      sstate_step(s, a(at), b(at));
+    if (at >= n) break;
+    const int by = sc_pace(short_blocks, at - pos);
+    if (leave && short_blocks == SC_POOR) return false;
+    pos = n - at < by ? n : at + by;
+    for (int64_t i = at; i < pos; ++i) {
+      sstate_step(s, a(i), b(i));
       sstate_uniform(s);
     }
-    pos = at + 1;
   }
   v = sstate_get(s);
   return true;

@@ -156,9 +156,9 @@ __global__ void __launch_bounds__(64) k_gemv_row_ref(int64_t m, int64_t n, q128 
                       odd ? ld(x + n - 1) : q_zero(0), alpha, beta, ld(yi)));
 }
 // Few rows: one wave per chain, 64 columns at a time (chain_scan.hpp); rows of a workgroup share x.
-// A pair's chains are neighbouring waves, the first of which ends the row.  LEAVE: a row that blocks of 64 fail on is
-// left, marked in left[], for the kernel above.
-template <bool LEAVE>
+// A pair's chains are neighbouring waves, the first of which ends the row.  MANY: in a launch of many chains, a row
+// that blocks of 64 fail on is left, marked in left[] unless that is null, for the kernel above.
+template <bool MANY>
 __global__ void __launch_bounds__(256) k_gemv_row_ref_scan(int64_t m, int64_t n, q128 alpha, const q128 *__restrict__ A,
                                                            int64_t lda, const q128 *__restrict__ x, int64_t incx,
                                                            q128 beta, q128 *__restrict__ y, int64_t incy,
@@ -174,8 +174,8 @@ __global__ void __launch_bounds__(256) k_gemv_row_ref_scan(int64_t m, int64_t n,
   bool leave = false;
   if (i < m) {
     const sc_strided a{A + i * lda + p, 1 + pair}, b{x + p, pair ? 2 : incx};
-    if constexpr (LEAVE) {
-      leave = !wave_chain_or_not(r, a, b, n >> pair);
+    if constexpr (MANY) {
+      leave = !wave_chain_or_not(r, a, b, n >> pair, left != nullptr);
     } else {
       __shared__ lane_lds lds[4];
       r = wave_chain(r, a, b, n >> pair, lds[w]);
@@ -187,9 +187,9 @@ __global__ void __launch_bounds__(256) k_gemv_row_ref_scan(int64_t m, int64_t n,
   }
   __syncthreads();
   if (i < m && p == 0 && (threadIdx.x & 63) == 0) {
-    if constexpr (LEAVE) {
+    if constexpr (MANY) {
       leave = s_left[w] || s_left[w ^ pair];
-      left[i] = leave;
+      if (left) left[i] = leave;
       if (leave) return;
     }
     const int odd = pair && (n & 1);
@@ -223,8 +223,8 @@ __global__ void __launch_bounds__(64) k_gemv_col_ref(int64_t m, int64_t n, const
     if (live) st(yi, cacc_get(ch));
   }
 }
-// Few rows: one wave per row; the eight rows of a workgroup share the 128-byte lines of A's columns.  LEAVE: as above.
-template <bool LEAVE>
+// Few rows: one wave per row; the eight rows of a workgroup share the 128-byte lines of A's columns.  MANY: as above.
+template <bool MANY>
 __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n, const q128 *__restrict__ A,
                                                            int64_t lda, const q128 *__restrict__ ax, q128 beta,
                                                            q128 *__restrict__ y, int64_t incy, int *__restrict__ left) {
@@ -235,9 +235,9 @@ __global__ void __launch_bounds__(512) k_gemv_col_ref_scan(int64_t m, int64_t n,
   q128 r = chain_mul(beta, ld(yi));
   const sc_strided a{A + i, lda}, b{ax, 1};
   bool leave = false;
-  if constexpr (LEAVE) {
-    leave = !wave_chain_or_not(r, a, b, n);
-    if ((threadIdx.x & 63) == 0) left[i] = leave;
+  if constexpr (MANY) {
+    leave = !wave_chain_or_not(r, a, b, n, left != nullptr);
+    if (left && (threadIdx.x & 63) == 0) left[i] = leave;
   } else {
     __shared__ lane_lds lds[8];
     r = wave_chain(r, a, b, n, lds[w]);
@@ -407,13 +407,13 @@ static bool few_chains(int64_t chains, int64_t len) {
   return chains <= 32768 && chains * ((len + 63) / 64 * 64 + 128) <= 36864 * len;
 }
 
-// Whether chains that get a wave each may be left to a lane each.  With more than four waves a SIMD, steps one at a time
+// Whether there are so many chains of a wave each that they may be left to a lane each.  With more than four waves a SIMD, steps one at a time
 // wait for each other: subnormal entries, 8192 x 2048 row-major, 2.5 ms left, 14 ms not; with fewer they do not (1500^2
 // 1.7 ms left, 2.3 ms not), and the second launch costs other calls 2.5 us of 66.
-static bool leaves_chains(int64_t chains) { return chains > 4096; }
+static bool many_chains(int64_t chains) { return chains > 4096; }
 size_t gemv_ref_left(int colmajor, int64_t m, int64_t n, int64_t incx) {
   const int pair = !colmajor && incx == 1;
-  return few_chains(m << pair, n >> pair) && leaves_chains(m << pair) ? (size_t)m * sizeof(int) : 0;
+  return few_chains(m << pair, n >> pair) && many_chains(m << pair) ? (size_t)m * sizeof(int) : 0;
 }
 
 hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const q128 *A, int64_t lda,
@@ -425,7 +425,7 @@ hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const
   if (!colmajor) {
     const int64_t lanes = m << pair;
     if (scan) {
-      const auto f = left ? k_gemv_row_ref_scan<true> : k_gemv_row_ref_scan<false>;
+      const auto f = many_chains(lanes) ? k_gemv_row_ref_scan<true> : k_gemv_row_ref_scan<false>;
       hipLaunchKernelGGL(f, dim3((unsigned)((lanes + 3) / 4)), dim3(256), 0, st, m, n, alpha, A, lda, x, incx, beta, y,
                          incy, left);
       if (!left) return hipGetLastError();
@@ -437,7 +437,7 @@ hipError_t launch_gemv_ref(int colmajor, int64_t m, int64_t n, q128 alpha, const
   } else {
     hipLaunchKernelGGL(k_scale_vec, dim3(stride_blocks(n, 256)), dim3(256), 0, st, n, alpha, x, incx, ax);
     if (scan) {
-      const auto f = left ? k_gemv_col_ref_scan<true> : k_gemv_col_ref_scan<false>;
+      const auto f = many_chains(m) ? k_gemv_col_ref_scan<true> : k_gemv_col_ref_scan<false>;
       hipLaunchKernelGGL(f, dim3((unsigned)((m + 7) / 8)), dim3(512), 0, st, m, n, A, lda, ax, beta, y, incy, left);
       if (!left) return hipGetLastError();
     }

@@ -208,15 +208,15 @@ static void wave_lossless(sstate &s, int &short_blocks, const vec &a, const vec 
   }
 }
 // wave_chain_or_not
-static bool wave_or_not(sstate &s, const vec &a, const vec &b, int64_t pos, int64_t n) {
-  for (int poor = 0; pos < n;) {
+static bool wave_or_not(sstate &s, const vec &a, const vec &b, int64_t pos, int64_t n, bool leave) {
+  int short_blocks = 0;
+  while (pos < n) {
     const int64_t at = wave<true>(s, a, b, pos, n);
-    if (at < n) {
-      poor = at - pos < 16 ? poor + 1 : 0;
-      if (poor == SC_POOR) return false;
-      sstate_step(s, a[at], b[at]);
-    }
-    pos = at + 1;
+    if (at >= n) break;
+    const int by = sc_pace(short_blocks, at - pos);
+    if (leave && short_blocks == SC_POOR) return false;
+    pos = n - at < by ? n : at + by;
+    for (int64_t i = at; i < pos; ++i) sstate_step(s, a[i], b[i]);
   }
   return true;
 }
@@ -330,12 +330,13 @@ int main(int argc, char **argv) {
         } else {
           sstate t = s;
           const long are = passes;
-          if (wave_or_not(t, a, b, at, n)) {
-            const q128 got = sstate_get(t);
-            wrong += got.lo != ref.lo || got.hi != ref.hi;
-          } else {
+          if (!wave_or_not(t, a, b, at, n, true)) {
             ++left;
+            t = s;
+            wave_or_not(t, a, b, at, n, false);
           }
+          const q128 got = sstate_get(t);
+          wrong += got.lo != ref.lo || got.hi != ref.hi;
           passes = are;
           int short_blocks = 0;
           wave_lossless(s, short_blocks, a, b, at, n);
